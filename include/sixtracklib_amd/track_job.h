@@ -39,10 +39,10 @@
  * tiles and one otherwise, and between one and two particles per resident
  * lane it runs mixed launches, some waves of every SIMD with two particles
  * per lane and the others with one (the most pair waves that leave one
- * single wave per SIMD); with 2 to 8 waves per SIMD of one particle per
- * lane, the particles spread evenly over that many waves of every SIMD (6
- * of them, 2 pairs, for 8); the mixed launches in both builds; results
- * identical), "mix=0|1" (default 1: the mixed launches of ppl=auto),
+ * single wave per SIMD), in both builds; results identical), "mix=0|1"
+ * (default 1: the mixed launches of ppl=auto), "hot=auto|0|1" (default
+ * auto: launches of one particle per lane run the scheduled record walk
+ * where it is faster; 0 never, 1 wherever it can run; results identical),
  * "balance=0|1" (default 1: with compact=1
  * every launch gives each resident wave one 64-particle tile, the
  * particles furthest behind first, and the host reads the counts back

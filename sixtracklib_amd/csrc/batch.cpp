@@ -27,6 +27,7 @@
 #include "lattice.h"
 #include "batch.h"
 #include "batch_runner.h"
+#include "lattice_hot.h"
 
 using st_batch::hip_ok;
 using st_batch::fail;
@@ -85,7 +86,7 @@ struct NS(TrackBatch)
         }
         std::vector< std::vector< uint64_t > > packed( S );
         std::vector< int64_t > n_elem( S );
-        std::vector< size_t > lat_off( S );
+        std::vector< size_t > lat_off( S ), hot_off( S );
         size_t total_lat = 0;
         for( int64_t s = 0; s < S; ++s )
         {
@@ -107,6 +108,12 @@ struct NS(TrackBatch)
             for( int64_t i = 0; i < ne; ++i )
                 run.max_record_words = std::max< int64_t >( run.max_record_words, offs[ i + 1 ] - offs[ i ] );
             n_elem[ s ] = ne;
+            // the hot stream of the lattice behind it
+            hot_off[ s ] = ( packed[ s ].size() + 31u ) & ~( size_t )31u;
+            std::vector< uint64_t > const hot = st::hot_stream( packed[ s ].data() );
+            packed[ s ].reserve( hot_off[ s ] + hot.size() );
+            packed[ s ].resize( hot_off[ s ], 0u );
+            packed[ s ].insert( packed[ s ].end(), hot.begin(), hot.end() );
             lat_off[ s ] = total_lat;
             total_lat += packed[ s ].size();
             total_lat = ( total_lat + 31u ) & ~( size_t )31u;         // 256-byte aligned streams
@@ -125,6 +132,7 @@ struct NS(TrackBatch)
             seeds[ s ].lat = d_lat + lat_off[ s ];
             seeds[ s ].n_elem = n_elem[ s ];
             seeds[ s ].list = nullptr;
+            seeds[ s ].hot = d_lat + lat_off[ s ] + hot_off[ s ];
         }
         return run.init( seeds, stream ) && push();     // both synchronise: packed outlives the copies
     }

@@ -14,6 +14,7 @@ typedef struct st_batch_seed_s
     const uint64_t* lat;        // packed lean lattice (device), END-terminated
     int64_t n_elem;             // elements per turn
     int32_t* list;              // active-particle list, capacity P.n
+    const uint64_t* hot;        // the lattice's hot stream (lattice_hot.h)
 }
 st_batch_seed_t;
 
@@ -49,7 +50,7 @@ st_batch_sched_t;
         int64_t max_particles, int64_t until_turn, hipStream_t stream );              \
     extern "C" hipError_t st_launch_batch_track##SUF( const st_batch_sched_t* s,     \
         int64_t until_turn, int64_t max_turns, int32_t* status, int block, int grid, \
-        int particles_per_lane, int heavy, int staging, hipStream_t stream );          \
+        int particles_per_lane, int heavy, int staging, int hot, hipStream_t stream ); \
     extern "C" hipError_t st_launch_batch_track_mix##SUF( const st_batch_sched_t* s, \
         int64_t until_turn, int64_t max_turns, int32_t* status, int grid,            \
         int64_t pair_waves, hipStream_t stream );

@@ -22,6 +22,7 @@
 #include "track_device.h"
 #include "track_lean.h"
 #include "track_lean_lds.h"
+#include "track_hot.h"
 #include "batch.h"
 
 #ifndef ST_KSUFFIX
@@ -44,9 +45,9 @@ namespace
 typedef __attribute__( ( address_space( 4 ) ) ) const int32_t ci32_t;
 
 static_assert( sizeof( st_dev_particles_t ) == 22 * 8, "particle view: count + 21 pointers" );
-static_assert( sizeof( st_batch_seed_t ) == 25 * 8, "seed descriptor: view, lat, n_elem, list" );
+static_assert( sizeof( st_batch_seed_t ) == 26 * 8, "seed descriptor: view, lat, n_elem, list, hot" );
 
-// Seed descriptor k, read as 25 words through the constant address space.
+// Seed descriptor k, read as 26 words through the constant address space.
 struct SeedView
 {
     st_dev_particles_t P;
@@ -57,7 +58,7 @@ struct SeedView
 
 ST_DEV SeedView load_seed( const st_batch_seed_t* seeds, int k )
 {
-    cptr_t const w = ( cptr_t )seeds + 25 * k;
+    cptr_t const w = ( cptr_t )seeds + 26 * k;
     SeedView v;
     v.P.n = ( int64_t )w[ 0 ];
     v.P.q0 = ( double* )w[ 1 ];      v.P.mass0 = ( double* )w[ 2 ];
@@ -107,7 +108,7 @@ __global__ void __launch_bounds__( 256 ) KN( st_k_batch_select )( st_batch_sched
 __global__ void __launch_bounds__( 256 ) KN( st_k_batch_minturn )( st_batch_sched_t s,
     int64_t until_turn )
 {
-    cptr_t const w = ( cptr_t )s.seeds + 25 * blockIdx.y;
+    cptr_t const w = ( cptr_t )s.seeds + 26 * blockIdx.y;
     int64_t const n = ( int64_t )w[ 0 ];
     if( ( int64_t )blockIdx.x * blockDim.x >= n ) return;            // whole block past the set
     int64_t const i = ( int64_t )blockIdx.x * blockDim.x + threadIdx.x;
@@ -134,7 +135,7 @@ __global__ void __launch_bounds__( 256 ) KN( st_k_batch_select_split )( st_batch
     int64_t until_turn )
 {
     int const k = ( int )blockIdx.y;
-    cptr_t const w = ( cptr_t )s.seeds + 25 * k;
+    cptr_t const w = ( cptr_t )s.seeds + 26 * k;
     int64_t const n = ( int64_t )w[ 0 ];
     if( ( int64_t )blockIdx.x * blockDim.x >= n ) return;            // whole block past the set
     int32_t* const list = ( int32_t* )w[ 24 ];
@@ -202,7 +203,7 @@ ST_DEV bool find_tile( const st_batch_sched_t& s, int qb, int qe, int t, int& se
             if( t < nt )
             {
                 seed = sd; count = n; tile = t;
-                list = ( const int32_t* )( ( cptr_t )s.seeds + 25 * sd )[ 24 ];
+                list = ( const int32_t* )( ( cptr_t )s.seeds + 26 * sd )[ 24 ];
                 return true;
             }
             t -= nt;
@@ -218,7 +219,7 @@ ST_DEV bool find_tile( const st_batch_sched_t& s, int qb, int qe, int t, int& se
             int const nt = ( n + TILE - 1 ) / TILE;
             if( t < nt )
             {
-                cptr_t const w = ( cptr_t )s.seeds + 25 * sd;
+                cptr_t const w = ( cptr_t )s.seeds + 26 * sd;
                 seed = sd; count = n; tile = t;
                 list = ( const int32_t* )w[ 24 ] + ( part == 0 ? 0 : ( int64_t )w[ 0 ] - n );
                 return true;
@@ -230,7 +231,7 @@ ST_DEV bool find_tile( const st_batch_sched_t& s, int qb, int qe, int t, int& se
 
 // Tile loop of the persistent track kernels (HEAVY: lattices that also
 // hold the maps outside the lean set).
-template< bool HEAVY >
+template< bool HEAVY, bool HOT = false >
 ST_DEV void batch_track_tiles( const st_batch_sched_t& s, int64_t until_turn, int64_t max_turns,
                                int32_t* status )
 {
@@ -252,11 +253,18 @@ ST_DEV void batch_track_tiles( const st_batch_sched_t& s, int64_t until_turn, in
             int32_t count = 0;
             const int32_t* list = nullptr;
             if( !find_tile< 64 >( s, qb, qe, t, seed, list, count, tile ) ) break;   // queue drained
-            if constexpr( HEAVY )
+            if constexpr( HOT )
+            {
+                cptr_t const w = ( cptr_t )s.seeds + 26 * seed;
+                track_hot_lane< HEAVY >( PDesc{ w }, list, count, ( int64_t )tile * 64 + __lane_id(),
+                                         ( cptr_t )w[ 22 ], ( cptr_t )w[ 25 ], ( int64_t )w[ 23 ],
+                                         until_turn, max_turns, status, wp );
+            }
+            else if constexpr( HEAVY )
             {
                 // the particle set is read from the seed descriptor where
                 // it is used (its first 22 words are the set's view)
-                cptr_t const w = ( cptr_t )s.seeds + 25 * seed;
+                cptr_t const w = ( cptr_t )s.seeds + 26 * seed;
                 track_lean_lane< true >( PDesc{ w }, list, count, ( int64_t )tile * 64 + __lane_id(),
                                          ( cptr_t )w[ 22 ], ( int64_t )w[ 23 ], until_turn, max_turns,
                                          status, wp );
@@ -277,6 +285,15 @@ KN( st_k_batch_track )( st_batch_sched_t s, int64_t until_turn, int64_t max_turn
                         int32_t* status )
 {
     batch_track_tiles< false >( s, until_turn, max_turns, status );
+}
+
+// The same with the scheduled record walk (track_hot.h), in one-wave
+// workgroups.  Its 108 SGPRs allow seven waves per SIMD.
+__global__ void __launch_bounds__( 64, 4 )
+KN( st_k_batch_track_hot )( st_batch_sched_t s, int64_t until_turn, int64_t max_turns,
+                            int32_t* status )
+{
+    batch_track_tiles< false, true >( s, until_turn, max_turns, status );
 }
 
 // The same for lattices with monitors, beam-beam, space charge or RF
@@ -353,7 +370,7 @@ KN( st_k_batch_track2 )( st_batch_sched_t s, int64_t until_turn, int64_t max_tur
             int32_t count = 0;
             const int32_t* list = nullptr;
             if( !find_tile< 128 >( s, qb, qe, t, seed, list, count, tile ) ) break;  // queue drained
-            cptr_t const w = ( cptr_t )s.seeds + 25 * seed;
+            cptr_t const w = ( cptr_t )s.seeds + 26 * seed;
             track_lean_lane2( PDesc{ w }, list, count, ( int64_t )tile * 128, ( cptr_t )w[ 22 ],
                               ( int64_t )w[ 23 ], until_turn, max_turns, status, wp );
             if( one_tile ) return;
@@ -461,7 +478,7 @@ extern "C" hipError_t KN( st_launch_batch_track_mix )( const st_batch_sched_t* s
 
 extern "C" hipError_t KN( st_launch_batch_track )( const st_batch_sched_t* s,
     int64_t until_turn, int64_t max_turns, int32_t* status, int block, int grid,
-    int particles_per_lane, int heavy, int staging, hipStream_t stream )
+    int particles_per_lane, int heavy, int staging, int hot, hipStream_t stream )
 {
     if( s->n_seeds <= 0 || s->n_queues <= 0 ) return hipSuccess;
     if( block <= 0 || block > 256 || ( block % 64 ) != 0 ) block = 256;
@@ -469,6 +486,9 @@ extern "C" hipError_t KN( st_launch_batch_track )( const st_batch_sched_t* s,
     if( staging && !heavy )
         hipLaunchKernelGGL( KN( st_k_batch_track_lds ), dim3( ( unsigned )grid ), dim3( 256 ), 0,
                             stream, *s, until_turn, max_turns, status );
+    else if( hot && !heavy && particles_per_lane == 1 )
+        hipLaunchKernelGGL( KN( st_k_batch_track_hot ), dim3( ( unsigned )grid ), dim3( 64 ), 0, stream,
+                            *s, until_turn, max_turns, status );
     else if( heavy )
         hipLaunchKernelGGL( KN( st_k_batch_track_heavy ), dim3( ( unsigned )grid ),
                             dim3( ( unsigned )block ), 0, stream, *s, until_turn, max_turns, status );

@@ -69,6 +69,8 @@ struct Config
                                  // (set by the owner, one particle per lane)
     bool balance = false;        // run_balanced() available (split lists)
     bool wave_prio = true;       // waves with more turns left issue first
+    int hot = -1;                // scheduled record walk (track_hot.h) where it applies: -1
+                                 // by rule, 0 never, 1 wherever it can run
     int staging = 0;             // lattice read through scalar loads (0) or staged
                                  // through LDS by 256-lane workgroups (1; lean
                                  // lattices, one particle per lane)
@@ -118,6 +120,7 @@ struct Config
             mix = false;
         }
         else if( k == "mix" ) mix = iv != 0;
+        else if( k == "hot" ) hot = v == "auto" ? -1 : ( iv != 0 ? 1 : 0 );
         else if( k == "staging" )
         {
             if( v == "scalar" || v == "0" ) staging = 0;
@@ -127,11 +130,23 @@ struct Config
         return true;
     }
 
+    // One particle per lane through the scheduled record walk, in one-wave
+    // workgroups (16 waves then run on 16 CUs, each with a scalar cache of
+    // its own: 54.6 against 59.2 ns per element with workgroups of four,
+    // FMA build, 1,000 particles on the 20,000-element ring).  It is faster
+    // than the compiled loop from 64 particles to 8 waves per SIMD, though
+    // its SGPRs allow 7 (ns per element and wave set on that ring, exact
+    // build and FMA build, loop / walk): 65,536 particles 198 / 88 and
+    // 169 / 63; 131,072: 212 / 125 and 178 / 91; 262,144: 284 / 229 and
+    // 242 / 156; 400,000: 411 / 372 and 307 / 255; 524,288: 478 / 424 and
+    // 344 / 328.
+    bool walk() const { return hot != 0 && ppl == 1 && !heavy && !lds(); }
+
     // the LDS-staged kernel runs lean lattices with one particle per lane
     bool lds() const { return staging != 0 && !heavy; }
     // particles per tile and tiles a workgroup tracks at once
     int64_t tile_particles() const { return lds() ? 256 : 64 * ppl; }
-    int tiles_per_block() const { return lds() ? 1 : block / 64; }
+    int tiles_per_block() const { return lds() || walk() ? 1 : block / 64; }
 
     bool parse( const char* cfg )
     {
@@ -303,7 +318,8 @@ struct BatchRunner
         return a256( s * sizeof( st_batch_seed_t ) ) + a256( ( s + 9 ) * 4 );
     }
 
-    bool init_borrowed( const st_dev_particles_t* views, const uint64_t* lat, int64_t n_elem_per_set,
+    bool init_borrowed( const st_dev_particles_t* views, const uint64_t* lat, const uint64_t* hot,
+                        int64_t n_elem_per_set,
                         int64_t S, unsigned char* d_region, size_t region_bytes, int32_t* h_region,
                         unsigned char* h_stage, int device_cu, hipStream_t stream )
     {
@@ -342,6 +358,7 @@ struct BatchRunner
         {
             hs[ s ].P = views[ s ];
             hs[ s ].lat = lat;
+            hs[ s ].hot = hot;
             hs[ s ].n_elem = n_elem_per_set;
             hs[ s ].list = d_lists + list_off;
             list_off += n_part[ s ];
@@ -419,7 +436,7 @@ struct BatchRunner
 
     int grid() const
     {
-        int const waves_per_block = ( cfg.lds() ? 256 : cfg.block ) / 64;
+        int const waves_per_block = cfg.walk() ? 1 : ( cfg.lds() ? 256 : cfg.block ) / 64;
         int const g = ( n_cu > 0 ? n_cu : 256 ) * cfg.waves_per_cu / waves_per_block;
         return g < cfg.queues ? cfg.queues : g;
     }
@@ -452,9 +469,9 @@ struct BatchRunner
             if( !enqueue_reset_select( until_turn, stream ) ) return false;
             hipError_t const e = cfg.fma
                 ? st_launch_batch_track_fma( &s, until_turn, k, d_status, cfg.block, grid(), cfg.ppl,
-                                             cfg.heavy ? 1 : 0, cfg.lds() ? 1 : 0, stream )
+                                             cfg.heavy ? 1 : 0, cfg.lds() ? 1 : 0, cfg.walk() ? 1 : 0, stream )
                 : st_launch_batch_track_exact( &s, until_turn, k, d_status, cfg.block, grid(), cfg.ppl,
-                                               cfg.heavy ? 1 : 0, cfg.lds() ? 1 : 0, stream );
+                                               cfg.heavy ? 1 : 0, cfg.lds() ? 1 : 0, cfg.walk() ? 1 : 0, stream );
             if( !hip_ok( e, "launch batch track" ) ) return false;
         }
         return true;
@@ -547,12 +564,16 @@ struct BatchRunner
     bool enqueue_track_split( int64_t until_turn, int64_t k, int32_t* d_status, int g,
                               hipStream_t stream ) const
     {
-        st_batch_sched_t const s = sched_split();
+        st_batch_sched_t s = sched_split();
+        // with one wave per SIMD there is nothing to put first, and the
+        // counter of the turns done (one atomic per wave and turn) is only
+        // a cost: 12 us per turn with 1,024 waves
+        if( cfg.walk() && g <= 4 * n_cu ) s.wave_prio = 0;
         hipError_t const e = cfg.fma
             ? st_launch_batch_track_fma( &s, until_turn, k, d_status, cfg.block, g, cfg.ppl,
-                                         cfg.heavy ? 1 : 0, cfg.lds() ? 1 : 0, stream )
+                                         cfg.heavy ? 1 : 0, cfg.lds() ? 1 : 0, cfg.walk() ? 1 : 0, stream )
             : st_launch_batch_track_exact( &s, until_turn, k, d_status, cfg.block, g, cfg.ppl,
-                                           cfg.heavy ? 1 : 0, cfg.lds() ? 1 : 0, stream );
+                                           cfg.heavy ? 1 : 0, cfg.lds() ? 1 : 0, cfg.walk() ? 1 : 0, stream );
         return hip_ok( e, "launch batch track" );
     }
 
@@ -579,18 +600,10 @@ struct BatchRunner
     //     pairs); used when n fills at least 90 % of the lanes (part-filled
     //     single waves cost as much as full ones).  For j = 16 every wave
     //     is a pair wave and n is spread evenly over them.
-    //   * At most one per resident lane: j = ceil(n / (64 x 4 x n_cu))
-    //     waves per SIMD hold n one per lane, and one wave per 64-particle
-    //     tile would leave some SIMDs with j waves and the others with
-    //     j - 1, idle once their waves end.  For 2 <= j <= 7 the launch
-    //     spreads n evenly over j waves on every SIMD (m = 0); for j = 8,
-    //     over 6 waves of which m = 2 pairs (the same lanes; up to 5 %
-    //     faster than one wave per tile in the FMA build and 8 % in the
-    //     exact build where the tiles leave lanes empty, equal where they
-    //     fill them).
+    //   * At most one per resident lane: no mixed launch, the scheduled record
+    //     walk with one particle per lane is faster (Config::walk).
     // false when the launch does not apply (several seeds, particles at
-    // several turns, a grid other than 8 workgroups of 256 per CU, at most
-    // one wave per SIMD).
+    // several turns, a grid other than 8 workgroups of 256 per CU).
     bool mix_shape( int64_t n, int64_t& pairs, int& grid_wgs ) const
     {
         pairs = 0;
@@ -608,21 +621,14 @@ struct BatchRunner
             // wave, n spread evenly over them (128-particle tiles would
             // leave whole waves idle)
             pairs = W;
-            grid_wgs = grid();
+            grid_wgs = 8 * n_cu;
             return true;
         }
-        if( n > 64 * W )
-        {
-            int64_t const w = ( j + 2 ) / 2, m = j - w;
-            if( w > 8 || 100 * n < 90 * j * per ) return false;
-            pairs = m * 4 * ( int64_t )n_cu;
-            grid_wgs = ( int )( w * n_cu );
-            return true;
-        }
-        if( j < 2 ) return false;
-        int64_t const m = j == 8 ? 2 : 0;
+        if( n <= 64 * W ) return false;
+        int64_t const w = ( j + 2 ) / 2, m = j - w;
+        if( w > 8 || 100 * n < 90 * j * per ) return false;
         pairs = m * 4 * ( int64_t )n_cu;
-        grid_wgs = ( int )( ( j - m ) * n_cu );
+        grid_wgs = ( int )( w * n_cu );
         return true;
     }
 

@@ -310,10 +310,17 @@ ST_DEV void srotation( Lane& p, cptr_t e )
 {
     double const cos_z = rd( e, 0 ), sin_z = rd( e, 1 );
     double const x = p.x, y = p.y, px = p.px, py = p.py;
+#if defined( ST_FMA_BUILD )
+    p.x = fma( cos_z, x, sin_z * y );
+    p.y = fma( cos_z, y, -( sin_z * x ) );
+    p.px = fma( cos_z, px, sin_z * py );
+    p.py = fma( cos_z, py, -( sin_z * px ) );
+#else
     p.x = cos_z * x + sin_z * y;
     p.y = -sin_z * x + cos_z * y;
     p.px = cos_z * px + sin_z * py;
     p.py = -sin_z * px + cos_z * py;
+#endif
 }
 
 // Aperture predicates (the caller applies state &= ok,

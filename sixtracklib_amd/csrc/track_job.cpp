@@ -31,6 +31,7 @@
 #include "track_launch.h"
 #include "batch.h"
 #include "batch_runner.h"
+#include "lattice_hot.h"
 
 // Scratch memory of NS(TrackJob_track_until_noalloc): the scheduler's
 // per-call device arrays (status word, seed descriptors, counts, queues,
@@ -214,7 +215,9 @@ struct NS(TrackJobBase)
     hipStream_t stream = nullptr;
     unsigned char* d_pbuf = nullptr; size_t pbuf_bytes = 0;
     unsigned char* d_obuf = nullptr; size_t obuf_bytes = 0;
+    // packed lattice, and behind it the hot stream of the same lattice
     uint64_t* d_lat = nullptr; int64_t lat_words = 0, n_elem = 0;
+    size_t hot_words_at = 0;
     std::vector< uint32_t > rec_offsets, monitor_fields;
     std::vector< uint64_t > lat_host;
     bool lat_full = false;
@@ -226,6 +229,7 @@ struct NS(TrackJobBase)
     int queues = 1;
     int ppl = 0;                         // particles per lane of the lean until path (0: auto)
     bool mix = true;                     // with ppl auto: mixed one/two-particle launches
+    int hot = -1;                        // scheduled record walk (track_hot.h): auto, never, always
     bool balance = true;                 // one tile per wave and launch, furthest behind first
     bool wave_prio = true;               // waves with more turns left issue first
     int staging = 0;                     // lean until path: lattice via scalar loads or LDS
@@ -478,6 +482,11 @@ struct NS(TrackJobBase)
                 }
             }
         }
+        hot_words_at = ( lat_host.size() + 31u ) & ~( size_t )31u;
+        std::vector< uint64_t > const hot = st::hot_stream( lat_host.data() );
+        lat_host.reserve( hot_words_at + hot.size() );
+        lat_host.resize( hot_words_at, 0u );
+        lat_host.insert( lat_host.end(), hot.begin(), hot.end() );
         if( d_lat ) { ( void )hipFree( d_lat ); d_lat = nullptr; }
         if( !hip_ok( hipMalloc( &d_lat, lat_host.size() * 8u ), "hipMalloc lattice" ) ) return false;
         return hip_ok( hipMemcpyAsync( d_lat, lat_host.data(), lat_host.size() * 8u,
@@ -650,6 +659,7 @@ struct NS(TrackJobBase)
         c.ppl_auto = !lat_full && ppl == 0 && staging == 0 && fma;
         c.mix = mix && !lat_full && ppl == 0 && staging == 0;
         c.balance = balance;
+        c.hot = hot;
         c.wave_prio = wave_prio;
         c.staging = ( lat_full || c.ppl == 2 ) ? 0 : staging;
         // resident waves per CU: 8 per SIMD (the lean kernels' register
@@ -670,6 +680,7 @@ struct NS(TrackJobBase)
         {
             st_batch_seed_t sd{};
             sd.P = v; sd.lat = d_lat; sd.n_elem = n_elem; sd.list = nullptr;
+            sd.hot = d_lat + hot_words_at;
             seeds.push_back( sd );
         }
         runner_ready = runner.init( seeds, stream );
@@ -735,7 +746,7 @@ struct NS(TrackJobBase)
         {
             na_runner.cfg = runner_config();
             na_runner.max_record_words = max_rec_words;
-            ok = na_runner.init_borrowed( views.data(), d_lat, n_elem, S,
+            ok = na_runner.init_borrowed( views.data(), d_lat, d_lat + hot_words_at, n_elem, S,
                                           base + ST_NOALLOC_STATUS_BYTES,
                                           ST_NOALLOC_SCRATCH_BYTES - ST_NOALLOC_STATUS_BYTES,
                                           na_host, na_stage, n_cu, stream );
@@ -852,6 +863,7 @@ struct NS(TrackJobBase)
             else if( k == "queues" ) queues = ( iv == 8 ) ? 8 : 1;
             else if( k == "ppl" ) ppl = ( v == "auto" ) ? 0 : ( iv == 2 ) ? 2 : 1;
             else if( k == "mix" ) mix = iv != 0;
+            else if( k == "hot" ) hot = ( v == "auto" ) ? -1 : ( iv != 0 ? 1 : 0 );
             else if( k == "balance" ) balance = iv != 0;
             else if( k == "wave_prio" ) wave_prio = iv != 0;
             else if( k == "staging" ) staging = ( v == "lds" || v == "1" ) ? 1 : 0;

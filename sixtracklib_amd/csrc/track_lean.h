@@ -21,6 +21,8 @@
 //     and a stored loss writes state 0.
 #pragma once
 
+#include <type_traits>
+
 #include "track_device.h"
 #include "track_heavy.h"
 
@@ -251,12 +253,18 @@ ST_DEV void lean_turn( const PA& pa, int64_t i, int64_t li, cptr_t lat, Lane& L,
 //   lat        packed lean lattice of n_elem records (END-terminated)
 //   max_turns  turns this launch may advance a lane (<= 0: until_turn)
 //   wp         issue priority of the wave (wave_priority)
+//   turn       another walk for the turns that every lane starts at s = +0
+//              (track_hot.h), or NoTurn
 // The OR of the per-particle statuses goes to *status_out.
-template< bool HEAVY = false, class PA = PDirect >
+struct NoTurn {};
+
+template< bool HEAVY = false, class PA = PDirect, class Turn = NoTurn >
 ST_DEV void track_lean_lane( const PA& pa, const int32_t* list, int64_t n_lanes,
                              int64_t tid, cptr_t lat, int64_t n_elem, int64_t until_turn,
-                             int64_t max_turns, int32_t* status_out, const WavePrio& wp = WavePrio() )
+                             int64_t max_turns, int32_t* status_out, const WavePrio& wp = WavePrio(),
+                             const Turn& turn = Turn() )
 {
+    constexpr bool OWN_TURN = !std::is_same< Turn, NoTurn >::value;
     bool const in_range = tid < n_lanes;
     int64_t const i = ( list != nullptr && in_range ) ? ( int64_t )list[ tid ] : tid;
     int64_t const li = in_range ? i : 0;          // out-of-range lanes never store
@@ -293,7 +301,13 @@ ST_DEV void track_lean_lane( const PA& pa, const int32_t* list, int64_t n_lanes,
         // record's s (lattice.h), kept in a scalar register and written only
         // when a lane is lost.  Lattices with monitors (HEAVY) store whole
         // particles mid-turn and keep the per-lane s.
-        if constexpr( HEAVY )
+        if constexpr( OWN_TURN )
+        {
+            if( ballot( lane_in( act ) && __double_as_longlong( L.s ) != 0 ) != 0u )
+                lean_turn< HEAVY, true >( pa, i, li, lat, L, chi, act, status, start, at_turn );
+            else turn( i, li, L, chi, act, status, start, at_turn );
+        }
+        else if constexpr( HEAVY )
             lean_turn< true, true >( pa, i, li, lat, L, chi, act, status, start, at_turn );
         else if( ballot( lane_in( act ) && __double_as_longlong( L.s ) != 0 ) != 0u )
             lean_turn< false, true >( pa, i, li, lat, L, chi, act, status, start, at_turn );
