@@ -139,8 +139,11 @@ struct Config
     // build and FMA build, loop / walk): 65,536 particles 198 / 88 and
     // 169 / 63; 131,072: 212 / 125 and 178 / 91; 262,144: 284 / 229 and
     // 242 / 156; 400,000: 411 / 372 and 307 / 255; 524,288: 478 / 424 and
-    // 344 / 328.
-    bool walk() const { return hot != 0 && ppl == 1 && !heavy && !lds(); }
+    // 344 / 328.  Lattices with the out-of-line maps run its heavy variant:
+    // 1,048,576 particles on the 20,019-element ring with beam-beam and
+    // space charge 1108 / 1026 and 905 / 750, 100,000 308 / 141 and
+    // 290 / 105.
+    bool walk() const { return hot != 0 && ppl == 1 && !lds(); }
 
     // the LDS-staged kernel runs lean lattices with one particle per lane
     bool lds() const { return staging != 0 && !heavy; }
