@@ -114,7 +114,7 @@ __global__ void __launch_bounds__( 256 ) KN( st_k_batch_minturn )( st_batch_sche
     int64_t const i = ( int64_t )blockIdx.x * blockDim.x + threadIdx.x;
     int64_t const t = ( i < n ) ? ( ( const int64_t* )w[ 20 ] )[ i ] : 0;
     bool const want = i < n && ( ( const int64_t* )w[ 21 ] )[ i ] == 1 && t < until_turn;
-    int32_t m = want ? ( int32_t )( t < 0 ? 0 : ( t > INT32_MAX ? INT32_MAX : t ) ) : INT32_MAX;
+    int32_t m = want ? ( int32_t )( t < INT32_MIN ? INT32_MIN : ( t > INT32_MAX ? INT32_MAX : t ) ) : INT32_MAX;
     for( int off = 32; off > 0; off >>= 1 ) m = min( m, __shfl_xor( m, off ) );
     __shared__ int32_t part[ 4 ];
     if( __lane_id() == 0 ) part[ threadIdx.x >> 6 ] = m;
@@ -230,29 +230,42 @@ ST_DEV bool find_tile( const st_batch_sched_t& s, int qb, int qe, int t, int& se
 }
 
 // Tile loop of the persistent track kernels (HEAVY: lattices that also
-// hold the maps outside the lean set).
+// hold the maps outside the lean set; HOT: the scheduled record walk).
+// Without counts (HOT only): one launch of one wave per 64 particles of
+// seed 0, no list.
 template< bool HEAVY, bool HOT = false >
 ST_DEV void batch_track_tiles( const st_batch_sched_t& s, int64_t until_turn, int64_t max_turns,
                                int32_t* status )
 {
     ci32_t* const qbegin = ( ci32_t* )s.queue_begin;
-    int const nq = s.n_queues;
+    bool const direct = HOT && s.counts == nullptr;
+    int const nq = direct ? 1 : s.n_queues;
     int const q0 = ( int )( blockIdx.x % ( unsigned )nq );
-    bool const one_tile = s.split != nullptr;
+    bool const one_tile = direct || s.split != nullptr;
     WavePrio const wp = launch_priority< 64 >( s, max_turns );
     for( int qi = 0; qi < nq; ++qi )
     {
         int const q = ( q0 + qi ) % nq;
-        int const qb = qbegin[ q ], qe = qbegin[ q + 1 ];
+        int const qb = direct ? 0 : qbegin[ q ], qe = direct ? 0 : qbegin[ q + 1 ];
         for( ;; )
         {
-            int t = 0;
-            if( __lane_id() == 0 ) t = atomicAdd( &s.queue_next[ q ], 1 );
-            t = __builtin_amdgcn_readfirstlane( __shfl( t, 0 ) );
             int seed = 0, tile = 0;
-            int32_t count = 0;
+            int64_t count = 0;
             const int32_t* list = nullptr;
-            if( !find_tile< 64 >( s, qb, qe, t, seed, list, count, tile ) ) break;   // queue drained
+            if( direct )
+            {
+                tile = ( int )blockIdx.x;
+                count = ( int64_t )( ( cptr_t )s.seeds )[ 0 ];
+            }
+            else
+            {
+                int t = 0;
+                if( __lane_id() == 0 ) t = atomicAdd( &s.queue_next[ q ], 1 );
+                t = __builtin_amdgcn_readfirstlane( __shfl( t, 0 ) );
+                int32_t n = 0;
+                if( !find_tile< 64 >( s, qb, qe, t, seed, list, n, tile ) ) break;   // queue drained
+                count = n;
+            }
             if constexpr( HOT )
             {
                 cptr_t const w = ( cptr_t )s.seeds + 26 * seed;
@@ -493,6 +506,8 @@ extern "C" hipError_t KN( st_launch_batch_track )( const st_batch_sched_t* s,
     int particles_per_lane, int heavy, int staging, int hot, hipStream_t stream )
 {
     if( s->n_seeds <= 0 || s->n_queues <= 0 ) return hipSuccess;
+    if( s->counts == nullptr && ( !hot || staging || particles_per_lane != 1 || s->n_seeds != 1 ) )
+        return hipErrorInvalidValue;
     if( block <= 0 || block > 256 || ( block % 64 ) != 0 ) block = 256;
     if( grid <= 0 ) grid = 1;
     if( staging && !heavy )

@@ -719,6 +719,8 @@ struct BatchRunner
                 // turns, and the next group decides again
                 if( launches++ >= limit ) return fail( "balanced tracking made no progress" );
                 if( !enqueue_track_mix( until_turn, k, d_status, pairs, mix_grid, stream ) ) return false;
+                // every active particle sat at min_turn and was in the launch
+                if( min_turn > INT32_MIN && k >= until_turn - min_turn ) return true;
                 continue;
             }
             int64_t const v = ( until_turn - min_turn + k - 1 ) / k;     // visits per particle
@@ -730,6 +732,13 @@ struct BatchRunner
                 if( j > 0 && !enqueue_select_split( until_turn, stream ) ) return false;
                 if( !enqueue_track_split( until_turn, k, d_status, g, stream ) ) return false;
             }
+            // One set with all its active particles at one turn and a wave for
+            // every tile: each launch advanced all that were left by k turns,
+            // so none is left and no further select pass has to say so.
+            // (A min_turn below the int32 range reads as its lowest value.)
+            if( n_seeds() == 1 && h_split[ 1 ] == 0 && tiles <= W && min_turn > INT32_MIN &&
+                n * k >= until_turn - min_turn )
+                return true;
         }
     }
 

@@ -49,10 +49,21 @@
 
 namespace st
 {
+/* Where the elements of a lattice are in its hot stream: entry i for element
+ * i, one more entry for the end of the lattice. */
+struct HotMap
+{
+    std::vector< uint32_t > off;       /* byte offset of the record that holds it; bit 0
+                                          set for the Multipole of a Drift's record  */
+    std::vector< uint32_t > handler;   /* handler offset of that record              */
+    std::vector< uint64_t > s;         /* path length before it, on a turn from s = 0 */
+};
+
 /* hot stream of the packed lattice ``lat`` (END-terminated), padding
  * included */
-inline std::vector< uint64_t > hot_stream( const uint64_t* lat )
+inline std::vector< uint64_t > hot_stream( const uint64_t* lat, HotMap* map = nullptr )
 {
+    if( map ) *map = HotMap();
     size_t end = 0;
     while( ST_REC_OP( lat[ end ] ) != ST_OP_END ) end += ST_REC_LEN( lat[ end ] );
     std::vector< uint64_t > w;
@@ -61,13 +72,23 @@ inline std::vector< uint64_t > hot_stream( const uint64_t* lat )
     size_t pos = 0, touched = 0;
     bool first = true;
     size_t last = 0, records = 0;
+    uint64_t s_before = 0;
+    uint32_t handler = 0;
     auto put = [ & ]( unsigned kind, size_t at )
     {
         // the record before names this one's handler
-        if( records > 0 ) w[ last ] |= kind * ST_HOT_SPACING + ( records % 2 ) * ST_HOT_SET_B;
+        handler = ( uint32_t )( kind * ST_HOT_SPACING + ( records % 2 ) * ST_HOT_SET_B );
+        if( records > 0 ) w[ last ] |= handler;
         last = w.size();
         ++records;
         w.push_back( ( uint64_t )( at * 8u ) << 32 );
+    };
+    auto element = [ & ]( unsigned second, uint64_t path )
+    {
+        if( map == nullptr ) return;
+        map->off.push_back( ( uint32_t )( last * 8u ) | second );
+        map->handler.push_back( handler );
+        map->s.push_back( path );
     };
     auto is_flat_mp = [ & ]( uint64_t h )
     { return ST_REC_OP( h ) == ST_OP_MULTIPOLE && ST_REC_AUX( h ) <= ST_HOT_MAX_ORDER; };
@@ -88,6 +109,7 @@ inline std::vector< uint64_t > hot_stream( const uint64_t* lat )
             first = false;
             put( ST_HOT_TOUCH, pos );
         }
+        s_before = s;
         uint64_t const h = lat[ pos ];
         const uint64_t* const e = lat + pos + ST_REC_PAYLOAD;
         size_t const next = pos + ST_REC_LEN( h );
@@ -101,6 +123,8 @@ inline std::vector< uint64_t > hot_stream( const uint64_t* lat )
                 put( ST_HOT_DRIFT_MP + ST_REC_AUX( lat[ next ] ), pos );
                 w.push_back( e[ 0 ] );
                 put_mp( next );
+                element( 0u, s_before );
+                element( 1u, s );
                 pos = next + ST_REC_LEN( lat[ next ] );
                 continue;
             }
@@ -135,6 +159,7 @@ inline std::vector< uint64_t > hot_stream( const uint64_t* lat )
             w.push_back( s );
             break;
         }
+        element( 0u, s_before );
         if( ST_REC_OP( h ) == ST_OP_END ) break;
         pos = next;
     }

@@ -43,6 +43,13 @@ ST_DEV bool lane_in( uint64_t m ) { return ( ( m >> __lane_id() ) & 1u ) != 0u; 
 ST_DEV double rd( cptr_t p, int k ) { return __longlong_as_double( ( long long )p[ k ] ); }
 ST_DEV int64_t ri( cptr_t p, int k ) { return ( int64_t )p[ k ]; }
 
+// A map failed: the call's status word becomes -1, the only status there is
+// besides 0.  A plain store, so that the word may also be host memory.
+ST_DEV void report_failure( int32_t* status_out )
+{
+    __hip_atomic_store( status_out, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM );
+}
+
 struct Lane
 {
     double x, px, y, py, zeta, delta, rpp, rvv, psigma, s;

@@ -185,6 +185,10 @@ namespace st
 // the aperture tests give the lost lanes directly.
 #define ST_HOT_HANDLERS R"(
 .macro ST_PRO X, Y, size
+.if %c[stops]
+  s_cmp_eq_u32 %[off], %[stop]
+  s_cbranch_scc1 .Lstop%=
+.endif
   s_waitcnt lgkmcnt(0)
 .if \size > 128
   s_load_dwordx16 s[68:83], %[hot], %[off] offset:64
@@ -314,14 +318,15 @@ namespace st
   s_addc_u32 s35, s35, 0
   s_add_u32 s34, s100, 0xffff
   s_cselect_b32 %[info], -1, 0
-  s_mov_b64 %[lost], 0
   s_cbranch_scc1 .Lnone%=
   s_add_u32 s34, s100, %[next]
   s_setpc_b64 s[34:35]
   ST_HANDLERS 36, 52, a
 .org .Latable%=+%c[setb]
   ST_HANDLERS 52, 36, b
+.Lstop%=:
 .Lnone%=:
+  s_mov_b64 %[lost], 0
   s_waitcnt lgkmcnt(0)
 .Lend%=:
   s_mov_b64 exec, %[exec]
@@ -342,8 +347,12 @@ namespace st
 #define ST_HOT_PURGE ".purgem ST_SUMS\n"
 #endif
 
-ST_DEV void hot_run( cptr_t hot, uint32_t& off, uint32_t& next, Lane& L, double const chi,
-                     uint64_t const act, uint64_t& lost, uint32_t& info )
+// With STOP the walk also returns at the record at byte offset ``stop``,
+// before running it (off = stop, lost = 0): one compare and branch more per
+// record, for segments of a lattice.
+template< bool STOP >
+ST_DEV void hot_run( cptr_t hot, uint32_t& off, uint32_t& next, uint32_t const stop, Lane& L,
+                     double const chi, uint64_t const act, uint64_t& lost, uint32_t& info )
 {
 #if defined( __HIP_DEVICE_COMPILE__ )
     double t0, t1, t2, t3;
@@ -354,40 +363,49 @@ ST_DEV void hot_run( cptr_t hot, uint32_t& off, uint32_t& next, Lane& L, double 
           [ info ] "=&s"( info ), [ m ] "=&s"( m ), [ exec ] "=&s"( exec ), [ t0 ] "=&v"( t0 ),
           [ t1 ] "=&v"( t1 ), [ t2 ] "=&v"( t2 ), [ t3 ] "=&v"( t3 )
         : [ rpp ] "v"( L.rpp ), [ rvv ] "v"( L.rvv ), [ chi ] "v"( chi ), [ hot ] "s"( hot ),
-          [ act ] "s"( act ), [ lines ] "n"( ST_HOT_TOUCH_LINES ), [ ahead ] "n"( ST_HOT_TOUCH_AHEAD ),
+          [ act ] "s"( act ), [ stop ] "s"( stop ), [ stops ] "n"( STOP ? 1 : 0 ),
+          [ lines ] "n"( ST_HOT_TOUCH_LINES ), [ ahead ] "n"( ST_HOT_TOUCH_AHEAD ),
           [ setb ] "n"( ST_HOT_SET_B )
         : "vcc", "scc", ST_HOT_SGPRS );
 #endif
 }
 
-// One turn of a lean until-turn lane whose particles all start it at s = +0,
-// through the hot stream: lean_turn<HEAVY, false> of track_lean.h with the
-// records of the hot kinds run by hot_run.
-template< bool HEAVY, class PA >
-ST_DEV void lean_turn_hot( const PA& pa, int64_t i, int64_t li, cptr_t lat, cptr_t hot, Lane& L,
-                           double chi, uint64_t& act, int32_t& status, int64_t start, int64_t at_turn )
+// The lanes ``lost`` leave at the element of the packed record r: their
+// state is stored, with path length s (bits).
+template< class PA >
+ST_DEV void hot_lose( const PA& pa, int64_t i, Lane& L, uint64_t lost, uint64_t& act, uint64_t s,
+                      int64_t at_element, int64_t at_turn )
 {
-    uint32_t off = 0, next = ST_HOT_TOUCH * ST_HOT_SPACING;      // a stream starts with a TOUCH
+    if( lane_in( lost ) )
+    {
+        L.s = __longlong_as_double( ( long long )s );
+        store_lane_state( pa.view(), i, L, 0, at_element, at_turn );
+    }
+    act &= ~lost;
+}
+
+// The hot records from byte offset off (handler offset next) to the END
+// record, or with STOP to the record at byte offset stop, for lanes that
+// came to off with the path length the stream holds for it: the element loop
+// of track_lean.h's lean_turn<HEAVY, false> with the records of the hot
+// kinds run by hot_run.  False when nothing was run (hot_run, info = ~0).
+template< bool HEAVY, bool STOP, class PA >
+ST_DEV bool hot_walk( const PA& pa, int64_t i, int64_t li, cptr_t lat, cptr_t hot, uint32_t off,
+                      uint32_t next, uint32_t stop, Lane& L, double chi, uint64_t& act,
+                      int32_t& status, int64_t start, int64_t at_turn )
+{
     while( act != 0u )
     {
+        if( STOP && off == stop ) break;
         uint64_t lost;
         uint32_t info;
-        hot_run( hot, off, next, L, chi, act, lost, info );
-        if( info == ~0u )
-        {
-            lean_turn< HEAVY, true >( pa, i, li, lat, L, chi, act, status, start, at_turn );
-            return;
-        }
+        hot_run< STOP >( hot, off, next, stop, L, chi, act, lost, info );
+        if( info == ~0u ) return false;
         if( lost != 0u )                              // at a Drift or an aperture
         {
             cptr_t const r = rec_at( lat, info & ~1u );
             uint64_t const s = ST_REC_OP( r[ 0 ] ) == ST_OP_DRIFT ? r[ 3 ] : rec_at( hot, off - 8u )[ 0 ];
-            if( lane_in( lost ) )
-            {
-                L.s = __longlong_as_double( ( long long )s );
-                store_lane_state( pa.view(), i, L, 0, start + ri( r, 1 ), at_turn );
-            }
-            act &= ~lost;
+            hot_lose( pa, i, L, lost, act, s, start + ri( r, 1 ), at_turn );
             if( info & 1u )                           // the Multipole of the same hot record
             {
                 cptr_t const m = r + ST_REC_LEN( r[ 0 ] );
@@ -395,6 +413,7 @@ ST_DEV void lean_turn_hot( const PA& pa, int64_t i, int64_t li, cptr_t lat, cptr
             }
             continue;
         }
+        if( STOP && off == stop ) break;
         cptr_t const x = rec_at( hot, off );
         cptr_t const r = rec_at( lat, info );
         uint64_t const h = r[ 0 ];
@@ -415,15 +434,11 @@ ST_DEV void lean_turn_hot( const PA& pa, int64_t i, int64_t li, cptr_t lat, cptr
         uint64_t const gone = ballot( !ok ) & act;
         if( gone != 0u )
         {
-            if( lane_in( gone ) )
-            {
-                L.s = __longlong_as_double( ( long long )x[ 1 ] );
-                store_lane_state( pa.view(), i, L, 0, start + ri( r, 1 ), at_turn );
-                if( fail ) status = -1;
-            }
-            act &= ~gone;
+            if( lane_in( gone ) && fail ) status = -1;
+            hot_lose( pa, i, L, gone, act, x[ 1 ], start + ri( r, 1 ), at_turn );
         }
     }
+    return true;
 }
 
 // As track_lean_lane, the turns through the hot stream.  A turn on which
@@ -437,7 +452,12 @@ ST_DEV void track_hot_lane( const PA& pa, const int32_t* list, int64_t n_lanes, 
     track_lean_lane< HEAVY >( pa, list, n_lanes, tid, lat, n_elem, until_turn, max_turns, status_out, wp,
         [ & ]( int64_t i, int64_t li, Lane& L, double chi, uint64_t& act, int32_t& status, int64_t start,
                int64_t at_turn )
-        { lean_turn_hot< HEAVY >( pa, i, li, lat, hot, L, chi, act, status, start, at_turn ); } );
+        {
+            // a stream starts with a TOUCH record
+            if( !hot_walk< HEAVY, false >( pa, i, li, lat, hot, 0u, ST_HOT_TOUCH * ST_HOT_SPACING, 0u, L,
+                                           chi, act, status, start, at_turn ) )
+                lean_turn< HEAVY, true >( pa, i, li, lat, L, chi, act, status, start, at_turn );
+        } );
 }
 
 }  // namespace st

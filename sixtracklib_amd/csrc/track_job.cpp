@@ -217,11 +217,14 @@ struct NS(TrackJobBase)
     unsigned char* d_obuf = nullptr; size_t obuf_bytes = 0;
     // packed lattice, and behind it the hot stream of the same lattice
     uint64_t* d_lat = nullptr; int64_t lat_words = 0, n_elem = 0;
-    size_t hot_words_at = 0;
+    // and the descriptors of the particle sets on it (batch.h, no lists)
+    size_t hot_words_at = 0, desc_words_at = 0;
+    st::HotMap hot_map;
+    bool lat_fails = false;              // holds a disabled map (ST_OP_FAIL)
     std::vector< uint32_t > rec_offsets, monitor_fields;
     std::vector< uint64_t > lat_host;
     bool lat_full = false;
-    int32_t* d_status = nullptr; int32_t* h_status = nullptr;
+    int32_t* h_status = nullptr;         // pinned, written by the kernels
     bool compact = true;                 // lean lattices: persistent tiles over active particles
     int64_t turns_per_launch = 0;        // 0: from the work size
     // one tile queue: a job's sets share one lattice, and with a queue per
@@ -326,7 +329,6 @@ struct NS(TrackJobBase)
         if( d_pbuf ) ( void )hipFree( d_pbuf );
         if( d_obuf ) ( void )hipFree( d_obuf );
         if( d_lat ) ( void )hipFree( d_lat );
-        if( d_status ) ( void )hipFree( d_status );
         runner.release();
         runner_ready = false;
         na_runner.release();
@@ -337,7 +339,7 @@ struct NS(TrackJobBase)
         if( ev_start ) ( void )hipEventDestroy( ev_start );
         if( ev_stop ) ( void )hipEventDestroy( ev_stop );
         if( stream ) ( void )hipStreamDestroy( stream );
-        d_pbuf = d_obuf = nullptr; d_lat = nullptr; d_status = nullptr;
+        d_pbuf = d_obuf = nullptr; d_lat = nullptr;
         h_status = nullptr; stream = nullptr; ev_start = ev_stop = nullptr;
         if( owns_obuf && obuf ) NS(Buffer_delete)( obuf );
         obuf = nullptr; owns_obuf = false;
@@ -458,11 +460,13 @@ struct NS(TrackJobBase)
         n_elem = n_elem_l;
         lat_words = nw;
         lat_full = false;
+        lat_fails = false;
         max_rec_words = 0;
         for( int64_t i = 0; i < n_elem; ++i )
         {
             unsigned const op = ST_REC_OP( lat_host[ rec_offsets[ i ] ] );
             if( !ST_OP_IS_LEAN( op ) ) lat_full = true;
+            if( op == ST_OP_FAIL ) lat_fails = true;
             max_rec_words = std::max< int64_t >( max_rec_words, rec_offsets[ i + 1 ] - rec_offsets[ i ] );
         }
         // point the monitors that have an output set at its device header
@@ -483,12 +487,19 @@ struct NS(TrackJobBase)
             }
         }
         hot_words_at = ( lat_host.size() + 31u ) & ~( size_t )31u;
-        std::vector< uint64_t > const hot = st::hot_stream( lat_host.data() );
+        std::vector< uint64_t > const hot = st::hot_stream( lat_host.data(), &hot_map );
         lat_host.reserve( hot_words_at + hot.size() );
         lat_host.resize( hot_words_at, 0u );
         lat_host.insert( lat_host.end(), hot.begin(), hot.end() );
+        desc_words_at = ( lat_host.size() + 31u ) & ~( size_t )31u;
+        lat_host.resize( desc_words_at + views.size() * sizeof( st_batch_seed_t ) / 8u, 0u );
         if( d_lat ) { ( void )hipFree( d_lat ); d_lat = nullptr; }
         if( !hip_ok( hipMalloc( &d_lat, lat_host.size() * 8u ), "hipMalloc lattice" ) ) return false;
+        for( size_t k = 0; k < views.size(); ++k )
+        {
+            st_batch_seed_t sd = seed( k );
+            std::memcpy( lat_host.data() + desc_words_at + k * sizeof( sd ) / 8u, &sd, sizeof( sd ) );
+        }
         return hip_ok( hipMemcpyAsync( d_lat, lat_host.data(), lat_host.size() * 8u,
                                        hipMemcpyHostToDevice, stream ), "upload lattice" ) &&
                hip_ok( hipStreamSynchronize( stream ), "hipStreamSynchronize" );
@@ -570,7 +581,6 @@ struct NS(TrackJobBase)
         if( !hip_ok( hipStreamCreate( &stream ), "hipStreamCreate" ) ) return false;
         if( !hip_ok( hipEventCreate( &ev_start ), "hipEventCreate" ) ||
             !hip_ok( hipEventCreate( &ev_stop ), "hipEventCreate" ) ) return false;
-        if( !hip_ok( hipMalloc( &d_status, sizeof( int32_t ) ), "hipMalloc status" ) ) return false;
         if( !hip_ok( hipHostMalloc( &h_status, sizeof( int32_t ) ), "hipHostMalloc" ) ) return false;
         if( !hip_ok( hipDeviceGetAttribute( &n_cu, hipDeviceAttributeMultiprocessorCount, device ),
                      "hipDeviceGetAttribute" ) ) return false;
@@ -596,9 +606,9 @@ struct NS(TrackJobBase)
             if( !hip_ok( hipMalloc( &d_obuf, obuf_bytes ), "hipMalloc output" ) ) return false;
             if( !upload_image( obuf, d_obuf, obuf_bytes ) ) return false;
         }
-        if( !pack_lattice() ) return false;
         views.clear();
         for( uint64_t k : sets ) views.push_back( device_view( pbuf, d_pbuf, k ) );
+        if( !pack_lattice() ) return false;
         if( plan.has_ebe ) ebe_view = device_view( obuf, d_obuf, ebe_offset );
         set_sizes_u64.assign( set_sizes.begin(), set_sizes.end() );
         monitor_indices_u64.assign( plan.monitor_elems.begin(), plan.monitor_elems.end() );
@@ -606,20 +616,19 @@ struct NS(TrackJobBase)
         return prepare_paddr();
     }
 
-    // status word cleared before and read back after the launches; the two
-    // events bracket the kernels on the job stream (kernel time only)
+    // the status word is pinned host memory that a kernel writes only when a
+    // map fails; every call ends with the stream idle.  The two events
+    // bracket the kernels on the job stream (kernel time only)
     bool begin_status()
     {
-        return hip_ok( hipMemsetAsync( d_status, 0, sizeof( int32_t ), stream ), "hipMemsetAsync" ) &&
-               hip_ok( hipEventRecord( ev_start, stream ), "hipEventRecord" );
+        *h_status = 0;
+        return hip_ok( hipEventRecord( ev_start, stream ), "hipEventRecord" );
     }
 
     int32_t end_status( bool launched_ok )
     {
-        if( !launched_ok ) { last_status = -1; return -1; }
+        if( !launched_ok ) { ( void )hipStreamSynchronize( stream ); last_status = -1; return -1; }
         if( !hip_ok( hipEventRecord( ev_stop, stream ), "hipEventRecord" ) ||
-            !hip_ok( hipMemcpyAsync( h_status, d_status, sizeof( int32_t ),
-                                     hipMemcpyDeviceToHost, stream ), "status D2H" ) ||
             !hip_ok( hipStreamSynchronize( stream ), "hipStreamSynchronize" ) )
         { last_status = -1; return -1; }
         float ms = 0.0f;
@@ -670,19 +679,53 @@ struct NS(TrackJobBase)
         return c;
     }
 
+    // particle set k on the job's lattice; the copy on the device
+    st_batch_seed_t seed( size_t k ) const
+    {
+        st_batch_seed_t sd{};
+        sd.P = views[ k ]; sd.lat = d_lat; sd.n_elem = n_elem; sd.list = nullptr;
+        sd.hot = d_lat + hot_words_at;
+        return sd;
+    }
+    const st_batch_seed_t* device_seed( size_t k ) const
+    {
+        return reinterpret_cast< const st_batch_seed_t* >( d_lat + desc_words_at ) + k;
+    }
+
+    // track_until of one particle set of at most one wave per SIMD: one
+    // launch of one wave per 64 particles, no select passes and no counts
+    // read back (a lost particle's lane costs such a launch nothing).  The
+    // launch is not split, so the request is bounded: 2^24 element passes,
+    // about 1.5 s.  402-element ring, 1,000 particles, one turn: 85 us of
+    // launches and waits less per call.
+    bool direct( int64_t until_turn ) const
+    {
+        return hot != 0 && ppl != 2 && staging == 0 && turns_per_launch == 0 && waves_per_cu == 0 &&
+               views.size() == 1u && views[ 0 ].n <= 64 * 4 * ( int64_t )n_cu &&
+               until_turn <= ( int64_t( 1 ) << 24 ) / n_elem;
+    }
+
+    bool launch_direct( int64_t until_turn, int32_t* status )
+    {
+        st_batch_sched_t s{};
+        s.seeds = device_seed( 0 );
+        s.n_seeds = 1;
+        s.n_queues = 1;
+        int const tiles = ( int )( ( views[ 0 ].n + 63 ) / 64 );
+        if( tiles == 0 ) return true;
+        hipError_t const e = fma
+            ? st_launch_batch_track_fma( &s, until_turn, 0, status, 64, tiles, 1, lat_full ? 1 : 0, 0, 1, stream )
+            : st_launch_batch_track_exact( &s, until_turn, 0, status, 64, tiles, 1, lat_full ? 1 : 0, 0, 1, stream );
+        return hip_ok( e, "launch track_until" );
+    }
+
     bool ensure_runner()
     {
         if( runner_ready ) return true;
         runner.cfg = runner_config();
         runner.max_record_words = max_rec_words;
         std::vector< st_batch_seed_t > seeds;
-        for( const st_dev_particles_t& v : views )
-        {
-            st_batch_seed_t sd{};
-            sd.P = v; sd.lat = d_lat; sd.n_elem = n_elem; sd.list = nullptr;
-            sd.hot = d_lat + hot_words_at;
-            seeds.push_back( sd );
-        }
+        for( size_t k = 0; k < views.size(); ++k ) seeds.push_back( seed( k ) );
         runner_ready = runner.init( seeds, stream );
         return runner_ready;
     }
@@ -694,22 +737,23 @@ struct NS(TrackJobBase)
         if( compact && n_elem > 0 )
         {
             int64_t n_active = 0, min_turn = 0;
+            if( balance && direct( until_turn ) ) return end_status( launch_direct( until_turn, h_status ) );
             if( balance ) return end_status( ensure_runner() &&
-                                             runner.run_balanced( until_turn, d_status, stream ) );
+                                             runner.run_balanced( until_turn, h_status, stream ) );
             ok = ensure_runner() && runner.select_sync( until_turn, stream, n_active, min_turn );
             if( ok && n_active > 0 )
             {
                 int64_t const k = runner.chunk_turns( n_active );
                 int64_t const chunks = ( until_turn - min_turn + k - 1 ) / k;
-                ok = runner.run( until_turn, chunks, k, d_status, stream );
+                ok = runner.run( until_turn, chunks, k, h_status, stream );
             }
             return end_status( ok );
         }
         for( const st_dev_particles_t& v : views )
         {
             hipError_t const err = fma
-                ? st_launch_track_until_fma( &v, d_lat, n_elem, until_turn, lat_full, d_status, block, stream )
-                : st_launch_track_until_exact( &v, d_lat, n_elem, until_turn, lat_full, d_status, block, stream );
+                ? st_launch_track_until_fma( &v, d_lat, n_elem, until_turn, lat_full, h_status, block, stream )
+                : st_launch_track_until_exact( &v, d_lat, n_elem, until_turn, lat_full, h_status, block, stream );
             ok = ok && hip_ok( err, "launch track_until" );
         }
         return end_status( ok );
@@ -805,8 +849,8 @@ struct NS(TrackJobBase)
         for( const st_dev_particles_t& v : views )
         {
             hipError_t const err = fma
-                ? st_launch_track_ebe_fma( &v, d_lat, n_elem, until_turn, &ebe_device_cfg(), plan.ebe_cap, &ebe_view, d_status, from_turn, block, stream )
-                : st_launch_track_ebe_exact( &v, d_lat, n_elem, until_turn, &ebe_device_cfg(), plan.ebe_cap, &ebe_view, d_status, from_turn, block, stream );
+                ? st_launch_track_ebe_fma( &v, d_lat, n_elem, until_turn, &ebe_device_cfg(), plan.ebe_cap, &ebe_view, h_status, from_turn, block, stream )
+                : st_launch_track_ebe_exact( &v, d_lat, n_elem, until_turn, &ebe_device_cfg(), plan.ebe_cap, &ebe_view, h_status, from_turn, block, stream );
             ok = ok && hip_ok( err, "launch track_elem_by_elem" );
         }
         return end_status( ok );
@@ -821,17 +865,51 @@ struct NS(TrackJobBase)
         return dev_cfg;
     }
 
+    // elements [b, e) in the hot stream
+    st_hot_segment_t hot_segment( uint64_t b, uint64_t e ) const
+    {
+        st_hot_segment_t seg{};
+        seg.begin = ( int64_t )b;
+        uint64_t first = b;
+        if( hot_map.off[ b ] & 1u )               // the Multipole of a Drift's record
+        {
+            seg.head = rec_offsets[ b ] * 8u;
+            ++first;
+        }
+        seg.off = hot_map.off[ first ];
+        seg.next = hot_map.handler[ first ];
+        seg.stop = hot_map.off[ e ] & ~1u;
+        if( first == e ) seg.stop = seg.off = hot_map.off[ e ] & ~1u;
+        else if( hot_map.off[ e ] & 1u ) seg.tail = rec_offsets[ e - 1 ] * 8u + 8u;
+        seg.s_begin = hot_map.s[ b ];
+        seg.s_end = hot_map.s[ e ];
+        return seg;
+    }
+
     int32_t track_line( uint64_t b, uint64_t e, bool finish )
     {
         if( b > e || e > ( uint64_t )n_elem ) { last_status = -1; return -1; }
         if( !begin_status() ) return end_status( false );
         bool ok = true;
         const uint64_t* lat = d_lat + rec_offsets[ b ];
+        if( hot != 0 && e > b && !lat_fails )
+        {
+            st_hot_segment_t seg = hot_segment( b, e );
+            for( size_t k = 0; k < views.size(); ++k )
+            {
+                seg.seed = device_seed( k );
+                hipError_t const err = fma
+                    ? st_launch_track_line_hot_fma( views[ k ].n, &seg, lat, ( int64_t )( e - b ), finish, lat_full, h_status, stream )
+                    : st_launch_track_line_hot_exact( views[ k ].n, &seg, lat, ( int64_t )( e - b ), finish, lat_full, h_status, stream );
+                ok = ok && hip_ok( err, "launch track_line" );
+            }
+            return end_status( ok );
+        }
         for( const st_dev_particles_t& v : views )
         {
             hipError_t const err = fma
-                ? st_launch_track_line_fma( &v, lat, ( int64_t )( e - b ), finish, d_status, block, stream )
-                : st_launch_track_line_exact( &v, lat, ( int64_t )( e - b ), finish, d_status, block, stream );
+                ? st_launch_track_line_fma( &v, lat, ( int64_t )( e - b ), finish, h_status, block, stream )
+                : st_launch_track_line_exact( &v, lat, ( int64_t )( e - b ), finish, h_status, block, stream );
             ok = ok && hip_ok( err, "launch track_line" );
         }
         return end_status( ok );

@@ -30,6 +30,7 @@
 
 #include "track_device.h"
 #include "track_lean.h"
+#include "track_hot.h"
 #include "track_launch.h"
 
 #ifndef ST_KSUFFIX
@@ -347,7 +348,7 @@ ST_DEV void track_body( const st_dev_particles_t& P, int64_t i, const Args& a )
         if( a.finish_turn ) { at_element = 0; ++at_turn; L.s = 0.0; }
         store_lane( P, i, L, at_element, at_turn );
     }
-    if( in_range && status != 0 ) atomicOr( a.status_out, status );
+    if( in_range && status != 0 ) report_failure( a.status_out );
 }
 
 ST_DEV void track_until_lean( const st_dev_particles_t& P, int64_t tid, const Args& a )
@@ -388,6 +389,83 @@ KN( st_k_track_ebe )( st_dev_particles_t P, Args a )
 __global__ void __launch_bounds__( 256 ) KN( st_k_track_line )( st_dev_particles_t P, Args a )
 {
     track_body< MODE_LINE, true >( P, ( int64_t )blockIdx.x * blockDim.x + threadIdx.x, a );
+}
+
+// track_line through the hot stream (track_hot.h): the segment's records
+// from seg.off to seg.stop, before them the Multipole and after them the
+// Drift of a record that the segment's ends cut in two.  Particles that
+// come with the path length a turn from s = 0 has at the segment's begin
+// (every segment of a turn tracked piece by piece) need no path length of
+// their own; a wave with any other runs the full kernel's loop.
+// HEAVY: the lattice holds maps outside the lean set.
+template< bool HEAVY >
+ST_DEV void track_line_hot( const Args& a, const st_hot_segment_t& seg )
+{
+    cptr_t const w = ( cptr_t )seg.seed;
+    PDesc const pa{ w };
+    int64_t const i = ( int64_t )blockIdx.x * blockDim.x + threadIdx.x;
+    Lane L;
+    double chi;
+    int64_t start, at_turn, li;
+    bool active0;
+    {
+        st_dev_particles_t const P = pa.view();
+        bool const in_range = i < P.n;
+        li = in_range ? i : 0;
+        L.x = P.x[ li ]; L.px = P.px[ li ]; L.y = P.y[ li ]; L.py = P.py[ li ];
+        L.zeta = P.zeta[ li ]; L.delta = P.delta[ li ]; L.rpp = P.rpp[ li ];
+        L.rvv = P.rvv[ li ]; L.psigma = P.psigma[ li ]; L.s = P.s[ li ];
+        chi = P.chi[ li ];
+        start = P.at_element[ li ];
+        at_turn = P.at_turn[ li ];
+        active0 = in_range && P.state[ li ] == 1;
+    }
+    cptr_t const lat = ( cptr_t )w[ 22 ], hot = ( cptr_t )w[ 25 ];
+    uint64_t act = ballot( active0 );
+    if( act == 0u ) return;
+    bool walked = ballot( active0 && ( uint64_t )__double_as_longlong( L.s ) != seg.s_begin ) == 0u;
+    int64_t const base = start - seg.begin;       // word 1 of a record is its element's index
+    int32_t status = 0;
+    if( walked )
+    {
+        L.s = 0.0;
+        if( seg.head != 0u )
+        {
+            cptr_t const r = rec_at( lat, seg.head );
+            multipole( L, chi, r + ST_REC_PAYLOAD, ST_REC_AUX( r[ 0 ] ), L.delta );
+        }
+        walked = hot_walk< HEAVY, true >( pa, i, li, lat, hot, seg.off, seg.next, seg.stop, L, chi, act,
+                                          status, base, at_turn );
+    }
+    if( !walked )                                 // nothing was stored yet
+    {
+        track_body< MODE_LINE, HEAVY >( pa.view(), i, a );
+        return;
+    }
+    if( seg.tail != 0u && act != 0u )
+    {
+        cptr_t const r = rec_at( lat, seg.tail - 8u );
+        drift_xz( L, rd( r, 2 ) );
+        uint64_t const lost = limit_global_lost_mask( L ) & act;
+        if( lost != 0u ) hot_lose( pa, i, L, lost, act, r[ 3 ], base + ri( r, 1 ), at_turn );
+    }
+    if( lane_in( act ) )
+    {
+        L.s = a.finish_turn ? 0.0 : __longlong_as_double( ( long long )seg.s_end );
+        store_lane_state( pa.view(), i, L, 1, a.finish_turn ? 0 : start + a.n_elem,
+                          a.finish_turn ? at_turn + 1 : at_turn );
+    }
+    if( status != 0 ) report_failure( a.status_out );
+}
+
+__global__ void __launch_bounds__( 64, 4 ) KN( st_k_track_line_hot )( Args a, st_hot_segment_t seg )
+{
+    track_line_hot< false >( a, seg );
+}
+
+__global__ void __launch_bounds__( 64, 4 ) KN( st_k_track_line_hot_heavy )( Args a, st_hot_segment_t seg )
+{
+    track_line_hot< true >( a, seg );
 }
 
 // ------------------------------------------------------------ launchers
@@ -507,5 +585,21 @@ extern "C" hipError_t KN( st_launch_track_line )( const st_dev_particles_t* P,
     a.status_out = status;
     hipLaunchKernelGGL( KN( st_k_track_line ), dim3( grid_for( P->n, block ) ), dim3( block ),
                         0, stream, *P, a );
+    return hipGetLastError();
+}
+
+extern "C" hipError_t KN( st_launch_track_line_hot )( int64_t n, const st_hot_segment_t* seg,
+    const uint64_t* lat, int64_t n_line, int finish_turn, int heavy, int32_t* status, hipStream_t stream )
+{
+    if( n <= 0 ) return hipSuccess;
+    Args a{};
+    a.lat = ( cptr_t )lat; a.n_elem = n_line; a.finish_turn = finish_turn != 0;
+    a.status_out = status;
+    if( heavy )
+        hipLaunchKernelGGL( KN( st_k_track_line_hot_heavy ), dim3( grid_for( n, 64 ) ), dim3( 64 ), 0,
+                            stream, a, *seg );
+    else
+        hipLaunchKernelGGL( KN( st_k_track_line_hot ), dim3( grid_for( n, 64 ) ), dim3( 64 ), 0, stream,
+                            a, *seg );
     return hipGetLastError();
 }

@@ -324,7 +324,7 @@ ST_DEV void track_lean_lane( const PA& pa, const int32_t* list, int64_t n_lanes,
         if( act != 0u ) wave_priority( wp, turns_done );
     }
     wave_priority_leave( wp, turns_done );
-    if( in_range && status != 0 ) atomicOr( status_out, status );
+    if( in_range && status != 0 ) report_failure( status_out );
 }
 
 // Store of a finished lane of the hot-state loop: delta and psigma are not
@@ -647,7 +647,7 @@ ST_DEV void track_lean_lane2( const PA& pa, const int32_t* list, int64_t n_lanes
         if( ( act[ 0 ] | act[ 1 ] ) != 0u ) wave_priority( wp, turns_done );
     }
     wave_priority_leave( wp, turns_done );
-    if( failed && __lane_id() == 0 ) atomicOr( status_out, -1 );
+    if( failed && __lane_id() == 0 ) report_failure( status_out );
 }
 
 // Indices of the particles a track_until call has work for (state 1 and

@@ -239,7 +239,7 @@ ST_DEV void track_lean_block( const st_dev_particles_t& P, const int32_t* list, 
             }
         }
     }
-    if( in_range && status != 0 ) atomicOr( status_out, status );
+    if( in_range && status != 0 ) report_failure( status_out );
 }
 
 }  // namespace st

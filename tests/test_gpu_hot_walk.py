@@ -108,3 +108,66 @@ def test_hot_walk_is_the_loop_and_the_oracle(n, n_blocks, lost_at_drift):
             if n >= 63:
                 alive = int(np.count_nonzero(loop["state"]))
                 assert 0 < alive < n
+
+
+def _run_lines(eb, pb, cfg, cuts, turns):
+    from sixtracklib_amd.trackjob import TrackJob
+    b = CBuffer.frombytes(pb.tobytes())
+    job = TrackJob(eb, b, config_str=cfg)
+    for _ in range(turns):
+        for lo, hi in zip(cuts, cuts[1:]):
+            job.track_line(lo, hi, finish_turn=hi == cuts[-1])
+    job.collect()
+    return particles_dict(particles_in(b))
+
+
+@pytest.mark.parametrize("n,n_blocks,step", [(1, 1, 1), (65, 1, 2), (200, 2, 3), (1000, 3, 17),
+                                             (1000, 3, 1000)])
+def test_hot_lines_are_the_full_kernel_and_track_until(n, n_blocks, step):
+    """track_line in pieces that cut records of a Drift and a Multipole in
+    two, against the full kernel (hot=0); with a wave of particles that
+    start at another path length (they keep their own), against it too."""
+    eb = _lattice(20 + n_blocks, n_blocks)
+    cuts = list(range(0, eb.n_objects, step)) + [eb.n_objects]
+    pb = _beam(n, 50 + n, n >= 65)
+    for fma in (0, 1):
+        want = _run_lines(eb, pb, "fma=%d hot=0" % fma, cuts, 2)
+        got = _run_lines(eb, pb, "fma=%d" % fma, cuts, 2)
+        assert_particles_equal(got, want, what="lines, fma=%d" % fma)
+        until = _run(eb, pb, "fma=%d" % fma, (2,))
+        if fma == 0:
+            assert_particles_equal(got, until, what="lines and track_until")
+    p = particles_in(pb)
+    np.asarray(p.s)[n // 2:] = 3.25
+    got, want = (_run_lines(eb, pb, "fma=0 hot=%s" % h, cuts, 1) for h in ("auto", "0"))
+    assert_particles_equal(got, want, what="lines from another path length")
+
+
+def test_lines_with_out_of_line_maps_and_monitors():
+    eb = lattices.kitchen_sink(with_monitor=True)
+    pb, _ = lattices.gaussian_beam(300, seed=3, sigma_x=8e-3, sigma_y=8e-3)
+    for step in (1, 2, 7):
+        cuts = list(range(0, eb.n_objects, step)) + [eb.n_objects]
+        for fma in (0, 1):
+            want = _run_lines(eb, pb, "fma=%d hot=0" % fma, cuts, 2)
+            assert_particles_equal(_run_lines(eb, pb, "fma=%d" % fma, cuts, 2), want, what="step %d" % step)
+
+
+@pytest.mark.parametrize("at_turn", [0, -3, "mixed"])
+def test_requests_end_with_every_particle_at_its_turn(at_turn):
+    """A request that ends without a further select pass (one launch of
+    small sets, or launches that hold every tile) leaves no particle
+    behind, also where the particles start at different or negative turns."""
+    eb = _lattice(31, 1)
+    pb, p = lattices.gaussian_beam(700, seed=4, sigma_x=4e-3, sigma_y=4e-3, sigma_px=1e-5, sigma_py=1e-5)
+    turns = np.asarray(p.at_turn)
+    if at_turn == "mixed":
+        turns[:] = np.random.default_rng(5).integers(-4, 4, turns.size)
+        turns[:3] = (0, -2, 3)
+    else:
+        turns[:] = at_turn
+    want = _run(eb, pb, "fma=0 compact=0", (3, 5))
+    assert set(want["at_turn"][want["state"] == 1].tolist()) == {5}
+    for cfg in ("fma=0", "fma=0 waves_per_cu=1", "fma=0 waves_per_cu=2 turns_per_launch=2",
+                "fma=0 hot=0", "fma=0 ppl=2", "fma=0 staging=lds"):
+        assert_particles_equal(_run(eb, pb, cfg, (3, 5)), want, what=cfg)
