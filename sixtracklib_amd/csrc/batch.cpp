@@ -93,14 +93,12 @@ struct NS(TrackBatch)
             NS(Buffer)* e = lat_bufs[ s ];
             if( e == nullptr || NS(Buffer_needs_remapping)( e ) ) return fail( "lattice buffer invalid" );
             const unsigned char* eb = NS(Buffer_get_const_data_begin)( e );
-            int64_t ne = 0, nm = 0;
-            int64_t const nw = NS(Lattice_pack)( eb, nullptr, 0, nullptr, &ne, nullptr, &nm );
-            if( nw < 0 ) return fail( "lattice could not be packed" );
-            std::vector< uint32_t > offs( ne + 1 );
-            std::vector< uint32_t > mons( nm > 0 ? nm : 1 );
-            packed[ s ].assign( nw + ST_LAT_PAD_WORDS, 0u );   // zero padding read ahead by the kernels
-            if( NS(Lattice_pack)( eb, packed[ s ].data(), nw, offs.data(), &ne, mons.data(), &nm ) != nw )
-                return fail( "lattice could not be packed" );
+            st::PackedLattice pk;
+            if( !st::pack_lattice( eb, nullptr, 0, pk ) ) return fail( "lattice could not be packed" );
+            int64_t const ne = ( int64_t )pk.offsets.size() - 1;
+            const std::vector< uint32_t >& offs = pk.offsets;
+            packed[ s ].swap( pk.words );
+            packed[ s ].resize( packed[ s ].size() + ST_LAT_PAD_WORDS, 0u );   // zero padding read ahead by the kernels
             for( int64_t i = 0; i < ne; ++i )
                 if( !ST_OP_IS_LEAN( ST_REC_OP( packed[ s ][ offs[ i ] ] ) ) )
                     return fail( "batched tracking needs lean lattices (no monitors, beam-beam, "

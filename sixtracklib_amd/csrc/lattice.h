@@ -110,4 +110,23 @@ typedef struct st_ebe_config_s
 }
 st_ebe_config_t;
 
+#if defined( __cplusplus )
+#include <vector>
+
+namespace st
+{
+/* The packed stream of a lattice (END record included), the word offset of
+ * every element's record and, last, of the END record, and the word index of
+ * every monitor's output-address slot; arguments as
+ * NS(Lattice_pack_with_tables).  One pass over the elements. */
+struct PackedLattice
+{
+    std::vector< uint64_t > words;
+    std::vector< uint32_t > offsets, monitor_fields;
+};
+bool pack_lattice( const unsigned char* belems, const unsigned char* const* table_buffers,
+                   int64_t n_table_buffers, PackedLattice& out );
+}  // namespace st
+#endif
+
 #endif /* SIXTRACKLIB_AMD_LATTICE_H__ */

@@ -17,6 +17,7 @@
 #ifndef SIXTRACKLIB_AMD_LATTICE_HOT_H__
 #define SIXTRACKLIB_AMD_LATTICE_HOT_H__
 
+#include <stddef.h>
 #include <stdint.h>
 
 #include "lattice.h"
@@ -63,108 +64,111 @@ struct HotMap
  * included */
 inline std::vector< uint64_t > hot_stream( const uint64_t* lat, HotMap* map = nullptr )
 {
-    if( map ) *map = HotMap();
-    size_t end = 0;
-    while( ST_REC_OP( lat[ end ] ) != ST_OP_END ) end += ST_REC_LEN( lat[ end ] );
-    std::vector< uint64_t > w;
-    w.reserve( end + end / 16 + ST_HOT_PAD_WORDS + 16 );
-    uint64_t s = 0;                               /* bits of +0.0 */
-    size_t pos = 0, touched = 0;
-    bool first = true;
-    size_t last = 0, records = 0;
-    uint64_t s_before = 0;
-    uint32_t handler = 0;
+    size_t words = 0, elements = 0;
+    for( ; ST_REC_OP( lat[ words ] ) != ST_OP_END; words += ST_REC_LEN( lat[ words ] ) ) ++elements;
+    /* no hot record is longer than the packed records it stands for, and a
+     * TOUCH record of one word comes before at least ST_HOT_TOUCH_BYTES */
+    std::vector< uint64_t > stream( words + 2u + words / ( ST_HOT_TOUCH_BYTES / 8u ) + 2u +
+                                    ST_HOT_PAD_WORDS, 0u );
+    uint64_t* const begin = stream.data();
+    uint64_t* w = begin;                          /* next word to write          */
+    uint64_t* last = nullptr;                     /* word 0 of the record before */
+    uint64_t* touched = nullptr;                  /* last TOUCH record           */
+    uint32_t handler = 0, parity = 0;             /* of the record being written */
+    uint32_t *m_off = nullptr, *m_handler = nullptr;
+    uint64_t* m_s = nullptr;
+    if( map != nullptr )
+    {
+        map->off.resize( elements + 1u );
+        map->handler.resize( elements + 1u );
+        map->s.resize( elements + 1u );
+        m_off = map->off.data(); m_handler = map->handler.data(); m_s = map->s.data();
+    }
     auto put = [ & ]( unsigned kind, size_t at )
     {
-        // the record before names this one's handler
-        handler = ( uint32_t )( kind * ST_HOT_SPACING + ( records % 2 ) * ST_HOT_SET_B );
-        if( records > 0 ) w[ last ] |= handler;
-        last = w.size();
-        ++records;
-        w.push_back( ( uint64_t )( at * 8u ) << 32 );
+        handler = ( uint32_t )( kind * ST_HOT_SPACING ) + parity;
+        parity ^= ST_HOT_SET_B;
+        if( last != nullptr ) *last |= handler;   /* the record before names it  */
+        last = w;
+        *w++ = ( uint64_t )( at * 8u ) << 32;
+    };
+    auto put_mp = [ & ]( const uint64_t* r )
+    {
+        for( int k = ( int )ST_REC_AUX( r[ 0 ] ); k >= 0; --k )
+        {
+            *w++ = r[ ST_REC_PAYLOAD + 2 * k ];
+            *w++ = r[ ST_REC_PAYLOAD + 2 * k + 1 ];
+        }
     };
     auto element = [ & ]( unsigned second, uint64_t path )
     {
         if( map == nullptr ) return;
-        map->off.push_back( ( uint32_t )( last * 8u ) | second );
-        map->handler.push_back( handler );
-        map->s.push_back( path );
+        *m_off++ = ( uint32_t )( ( last - begin ) * 8 ) | second;
+        *m_handler++ = handler;
+        *m_s++ = path;
     };
-    auto is_flat_mp = [ & ]( uint64_t h )
-    { return ST_REC_OP( h ) == ST_OP_MULTIPOLE && ST_REC_AUX( h ) <= ST_HOT_MAX_ORDER; };
-    auto put_mp = [ & ]( size_t at )
+    uint64_t s = 0;                               /* bits of +0.0                */
+    for( size_t pos = 0;; )
     {
-        int const order = ( int )ST_REC_AUX( lat[ at ] );
-        for( int k = order; k >= 0; --k )
+        if( touched == nullptr || ( size_t )( w - touched ) * 8u >= ST_HOT_TOUCH_BYTES )
         {
-            w.push_back( lat[ at + ST_REC_PAYLOAD + 2 * k ] );
-            w.push_back( lat[ at + ST_REC_PAYLOAD + 2 * k + 1 ] );
-        }
-    };
-    for( ;; )
-    {
-        if( first || ( w.size() - touched ) * 8u >= ST_HOT_TOUCH_BYTES )
-        {
-            touched = w.size();
-            first = false;
+            touched = w;
             put( ST_HOT_TOUCH, pos );
         }
-        s_before = s;
-        uint64_t const h = lat[ pos ];
-        const uint64_t* const e = lat + pos + ST_REC_PAYLOAD;
-        size_t const next = pos + ST_REC_LEN( h );
-        switch( ST_REC_OP( h ) )
+        const uint64_t* const r = lat + pos;
+        const uint64_t* const e = r + ST_REC_PAYLOAD;
+        unsigned const op = ST_REC_OP( r[ 0 ] ), aux = ST_REC_AUX( r[ 0 ] );
+        uint64_t const s_before = s;
+        pos += ST_REC_LEN( r[ 0 ] );
+        switch( op )
         {
         case ST_OP_DRIFT:
         {
+            const uint64_t* const m = lat + pos;
             s = e[ 1 ];
-            if( is_flat_mp( lat[ next ] ) )
+            if( ST_REC_OP( m[ 0 ] ) == ST_OP_MULTIPOLE && ST_REC_AUX( m[ 0 ] ) <= ST_HOT_MAX_ORDER )
             {
-                put( ST_HOT_DRIFT_MP + ST_REC_AUX( lat[ next ] ), pos );
-                w.push_back( e[ 0 ] );
-                put_mp( next );
+                put( ST_HOT_DRIFT_MP + ST_REC_AUX( m[ 0 ] ), r - lat );
+                *w++ = e[ 0 ];
+                put_mp( m );
                 element( 0u, s_before );
                 element( 1u, s );
-                pos = next + ST_REC_LEN( lat[ next ] );
+                pos += ST_REC_LEN( m[ 0 ] );
                 continue;
             }
-            put( ST_HOT_DRIFT, pos );
-            w.push_back( e[ 0 ] );
+            put( ST_HOT_DRIFT, r - lat );
+            *w++ = e[ 0 ];
             break;
         }
         case ST_OP_XYSHIFT:
         case ST_OP_SROTATION:
-            put( ST_REC_OP( h ) == ST_OP_XYSHIFT ? ST_HOT_XYSHIFT : ST_HOT_SROTATION, pos );
-            w.push_back( e[ 0 ] ); w.push_back( e[ 1 ] );
+            put( op == ST_OP_XYSHIFT ? ST_HOT_XYSHIFT : ST_HOT_SROTATION, r - lat );
+            *w++ = e[ 0 ];
+            *w++ = e[ 1 ];
             break;
         case ST_OP_LIMIT_RECT:
-            put( ST_HOT_LIMIT_RECT, pos );
-            w.insert( w.end(), e, e + 4 );
-            w.push_back( s );
-            break;
         case ST_OP_LIMIT_ELLIPSE:
-            put( ST_HOT_LIMIT_ELLIPSE, pos );
-            w.insert( w.end(), e, e + 3 );
-            w.push_back( s );
+            put( op == ST_OP_LIMIT_RECT ? ST_HOT_LIMIT_RECT : ST_HOT_LIMIT_ELLIPSE, r - lat );
+            for( int k = 0; k < ( op == ST_OP_LIMIT_RECT ? 4 : 3 ); ++k ) *w++ = e[ k ];
+            *w++ = s;
             break;
         default:
-            if( is_flat_mp( h ) )
+            if( op == ST_OP_MULTIPOLE && aux <= ST_HOT_MAX_ORDER )
             {
-                put( ST_HOT_MULTIPOLE + ST_REC_AUX( h ), pos );
-                put_mp( pos );
+                put( ST_HOT_MULTIPOLE + aux, r - lat );
+                put_mp( r );
                 break;
             }
-            if( ST_REC_OP( h ) == ST_OP_DRIFT_EXACT ) s = e[ 1 ];
-            put( ST_HOT_EXIT, pos );
-            w.push_back( s );
+            if( op == ST_OP_DRIFT_EXACT ) s = e[ 1 ];
+            put( ST_HOT_EXIT, r - lat );
+            *w++ = s;
             break;
         }
         element( 0u, s_before );
-        if( ST_REC_OP( h ) == ST_OP_END ) break;
-        pos = next;
+        if( op == ST_OP_END ) break;
     }
-    w.resize( w.size() + ST_HOT_PAD_WORDS, 0u );
-    return w;
+    stream.resize( ( size_t )( w - begin ) + ST_HOT_PAD_WORDS );
+    return stream;
 }
 }  // namespace st
 #endif

@@ -214,15 +214,13 @@ struct Packer
 };
 }  // namespace
 
-extern "C" int64_t NS(Lattice_pack_with_tables)( const unsigned char* belems,
-    const unsigned char* const* table_buffers, int64_t n_table_buffers, uint64_t* out,
-    int64_t out_capacity, uint32_t* rec_offsets, int64_t* n_elem_out,
-    uint32_t* monitor_fields, int64_t* n_monitors_out )
+bool st::pack_lattice( const unsigned char* belems, const unsigned char* const* table_buffers,
+                       int64_t n_table_buffers, st::PackedLattice& out )
 {
     if( belems == nullptr || n_table_buffers < 0 ||
-        ( n_table_buffers > 0 && table_buffers == nullptr ) ) return -1;
+        ( n_table_buffers > 0 && table_buffers == nullptr ) ) return false;
     const uint64_t* h = reinterpret_cast< const uint64_t* >( belems );
-    if( h[ 0 ] != reinterpret_cast< uint64_t >( belems ) ) return -1;   // not relocated
+    if( h[ 0 ] != reinterpret_cast< uint64_t >( belems ) ) return false;   // not relocated
     int64_t n = 0;
     const Obj* obj = objects( belems, &n );
     Packer pk;
@@ -231,7 +229,7 @@ extern "C" int64_t NS(Lattice_pack_with_tables)( const unsigned char* belems,
     for( int64_t k = 0; k < n_table_buffers; ++k )
     {
         const uint64_t* t = reinterpret_cast< const uint64_t* >( table_buffers[ k ] );
-        if( t == nullptr || t[ 0 ] != reinterpret_cast< uint64_t >( t ) ) return -1;
+        if( t == nullptr || t[ 0 ] != reinterpret_cast< uint64_t >( t ) ) return false;
         pk.tables.emplace_back( t[ 0 ], t[ 0 ] + t[ 1 ] );
     }
     pk.offs.reserve( n + 1 );
@@ -239,20 +237,33 @@ extern "C" int64_t NS(Lattice_pack_with_tables)( const unsigned char* belems,
     {
         pk.offs.push_back( static_cast< uint32_t >( pk.w.size() ) );
         pk.index = static_cast< uint64_t >( i );
-        if( !pk.add( obj[ i ] ) ) return -1;
-        if( pk.w.size() >= ( 1u << 28 ) ) return -1;    // offsets and byte lengths fit 32 bits
+        if( !pk.add( obj[ i ] ) ) return false;
+        if( pk.w.size() >= ( 1u << 28 ) ) return false;    // offsets and byte lengths fit 32 bits
     }
     pk.offs.push_back( static_cast< uint32_t >( pk.w.size() ) );
     pk.index = static_cast< uint64_t >( n );
     pk.rec( ST_OP_END, 0, {} );
-    int64_t const nw = static_cast< int64_t >( pk.w.size() );
-    if( n_elem_out ) *n_elem_out = n;
+    out.words.swap( pk.w );
+    out.offsets.swap( pk.offs );
+    out.monitor_fields.swap( pk.monitor_fields );
+    return true;
+}
+
+extern "C" int64_t NS(Lattice_pack_with_tables)( const unsigned char* belems,
+    const unsigned char* const* table_buffers, int64_t n_table_buffers, uint64_t* out,
+    int64_t out_capacity, uint32_t* rec_offsets, int64_t* n_elem_out,
+    uint32_t* monitor_fields, int64_t* n_monitors_out )
+{
+    st::PackedLattice pk;
+    if( !st::pack_lattice( belems, table_buffers, n_table_buffers, pk ) ) return -1;
+    int64_t const nw = static_cast< int64_t >( pk.words.size() );
+    if( n_elem_out ) *n_elem_out = static_cast< int64_t >( pk.offsets.size() ) - 1;
     if( n_monitors_out ) *n_monitors_out = static_cast< int64_t >( pk.monitor_fields.size() );
     if( out != nullptr )
     {
         if( out_capacity < nw ) return -1;
-        std::memcpy( out, pk.w.data(), sizeof( uint64_t ) * nw );
-        if( rec_offsets ) std::memcpy( rec_offsets, pk.offs.data(), sizeof( uint32_t ) * pk.offs.size() );
+        std::memcpy( out, pk.words.data(), sizeof( uint64_t ) * nw );
+        if( rec_offsets ) std::memcpy( rec_offsets, pk.offsets.data(), sizeof( uint32_t ) * pk.offsets.size() );
         if( monitor_fields && !pk.monitor_fields.empty() )
             std::memcpy( monitor_fields, pk.monitor_fields.data(), sizeof( uint32_t ) * pk.monitor_fields.size() );
     }

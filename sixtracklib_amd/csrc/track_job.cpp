@@ -439,26 +439,22 @@ struct NS(TrackJobBase)
     bool pack_lattice()
     {
         runner_ready = false;                   // seeds point at the lattice
-        int64_t n_elem_l = 0, n_mon = 0;
         const unsigned char* eb = NS(Buffer_get_const_data_begin)( ebuf );
         // stored buffers may hold line-density tables of space-charge elements
         std::vector< const unsigned char* > tables;
         for( const Stored& b : stored )
             if( b.buf ) tables.push_back( NS(Buffer_get_const_data_begin)( b.buf ) );
-        int64_t const nt = ( int64_t )tables.size();
-        int64_t const nw = NS(Lattice_pack_with_tables)( eb, tables.data(), nt, nullptr, 0, nullptr,
-                                                         &n_elem_l, nullptr, &n_mon );
-        if( nw < 0 ) { g_err = "lattice could not be packed"; return false; }
+        st::PackedLattice packed;
+        if( !st::pack_lattice( eb, tables.data(), ( int64_t )tables.size(), packed ) )
+        { g_err = "lattice could not be packed"; return false; }
+        n_elem = ( int64_t )packed.offsets.size() - 1;
+        lat_words = ( int64_t )packed.words.size();
+        rec_offsets.swap( packed.offsets );
+        monitor_fields.swap( packed.monitor_fields );
+        lat_host.swap( packed.words );
         // zero padding: the kernels read the header one record ahead and
         // fetch multipole coefficients in batches of up to 16 words
-        lat_host.assign( nw + ST_LAT_PAD_WORDS, 0u );
-        rec_offsets.assign( n_elem_l + 1, 0u );
-        monitor_fields.assign( n_mon, 0u );
-        if( NS(Lattice_pack_with_tables)( eb, tables.data(), nt, lat_host.data(), nw,
-                                          rec_offsets.data(), &n_elem_l, monitor_fields.data(),
-                                          &n_mon ) != nw ) return false;
-        n_elem = n_elem_l;
-        lat_words = nw;
+        lat_host.resize( lat_host.size() + ST_LAT_PAD_WORDS, 0u );
         lat_full = false;
         lat_fails = false;
         max_rec_words = 0;
@@ -486,22 +482,24 @@ struct NS(TrackJobBase)
                 }
             }
         }
-        hot_words_at = ( lat_host.size() + 31u ) & ~( size_t )31u;
+        // device: the packed lattice, its hot stream, the set descriptors
         std::vector< uint64_t > const hot = st::hot_stream( lat_host.data(), &hot_map );
-        lat_host.reserve( hot_words_at + hot.size() );
-        lat_host.resize( hot_words_at, 0u );
-        lat_host.insert( lat_host.end(), hot.begin(), hot.end() );
-        desc_words_at = ( lat_host.size() + 31u ) & ~( size_t )31u;
-        lat_host.resize( desc_words_at + views.size() * sizeof( st_batch_seed_t ) / 8u, 0u );
+        hot_words_at = ( lat_host.size() + 31u ) & ~( size_t )31u;
+        desc_words_at = ( hot_words_at + hot.size() + 31u ) & ~( size_t )31u;
         if( d_lat ) { ( void )hipFree( d_lat ); d_lat = nullptr; }
-        if( !hip_ok( hipMalloc( &d_lat, lat_host.size() * 8u ), "hipMalloc lattice" ) ) return false;
-        for( size_t k = 0; k < views.size(); ++k )
-        {
-            st_batch_seed_t sd = seed( k );
-            std::memcpy( lat_host.data() + desc_words_at + k * sizeof( sd ) / 8u, &sd, sizeof( sd ) );
-        }
+        if( !hip_ok( hipMalloc( &d_lat, desc_words_at * 8u +
+                                std::max< size_t >( views.size(), 1u ) * sizeof( st_batch_seed_t ) ),
+                     "hipMalloc lattice" ) ) return false;
+        std::vector< st_batch_seed_t > desc;
+        for( size_t k = 0; k < views.size(); ++k ) desc.push_back( seed( k ) );
         return hip_ok( hipMemcpyAsync( d_lat, lat_host.data(), lat_host.size() * 8u,
                                        hipMemcpyHostToDevice, stream ), "upload lattice" ) &&
+               hip_ok( hipMemcpyAsync( d_lat + hot_words_at, hot.data(), hot.size() * 8u,
+                                       hipMemcpyHostToDevice, stream ), "upload lattice" ) &&
+               ( desc.empty() ||
+                 hip_ok( hipMemcpyAsync( d_lat + desc_words_at, desc.data(),
+                                         desc.size() * sizeof( st_batch_seed_t ), hipMemcpyHostToDevice,
+                                         stream ), "upload lattice" ) ) &&
                hip_ok( hipStreamSynchronize( stream ), "hipStreamSynchronize" );
     }
 
