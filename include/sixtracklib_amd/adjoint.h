@@ -75,6 +75,64 @@ ST_API int NS(Adjoint_reduce_coefficients)( const st_adj_problem_t* p, int fma,
     const int32_t* mp_order, int64_t n_mp, const double* coef, double* grad_bal,
     int64_t stride, void* stream );
 
+/* ------------------------------------------------------------------------
+ * The same forward pass and gradients in four kernels, for all turns at
+ * once: a problem plus the lattice's hot stream.  NS(Adjoint_hot_size) and
+ * NS(Adjoint_hot_build) make the host data of a plan from a packed lattice;
+ * its arrays are uploaded by the caller. */
+
+/* A piece of K elements in the hot stream (byte offsets; head / tail: byte
+ * offset in the packed lattice of a Multipole to run first / of a Drift to
+ * run last, + 1, 0 for none). */
+typedef struct st_adj_segment_s
+{
+    uint32_t off, next, stop, head, tail, unused;
+}
+st_adj_segment_t;
+
+typedef struct st_adj_plan_s
+{
+    st_adj_problem_t base;      /* lat, rec_off, mp_index, ... as above; ckpt has
+                                   9 n doubles more than NS(Adjoint_checkpoint_doubles):
+                                   the state after the last turn             */
+    uint64_t* lat;              /* = base.lat, written by NS(Adjoint_coefficients) */
+    uint64_t* hot;              /* hot stream                                */
+    const st_adj_segment_t* segments;  /* [ceil(n_elem / K)]                 */
+    const int32_t* mp_order;    /* [n_mp] orders, at most 10                 */
+    const uint32_t* mp_lat;     /* [n_mp] word of bal[0] in lat              */
+    const uint32_t* mp_hot;     /* [n_mp] word of bal[0] in hot (bal[2k], bal[2k+1]
+                                   lie 2 k words before it)                  */
+    int64_t n_mp;
+    int64_t max_order;
+}
+st_adj_plan_t;
+
+/* words of the hot stream of a packed lattice (host memory, END-terminated) */
+ST_API int64_t NS(Adjoint_hot_size)( const uint64_t* lat );
+/* the hot stream, the ceil(n_elem / K) segments and per multipole, in order,
+ * mp_hot (all host memory); returns 0, or -1 on bad arguments */
+ST_API int NS(Adjoint_hot_build)( const uint64_t* lat, int64_t K, uint64_t* hot, int64_t hot_words,
+    st_adj_segment_t* segments, int64_t n_segments, uint32_t* mp_hot, int64_t n_mp );
+
+/* bal[2k] = knl[m][k] / k!, bal[2k+1] = ksl[m][k] / k! for k <= the order of
+ * multipole m, into lat and hot; rows of max_order + 1 doubles.  With
+ * scaled != 0 knl / ksl hold bal itself. */
+ST_API int NS(Adjoint_coefficients)( const st_adj_plan_t* p, int fma, const double* knl,
+    const double* ksl, int scaled, void* stream );
+
+/* forward pass: coords [n][6], loss [n]; status as NS(Adjoint_forward) */
+ST_API int NS(Adjoint_loss)( const st_adj_plan_t* p, int fma, const double* coords, double* loss,
+    int32_t* status, void* stream );
+
+/* doubles of work NS(Adjoint_gradients) needs */
+ST_API int64_t NS(Adjoint_gradient_doubles)( const st_adj_plan_t* p );
+
+/* gradients of grad_out (device scalar) x the sum of the losses after
+ * NS(Adjoint_loss): grad_coords [n][6]; grad_knl, grad_ksl
+ * [n_mp][max_order + 1], zero above a multipole's order */
+ST_API int NS(Adjoint_gradients)( const st_adj_plan_t* p, int fma, const double* grad_out,
+    double* work, double* grad_coords, double* grad_knl, double* grad_ksl, void* stream );
+
 #if defined( __cplusplus )
 }
 #endif

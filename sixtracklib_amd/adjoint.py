@@ -39,7 +39,6 @@ OP_LIMITS = (0x85, 0x86, 0x87)
 ACCEPTED = {OP_DRIFT, OP_MULTIPOLE, OP_CAVITY, OP_XYSHIFT, OP_SROTATION} | set(OP_LIMITS)
 MP_CURV_FLAG = 0x8000
 MAX_ORDER = 10
-STRIDE = 2 * MAX_ORDER + 2
 
 
 class AdjProblem(ct.Structure):
@@ -50,6 +49,13 @@ class AdjProblem(ct.Structure):
                 ("q0", ct.c_double), ("mass0", ct.c_double), ("beta0", ct.c_double),
                 ("p0c", ct.c_double), ("chi", ct.c_double), ("charge_ratio", ct.c_double),
                 ("weights", ct.c_double * 6), ("target", ct.c_void_p), ("ckpt", ct.c_void_p)]
+
+
+class AdjPlan(ct.Structure):
+    """st_adj_plan_t (include/sixtracklib_amd/adjoint.h)"""
+    _fields_ = [("base", AdjProblem), ("lat", ct.c_void_p), ("hot", ct.c_void_p),
+                ("segments", ct.c_void_p), ("mp_order", ct.c_void_p), ("mp_lat", ct.c_void_p),
+                ("mp_hot", ct.c_void_p), ("n_mp", ct.c_int64), ("max_order", ct.c_int64)]
 
 
 _lib = st.sixtracklib
@@ -68,6 +74,21 @@ _lib.st_Adjoint_reduce_coefficients.restype = ct.c_int
 _lib.st_Adjoint_reduce_coefficients.argtypes = [ct.POINTER(AdjProblem), ct.c_int, ct.c_void_p,
                                                 ct.c_int64, ct.c_void_p, ct.c_void_p,
                                                 ct.c_int64, ct.c_void_p]
+_lib.st_Adjoint_hot_size.restype = ct.c_int64
+_lib.st_Adjoint_hot_size.argtypes = [ct.c_void_p]
+_lib.st_Adjoint_hot_build.restype = ct.c_int
+_lib.st_Adjoint_hot_build.argtypes = [ct.c_void_p, ct.c_int64, ct.c_void_p, ct.c_int64, ct.c_void_p,
+                                      ct.c_int64, ct.c_void_p, ct.c_int64]
+_lib.st_Adjoint_coefficients.restype = ct.c_int
+_lib.st_Adjoint_coefficients.argtypes = [ct.POINTER(AdjPlan), ct.c_int, ct.c_void_p, ct.c_void_p,
+                                         ct.c_int, ct.c_void_p]
+_lib.st_Adjoint_loss.restype = ct.c_int
+_lib.st_Adjoint_loss.argtypes = [ct.POINTER(AdjPlan), ct.c_int, ct.c_void_p, ct.c_void_p,
+                                 ct.c_void_p, ct.c_void_p]
+_lib.st_Adjoint_gradient_doubles.restype = ct.c_int64
+_lib.st_Adjoint_gradient_doubles.argtypes = [ct.POINTER(AdjPlan)]
+_lib.st_Adjoint_gradients.restype = ct.c_int
+_lib.st_Adjoint_gradients.argtypes = [ct.POINTER(AdjPlan), ct.c_int] + [ct.c_void_p] * 6
 
 
 def _check(rc, what):
@@ -138,7 +159,6 @@ class AdjointTracker:
             mask[m, :o + 1] = True
             pos_re[m, :o + 1] = int(off) + 2 + 2 * np.arange(o + 1)
         wf = words.view(np.float64)
-        inv_f = np.array([1.0 / math.factorial(k) for k in range(no)])
         fact = np.array([float(math.factorial(k)) for k in range(no)])
         knl0 = np.where(mask, wf[np.where(mask, pos_re, 0)] * fact, 0.0)
         ksl0 = np.where(mask, wf[np.where(mask, pos_re + 1, 0)] * fact, 0.0)
@@ -148,27 +168,59 @@ class AdjointTracker:
         self.lat = torch.from_numpy(words.view(np.int64).copy()).to(dev)
         self.rec_off = torch.from_numpy(offs.astype(np.int32)).to(dev)
         self.mp_index = torch.from_numpy(mp_index).to(dev)
-        self._pos_re = torch.from_numpy(pos_re[mask]).to(dev)
-        self._inv_f = torch.from_numpy(inv_f).to(dev)
+        # the same lattice as a hot stream, in segments of K elements
+        hot = np.zeros(int(_lib.st_Adjoint_hot_size(words.ctypes.data)), dtype=np.uint64)
+        n_seg = (self.n_elem + self.K - 1) // self.K if self.K > 0 else 0
+        segments = np.zeros((n_seg, 6), dtype=np.uint32)
+        mp_hot = np.zeros(max(self.n_mp, 1), dtype=np.uint32)
+        if n_seg and _lib.st_Adjoint_hot_build(words.ctypes.data, self.K, hot.ctypes.data, hot.size,
+                                     segments.ctypes.data, segments.shape[0], mp_hot.ctypes.data,
+                                     self.n_mp) != 0:
+            raise ValueError("the lattice's hot stream could not be built")
+        self.hot = torch.from_numpy(hot.view(np.int64)).to(dev)
+        self.segments = torch.from_numpy(segments.view(np.int32)).to(dev)
+        self._mp_hot = torch.from_numpy(mp_hot.view(np.int32)).to(dev)
+        self._mp_lat = torch.from_numpy((offs[is_mp] + 2).astype(np.int32)).to(dev)
         # the lattice's own bal words: written back when the default
         # coefficients are used, so that knl0 / ksl0 track bit for bit like
         # the lattice (knl0 = bal * n! does not always round-trip)
-        self._bal0_re = torch.from_numpy(wf[pos_re[mask]].copy()).to(dev)
-        self._bal0_im = torch.from_numpy(wf[pos_re[mask] + 1].copy()).to(dev)
+        self._bal0_re = torch.from_numpy(np.where(mask, wf[np.where(mask, pos_re, 0)], 0.0)).to(dev)
+        self._bal0_im = torch.from_numpy(np.where(mask, wf[np.where(mask, pos_re + 1, 0)], 0.0)).to(dev)
         self.knl0 = torch.from_numpy(knl0).to(dev)
         self.ksl0 = torch.from_numpy(ksl0).to(dev)
 
     # -- coefficients --------------------------------------------------------
-    def write_coefficients(self, knl, ksl):
+    def write_coefficients(self, knl, ksl, plan=None):
         """bal[2n] = knl[n] * (1/n!), bal[2n+1] = ksl[n] * (1/n!) into the
-        packed lattice (be_multipole.h:437-469)."""
-        lat = self.lat.view(torch.float64)
-        if knl is self.knl0 and ksl is self.ksl0:
-            lat[self._pos_re] = self._bal0_re
-            lat[self._pos_re + 1] = self._bal0_im
-            return
-        lat[self._pos_re] = (knl * self._inv_f)[self.mask]
-        lat[self._pos_re + 1] = (ksl * self._inv_f)[self.mask]
+        packed lattice and its hot stream (be_multipole.h:437-469)."""
+        if plan is None:
+            plan = self.plan(0, self.knl0, self.lat)
+        own = knl is self.knl0 and ksl is self.ksl0
+        if own:
+            knl, ksl = self._bal0_re, self._bal0_im
+        shape = (self.n_mp, self.max_order + 1)
+        for t in (knl, ksl):
+            if t.dim() and t.device != self.lat.device:
+                raise RuntimeError("knl and ksl must be on %s" % self.lat.device)
+        # rows of max_order + 1 doubles; also from other shapes, types and
+        # strides that broadcast to them
+        knl, ksl = (t.to(self.lat.device, torch.float64).expand(shape).contiguous()
+                    for t in (knl, ksl))
+        _check(_lib.st_Adjoint_coefficients(ct.byref(plan), self.fma, knl.data_ptr(), ksl.data_ptr(),
+                                            1 if own else 0, _stream()), "adjoint coefficients")
+
+    def plan(self, n, target, ckpt):
+        """st_adj_plan_t of n particles (the tensors have to outlive it)."""
+        p = AdjPlan()
+        p.base = self.problem(n, target, ckpt)
+        p.lat = self.lat.data_ptr()
+        p.hot = self.hot.data_ptr()
+        p.segments = self.segments.data_ptr()
+        p.mp_order = self.orders.data_ptr()
+        p.mp_lat = self._mp_lat.data_ptr()
+        p.mp_hot = self._mp_hot.data_ptr()
+        p.n_mp, p.max_order = self.n_mp, self.max_order
+        return p
 
     def problem(self, n, target, ckpt):
         pr = AdjProblem()
@@ -219,14 +271,17 @@ class AdjointTracker:
 
 def _forward(tr, coords, knl, ksl, tgt):
     n = coords.shape[0]
-    tr.write_coefficients(knl, ksl)
-    X = coords.to(torch.float64).t().contiguous()
-    ckpt = torch.empty(max(tr.checkpoint_size(n), 1), dtype=torch.float64, device=tr.device)
+    if coords.dim() != 2 or coords.shape[1] < 6:
+        raise ValueError("coords must have shape (n, 6)")
+    X = coords[:, :6].to(torch.float64).contiguous()
+    # the checkpoints, and the state after the last turn
+    ckpt = torch.empty(tr.checkpoint_size(n) + 9 * n + 1, dtype=torch.float64, device=tr.device)
     loss = torch.empty(n, dtype=torch.float64, device=tr.device)
     status = torch.zeros(1, dtype=torch.int32, device=tr.device)
-    pr = tr.problem(n, tgt, ckpt)
-    _check(_lib.st_Adjoint_forward(ct.byref(pr), tr.fma, X.data_ptr(), loss.data_ptr(),
-                                   status.data_ptr(), _stream()), "adjoint forward")
+    plan = tr.plan(n, tgt, ckpt)
+    tr.write_coefficients(knl, ksl, plan)
+    _check(_lib.st_Adjoint_loss(ct.byref(plan), tr.fma, X.data_ptr(), loss.data_ptr(),
+                                status.data_ptr(), _stream()), "adjoint forward")
     if int(status.item()) != 0:
         raise RuntimeError("a particle reached an aperture: the loss is not differentiable there")
     return loss, (X, ckpt)
@@ -250,26 +305,16 @@ class _TrackLoss(torch.autograd.Function):
         knl, ksl, tgt, ckpt = ctx.saved_tensors
         n = ctx.n
         dev = tr.device
+        plan = tr.plan(n, tgt, ckpt)
         # the lattice may have been rewritten since the forward pass
-        tr.write_coefficients(*((tr.knl0, tr.ksl0) if ctx.default else (knl, ksl)))
-        pr = tr.problem(n, tgt, ckpt)
-        seg = torch.empty(max(int(_lib.st_Adjoint_segment_doubles(ct.byref(pr))), 1),
-                          dtype=torch.float64, device=dev)
-        coef = torch.empty(max(tr.n_mp * 4 * n, 1), dtype=torch.float64, device=dev)
-        cot = torch.zeros(6, n, dtype=torch.float64, device=dev)
-        gbal = torch.zeros(max(tr.n_mp, 1), STRIDE, dtype=torch.float64, device=dev)
+        tr.write_coefficients(*((tr.knl0, tr.ksl0) if ctx.default else (knl, ksl)), plan)
+        work = torch.empty(int(_lib.st_Adjoint_gradient_doubles(ct.byref(plan))) + 1,
+                           dtype=torch.float64, device=dev)
+        grad_coords = torch.empty(n, 6, dtype=torch.float64, device=dev)
+        grad_knl = torch.empty(tr.n_mp, tr.max_order + 1, dtype=torch.float64, device=dev)
+        grad_ksl = torch.empty_like(grad_knl)
         g = grad_out.to(torch.float64).reshape(1).contiguous()
-        s = _stream()
-        for turn in range(tr.n_turns - 1, -1, -1):
-            _check(_lib.st_Adjoint_backward_turn(ct.byref(pr), tr.fma, turn, g.data_ptr(),
-                                                 seg.data_ptr(), coef.data_ptr(),
-                                                 cot.data_ptr(), s), "adjoint backward")
-            if tr.n_mp:
-                _check(_lib.st_Adjoint_reduce_coefficients(
-                    ct.byref(pr), tr.fma, tr.orders.data_ptr(), tr.n_mp, coef.data_ptr(),
-                    gbal.data_ptr(), STRIDE, s), "adjoint reduce")
-        no = tr.max_order + 1
-        gbal = gbal[:tr.n_mp]
-        grad_knl = torch.where(tr.mask, gbal[:, 0:2 * no:2] * tr._inv_f, 0.0)
-        grad_ksl = torch.where(tr.mask, gbal[:, 1:2 * no:2] * tr._inv_f, 0.0)
-        return cot.t(), grad_knl, grad_ksl, None, None
+        _check(_lib.st_Adjoint_gradients(ct.byref(plan), tr.fma, g.data_ptr(), work.data_ptr(),
+                                         grad_coords.data_ptr(), grad_knl.data_ptr(),
+                                         grad_ksl.data_ptr(), _stream()), "adjoint gradients")
+        return grad_coords, grad_knl, grad_ksl, None, None

@@ -72,7 +72,8 @@ ST_DEV void multipole_adj( const Lane& p, double const chi, cptr_t bal, int cons
 // tangents through the same sequence of operations, then transposed onto
 // (zeta', delta') cotangents.  p is the state before; x, px, y, py are not
 // touched.
-ST_DEV void cavity_adj( const Lane& p, const LaneConst& c, cptr_t e, Cot& a )
+ST_DEV void cavity_jacobian( const Lane& p, const LaneConst& c, cptr_t e, double& dzn_z, double& dzn_d,
+                             double& ddn_z, double& ddn_d )
 {
     double const voltage = rd( e, 0 ), lag_rad = rd( e, 1 ), kfreq = rd( e, 2 );
     double const beta0 = c.beta0, b2 = beta0 * beta0;
@@ -100,16 +101,22 @@ ST_DEV void cavity_adj( const Lane& p, const LaneConst& c, cptr_t e, Cot& a )
     double const opd_new = sqrt( ptau * ptau + 2.0 * psigma + 1.0 );     // 1 + delta'
     // d(1 + delta') = (ptau dptau + dpsigma) / (1 + delta'), dptau = dpb / beta0,
     // dpsigma = dptau / beta0
-    double const ddn_z = ( ptau * dpb_z / beta0 + dpb_z / b2 ) / opd_new;
-    double const ddn_d = ( ptau * dpb_d / beta0 + dpb_d / b2 ) / opd_new;
+    ddn_z = ( ptau * dpb_z / beta0 + dpb_z / b2 ) / opd_new;
+    ddn_d = ( ptau * dpb_d / beta0 + dpb_d / b2 ) / opd_new;
     double const den = 1.0 + ptau_beta0;
     double const rvv_new = opd_new / den;
     double const drn_z = ( ddn_z * den - opd_new * dpb_z ) / ( den * den );
     double const drn_d = ( ddn_d * den - opd_new * dpb_d ) / ( den * den );
     // zeta' = zeta rvv_new / rvv
     double const ratio = rvv_new / rvv;
-    double const dzn_z = ratio + zeta * drn_z / rvv;
-    double const dzn_d = zeta * ( drn_d / rvv - rvv_new * drvv / ( rvv * rvv ) );
+    dzn_z = ratio + zeta * drn_z / rvv;
+    dzn_d = zeta * ( drn_d / rvv - rvv_new * drvv / ( rvv * rvv ) );
+}
+
+ST_DEV void cavity_adj( const Lane& p, const LaneConst& c, cptr_t e, Cot& a )
+{
+    double dzn_z, dzn_d, ddn_z, ddn_d;
+    cavity_jacobian( p, c, e, dzn_z, dzn_d, ddn_z, ddn_d );
     double const zb = a.zeta, db = a.delta;
     a.zeta = zb * dzn_z + db * ddn_z;
     a.delta = zb * dzn_d + db * ddn_d;

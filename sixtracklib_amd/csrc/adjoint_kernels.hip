@@ -23,6 +23,7 @@
 
 #include "track_device.h"
 #include "adjoint_device.h"
+#include "track_hot.h"
 #include "adjoint_launch.h"
 
 #ifndef ST_KSUFFIX
@@ -229,6 +230,532 @@ __global__ void __launch_bounds__( 256 ) KN( st_k_adj_reduce )( int64_t n,
     }
 }
 
+// ---------------------------------------------------------------------
+// The same gradients for all turns in few launches.
+//
+// What bounds them: the particles of such a problem are few (a few thousand:
+// 64 waves on 1,024 SIMDs), and the loop over elements x turns is a chain, so
+// the forward pass above takes 390 ns per element and the reverse pass 960.
+// Here
+//   * the forward pass runs the scheduled record walk (track_hot.h), segment
+//     by segment between checkpoints;
+//   * the reverse pass is linear in the cotangent.  st_k_adj_jacobian forms
+//     the transposed Jacobian of every piece of 64 elements of every turn,
+//     all pieces side by side (six cotangents through the piece at once,
+//     sharing its states and coefficients); st_k_adj_chain carries the
+//     cotangent from piece to piece, 36 multiply-adds each; st_k_adj_reverse
+//     then goes through every piece once more, again side by side, from its
+//     now known end cotangent, for the coefficient gradients.  Above
+//     ST_ADJ_PARALLEL_MAX particles the waves fill the chip without that,
+//     and st_k_adj_reverse alone goes through the pieces one after another;
+//   * a piece's states are recomputed from the nearest checkpoint in parts
+//     of 16 elements, the two coordinates each map's Jacobian needs kept in
+//     LDS (16 KB a wave) instead of nine in memory;
+//   * the sums over particles are formed in the wave (DPP adds, a fixed
+//     order) instead of through four values per particle and multipole.
+// 4,096 particles, 1,000 elements, 10 turns, exact build: forward 3.9 -> 0.78
+// ms, reverse 9.6 -> 0.70 ms (Jacobians 0.25, chain 0.08, pieces 0.34, sums
+// 0.03).  Reverse and forward, before / now: 64 particles 10.8 / 1.2 ms,
+// 16,384 17.7 / 3.4, 262,144 particles and 2 turns 21.3 / 6.0.  Side by side
+// costs two and a half sweeps instead of one: at 65,536 particles and 2
+// turns 2.4 ms against 2.9 from one wave through all pieces, which wins
+// above.
+namespace
+{
+struct PlanArgs
+{
+    cptr_t lat, hot;
+    cu32_t* rec_off;
+    ci32_t* mp_index;
+    cptr_t segments;             // st_adj_segment_t as three words each
+    int64_t n_elem, K, n_seg, n_turns, n, n_mp;
+    int32_t no;                  // max_order + 1
+    int32_t tiles, pieces;
+    int32_t t0, turns;           // turns [t0, t0 + turns) of this launch
+    int32_t add;                 // partial sums are added to (not the first group)
+    LaneConst C;
+    double w[ 6 ];
+    const double* target;
+    double* ckpt;
+    const double* grad_out;
+    double *jac, *cend, *partial, *grad_coords;
+};
+
+// sum over the 64 lanes, in lane 63, in a fixed order (rows of 16 by shifts,
+// then the rows)
+template< int CTRL, int ROWS >
+ST_DEV double dpp_add( double v )
+{
+    int const lo = __builtin_amdgcn_update_dpp( 0, __double2loint( v ), CTRL, ROWS, 0xf, false );
+    int const hi = __builtin_amdgcn_update_dpp( 0, __double2hiint( v ), CTRL, ROWS, 0xf, false );
+    return v + __hiloint2double( hi, lo );
+}
+
+ST_DEV double wave_sum( double v )
+{
+    v = dpp_add< 0x111, 0xf >( v );
+    v = dpp_add< 0x112, 0xf >( v );
+    v = dpp_add< 0x114, 0xf >( v );
+    v = dpp_add< 0x118, 0xf >( v );
+    v = dpp_add< 0x142, 0xa >( v );
+    v = dpp_add< 0x143, 0xc >( v );
+    return v;
+}
+
+// state at element e of turn t: the checkpoint before it, and the elements
+// between
+ST_DEV Lane state_at( const PlanArgs& a, int64_t t, int64_t e, int64_t i );
+
+// Elements [b, e) forward; with SAVE the two coordinates the adjoint map of
+// each needs go to lds[2 k], lds[2 k + 1] of element b + k (this lane's
+// column): px, py of a Drift, x, y of a Multipole, zeta, delta of a Cavity.
+template< bool SAVE >
+ST_DEV void run_elements( const PlanArgs& a, int64_t b, int64_t e, Lane& L, double* lds )
+{
+    if( b >= e ) return;
+    cptr_t r = a.lat + a.rec_off[ b ];
+    uint64_t h = r[ 0 ];
+    double* s = lds;
+    for( int64_t k = b; k < e; ++k )
+    {
+        cptr_t const prm = r + ST_REC_PAYLOAD;
+        cptr_t const nr = r + ST_REC_LEN( h );
+        uint64_t const hn = nr[ 0 ];
+        switch( ST_REC_OP( h ) )
+        {
+        case ST_OP_DRIFT:
+            if( SAVE ) { s[ 0 ] = L.px; s[ 64 ] = L.py; }
+            drift_xz( L, rd( prm, 0 ) );
+            break;
+        case ST_OP_MULTIPOLE:
+            if( SAVE ) { s[ 0 ] = L.x; s[ 64 ] = L.y; }
+            multipole( L, a.C.chi, prm, ST_REC_AUX( h ), L.delta );
+            break;
+        case ST_OP_CAVITY:
+            if( SAVE ) { s[ 0 ] = L.zeta; s[ 64 ] = L.delta; }
+            cavity( L, a.C, prm );
+            break;
+        case ST_OP_XYSHIFT: xyshift( L, prm ); break;
+        case ST_OP_SROTATION: srotation( L, prm ); break;
+        default: break;                           // apertures: checked by the forward pass
+        }
+        if( SAVE ) s += 128;
+        r = nr;
+        h = hn;
+    }
+}
+
+ST_DEV Lane state_at( const PlanArgs& a, int64_t t, int64_t e, int64_t i )
+{
+    int64_t const c = e / a.K;
+    Lane L;
+    get_lane( a.ckpt + ( ( t * a.n_seg + c ) * 9 ) * a.n, a.n, i, L );
+    run_elements< false >( a, c * a.K, e, L, nullptr );
+    return L;
+}
+
+// The adjoint maps of elements [b, e), last first, on COLS cotangents; lds
+// as run_elements< true > left it, L the state after the last element.
+// COEF: part receives the wave's sums for the coefficient gradients of every
+// multipole (rows of 2 no: d loss / d bal[2k], d loss / d bal[2k + 1]).
+template< int COLS, bool COEF >
+ST_DEV void reverse_elements( const PlanArgs& a, int64_t b, int64_t e, const Lane& L, const double* lds,
+                              Cot* c, double* part, bool add )
+{
+    double delta = L.delta, rpp = L.rpp, drpp = -rpp * rpp;
+    double drvv = drvv_ddelta( delta, a.C.beta0 );
+    double const chi = a.C.chi;
+    for( int64_t k = e - 1; k >= b; --k )
+    {
+        cptr_t const r = a.lat + a.rec_off[ k ];
+        uint64_t const h = r[ 0 ];
+        cptr_t const prm = r + ST_REC_PAYLOAD;
+        double const s0 = lds[ 128 * ( k - b ) ], s1 = lds[ 128 * ( k - b ) + 64 ];
+        switch( ST_REC_OP( h ) )
+        {
+        case ST_OP_DRIFT:                         // drift_adj, s = (px, py)
+        {
+            double const len = rd( prm, 0 );
+            double const xp = s0 * rpp, yp = s1 * rpp;
+            double const px = s0 * drpp, py = s1 * drpp;
+            double const dz = fma( -xp, px, fma( -yp, py, drvv ) ), lr = len * rpp;
+#pragma unroll
+            for( int q = 0; q < COLS; ++q )
+            {
+                double const d = fma( c[ q ].x, px, fma( c[ q ].y, py, c[ q ].zeta * dz ) );
+                c[ q ].delta = fma( len, d, c[ q ].delta );
+                c[ q ].px = fma( lr, fma( -c[ q ].zeta, xp, c[ q ].x ), c[ q ].px );
+                c[ q ].py = fma( lr, fma( -c[ q ].zeta, yp, c[ q ].y ), c[ q ].py );
+            }
+            break;
+        }
+        case ST_OP_MULTIPOLE:                     // multipole_adj, s = (x, y)
+        {
+            int const order = ( int )( ST_REC_AUX( h ) & 0x7fffu );
+            if( COEF )
+            {
+                int64_t const m = a.mp_index[ k ];
+                double* const g = part + m * ( 2 * a.no );
+                double const cx = chi * c[ 0 ].px, cy = chi * c[ 0 ].py;
+                double wr = 1.0, wi = 0.0;
+                for( int n = 0;; ++n )
+                {
+                    double const gr = wave_sum( fma( cy, wi, -cx * wr ) );
+                    double const gi = wave_sum( fma( cx, wi, cy * wr ) );
+                    if( __lane_id() == 63 )
+                    {
+                        g[ 2 * n ] = add ? g[ 2 * n ] + gr : gr;
+                        g[ 2 * n + 1 ] = add ? g[ 2 * n + 1 ] + gi : gi;
+                    }
+                    if( n == order ) break;
+                    double const nr = fma( wr, s0, -wi * s1 );
+                    wi = fma( wr, s1, wi * s0 );
+                    wr = nr;
+                }
+            }
+            double dre = 0.0, dim = 0.0;          // chi P'(z)
+            for( int n = order; n >= 1; --n )
+            {
+                double const nre = fma( dre, s0, fma( -dim, s1, n * rd( prm, 2 * n ) ) );
+                dim = fma( dre, s1, fma( dim, s0, n * rd( prm, 2 * n + 1 ) ) );
+                dre = nre;
+            }
+            dre *= chi;
+            dim *= chi;
+#pragma unroll
+            for( int q = 0; q < COLS; ++q )
+            {
+                c[ q ].x = fma( -c[ q ].px, dre, fma( c[ q ].py, dim, c[ q ].x ) );
+                c[ q ].y = fma( c[ q ].px, dim, fma( c[ q ].py, dre, c[ q ].y ) );
+            }
+            break;
+        }
+        case ST_OP_CAVITY:                        // s = (zeta, delta)
+        {
+            double const b2 = a.C.beta0 * a.C.beta0;
+            Lane P;
+            P.zeta = s0;
+            P.delta = delta = s1;
+            P.rvv = ( 1.0 + delta ) / sqrt( b2 * ( delta * delta + 2.0 * delta ) + 1.0 );
+            rpp = 1.0 / ( 1.0 + delta );
+            drpp = -rpp * rpp;
+            drvv = drvv_ddelta( delta, a.C.beta0 );
+            double zz, zd, dz, dd;
+            cavity_jacobian( P, a.C, prm, zz, zd, dz, dd );
+#pragma unroll
+            for( int q = 0; q < COLS; ++q )
+            {
+                double const zb = c[ q ].zeta, db = c[ q ].delta;
+                c[ q ].zeta = fma( zb, zz, db * dz );
+                c[ q ].delta = fma( zb, zd, db * dd );
+            }
+            break;
+        }
+        case ST_OP_SROTATION:
+#pragma unroll
+            for( int q = 0; q < COLS; ++q ) srotation_adj( prm, c[ q ] );
+            break;
+        default: break;                           // XYShift and apertures: identity
+        }
+    }
+}
+
+// One piece, elements [b, e): the states at the starts of its parts, then
+// part by part, the last first.
+template< int COLS, bool COEF >
+ST_DEV void reverse_piece( const PlanArgs& a, int64_t t, int64_t b, int64_t e, int64_t i, double* lds,
+                           Cot* c, double* part, bool add )
+{
+    constexpr int PARTS = ST_ADJ_PIECE / ST_ADJ_SUB;
+    Lane at[ PARTS ];
+    at[ 0 ] = state_at( a, t, b, i );
+#pragma unroll
+    for( int k = 1; k < PARTS; ++k )
+    {
+        int64_t const pb = b + ( k - 1 ) * ST_ADJ_SUB, pe = pb + ST_ADJ_SUB;
+        at[ k ] = at[ k - 1 ];
+        if( pe < e ) run_elements< false >( a, pb, pe, at[ k ], nullptr );
+    }
+#pragma unroll
+    for( int k = PARTS - 1; k >= 0; --k )
+    {
+        int64_t const pb = b + k * ST_ADJ_SUB, pe = pb + ST_ADJ_SUB < e ? pb + ST_ADJ_SUB : e;
+        if( pb >= e ) continue;
+        Lane L = at[ k ];
+        run_elements< true >( a, pb, pe, L, lds );
+        reverse_elements< COLS, COEF >( a, pb, pe, L, lds, c, part, add );
+    }
+}
+
+// loss terms of turn t added to the cotangent at its end
+ST_DEV void add_loss_terms( const PlanArgs& a, int64_t t, int64_t i, Cot& c )
+{
+    const double* const b = a.ckpt + ( ( t + 1 ) * a.n_seg * 9 ) * a.n;   // the next turn's first
+    const double* const tg = a.target + t * 6;
+    double const g = 2.0 * *a.grad_out;
+    c.x += g * a.w[ 0 ] * ( b[ 0 * a.n + i ] - tg[ 0 ] );
+    c.px += g * a.w[ 1 ] * ( b[ 1 * a.n + i ] - tg[ 1 ] );
+    c.y += g * a.w[ 2 ] * ( b[ 2 * a.n + i ] - tg[ 2 ] );
+    c.py += g * a.w[ 3 ] * ( b[ 3 * a.n + i ] - tg[ 3 ] );
+    c.zeta += g * a.w[ 4 ] * ( b[ 4 * a.n + i ] - tg[ 4 ] );
+    c.delta += g * a.w[ 5 ] * ( b[ 5 * a.n + i ] - tg[ 5 ] );
+}
+
+ST_DEV Cot load_cot( const double* g, int64_t i )
+{ return Cot{ g[ 6 * i ], g[ 6 * i + 1 ], g[ 6 * i + 2 ], g[ 6 * i + 3 ], g[ 6 * i + 4 ], g[ 6 * i + 5 ] }; }
+
+ST_DEV void store_cot( double* g, int64_t i, const Cot& c )
+{
+    g[ 6 * i ] = c.x; g[ 6 * i + 1 ] = c.px; g[ 6 * i + 2 ] = c.y;
+    g[ 6 * i + 3 ] = c.py; g[ 6 * i + 4 ] = c.zeta; g[ 6 * i + 5 ] = c.delta;
+}
+}  // namespace
+
+// bal of every multipole into the packed lattice and the hot stream
+__global__ void __launch_bounds__( 256 ) KN( st_k_adj_coefficients )( st_adj_plan_t p,
+    const double* knl, const double* ksl, int scaled )
+{
+    int64_t const j = ( int64_t )blockIdx.x * blockDim.x + threadIdx.x;
+    int const no = ( int )p.max_order + 1;
+    if( j >= p.n_mp * no ) return;
+    int64_t const m = j / no;
+    int const k = ( int )( j % no );
+    if( k > p.mp_order[ m ] ) return;
+    double f = 1.0;
+    for( int q = 2; q <= k; ++q ) f *= q;
+    double const inv = scaled ? 1.0 : 1.0 / f;
+    double const re = scaled ? knl[ j ] : knl[ j ] * inv, im = scaled ? ksl[ j ] : ksl[ j ] * inv;
+    double* const lat = reinterpret_cast< double* >( p.lat ) + p.mp_lat[ m ] + 2 * k;
+    double* const hot = reinterpret_cast< double* >( p.hot ) + p.mp_hot[ m ] - 2 * k;
+    lat[ 0 ] = re; lat[ 1 ] = im;
+    hot[ 0 ] = re; hot[ 1 ] = im;
+}
+
+// Forward pass through the hot stream: per segment the checkpoint, then its
+// records.  A lane that an aperture would remove sets the status and stops.
+__global__ void __launch_bounds__( 64, 4 ) KN( st_k_adj_loss )( PlanArgs a, const double* coords,
+    double* loss_out, int32_t* status )
+{
+    int64_t const n = a.n, tid = ( int64_t )blockIdx.x * 64 + threadIdx.x;
+    bool const in_range = tid < n;
+    int64_t const i = in_range ? tid : n - 1;
+    Lane L;
+    L.x = coords[ 6 * i ]; L.px = coords[ 6 * i + 1 ];
+    L.y = coords[ 6 * i + 2 ]; L.py = coords[ 6 * i + 3 ];
+    L.zeta = coords[ 6 * i + 4 ];
+    update_delta( L, a.C, coords[ 6 * i + 5 ] );
+    L.s = 0.0;
+    double loss = 0.0;
+    uint64_t act = ballot( in_range );
+    bool ok = true;
+    for( int64_t t = 0; t < a.n_turns && act != 0u; ++t )
+    {
+        for( int64_t j = 0; j < a.n_seg && act != 0u; ++j )
+        {
+            if( in_range ) put_lane( a.ckpt + ( ( t * a.n_seg + j ) * 9 ) * n, n, i, L );
+            cptr_t const sg = a.segments + 3 * j;
+            uint64_t const s0 = sg[ 0 ], s1 = sg[ 1 ], s2 = sg[ 2 ];
+            uint32_t off = ( uint32_t )s0, next = ( uint32_t )( s0 >> 32 );
+            uint32_t const stop = ( uint32_t )s1, head = ( uint32_t )( s1 >> 32 ), tail = ( uint32_t )s2;
+            if( head != 0u )
+            {
+                cptr_t const r = rec_at( a.lat, head - 1u );
+                multipole( L, a.C.chi, r + ST_REC_PAYLOAD, ST_REC_AUX( r[ 0 ] ), L.delta );
+            }
+            while( off != stop && act != 0u )
+            {
+                uint64_t lost;
+                uint32_t info;
+                hot_run< true >( a.hot, off, next, stop, L, a.C.chi, act, lost, info );
+                if( info == ~0u )                 // not run: the packed records of the segment
+                {
+                    int64_t const b = j * a.K + ( head != 0u ? 1 : 0 );
+                    int64_t e = ( j + 1 ) * a.K < a.n_elem ? ( j + 1 ) * a.K : a.n_elem;
+                    if( tail != 0u ) --e;
+                    for( int64_t k = b; k < e; ++k ) ok = apply( a.lat + a.rec_off[ k ], L, a.C ) && ok;
+                    break;
+                }
+                if( lost != 0u )
+                {
+                    if( lane_in( lost ) ) ok = false;
+                    act &= ~lost;
+                    if( info & 1u )
+                    {
+                        cptr_t const r = rec_at( a.lat, info & ~1u );
+                        cptr_t const m = r + ST_REC_LEN( r[ 0 ] );
+                        multipole( L, a.C.chi, m + ST_REC_PAYLOAD, ST_REC_AUX( m[ 0 ] ), L.delta );
+                    }
+                    continue;
+                }
+                if( off == stop ) break;
+                off += 16u;
+                ok = apply( rec_at( a.lat, info ), L, a.C ) && ok;
+            }
+            if( tail != 0u )
+            {
+                cptr_t const r = rec_at( a.lat, tail - 1u );
+                drift_xz( L, rd( r, 2 ) );
+                ok = limit_global_ok( L ) && ok;
+            }
+        }
+        double const X[ 6 ] = { L.x, L.px, L.y, L.py, L.zeta, L.delta };
+        for( int c = 0; c < 6; ++c )
+        {
+            double const d = X[ c ] - a.target[ t * 6 + c ];
+            loss += a.w[ c ] * d * d;
+        }
+    }
+    if( !in_range ) return;
+    put_lane( a.ckpt + ( a.n_turns * a.n_seg * 9 ) * n, n, i, L );
+    loss_out[ i ] = loss;
+    if( !ok ) report_failure( status );
+}
+
+// block (turn, piece, tile), tile fastest: d (cotangent at the piece's
+// start) / d (at its end), column q for the unit cotangent q
+__global__ void __launch_bounds__( 64, 2 ) KN( st_k_adj_jacobian )( PlanArgs a )
+{
+    __shared__ double lds[ ST_ADJ_SUB * 128 ];
+    int64_t const tile = blockIdx.x % a.tiles, tp = blockIdx.x / a.tiles;
+    int64_t const j = tp % a.pieces, t = a.t0 + tp / a.pieces;
+    int64_t const tid = tile * 64 + threadIdx.x;
+    int64_t const i = tid < a.n ? tid : a.n - 1;
+    int64_t const b = j * ST_ADJ_PIECE, e = b + ST_ADJ_PIECE < a.n_elem ? b + ST_ADJ_PIECE : a.n_elem;
+    Cot c[ 6 ];
+#pragma unroll
+    for( int q = 0; q < 6; ++q )
+        c[ q ] = Cot{ q == 0 ? 1.0 : 0.0, q == 1 ? 1.0 : 0.0, q == 2 ? 1.0 : 0.0,
+                      q == 3 ? 1.0 : 0.0, q == 4 ? 1.0 : 0.0, q == 5 ? 1.0 : 0.0 };
+    reverse_piece< 6, false >( a, t, b, e, i, lds + threadIdx.x, c, nullptr, false );
+    int64_t const N = 64 * ( int64_t )a.tiles;
+    double* const J = a.jac + tp * 36 * N + tid;
+#pragma unroll
+    for( int q = 0; q < 6; ++q )
+    {
+        J[ ( 6 * q + 0 ) * N ] = c[ q ].x; J[ ( 6 * q + 1 ) * N ] = c[ q ].px;
+        J[ ( 6 * q + 2 ) * N ] = c[ q ].y; J[ ( 6 * q + 3 ) * N ] = c[ q ].py;
+        J[ ( 6 * q + 4 ) * N ] = c[ q ].zeta; J[ ( 6 * q + 5 ) * N ] = c[ q ].delta;
+    }
+}
+
+// The cotangent through the pieces of the group's turns, last first; every
+// piece's end cotangent is kept.  The next piece's Jacobian is loaded while
+// one is applied.
+__global__ void __launch_bounds__( 64, 1 ) KN( st_k_adj_chain )( PlanArgs a )
+{
+    int64_t const tid = ( int64_t )blockIdx.x * 64 + threadIdx.x;
+    bool const in_range = tid < a.n;
+    int64_t const i = in_range ? tid : a.n - 1;
+    int64_t const N = 64 * ( int64_t )a.tiles;
+    Cot c{ 0.0, 0.0, 0.0, 0.0, 0.0, 0.0 };
+    if( a.add ) c = load_cot( a.grad_coords, i );
+    double J[ 2 ][ 36 ];
+    int64_t const last = ( int64_t )a.turns * a.pieces - 1;
+    auto load = [ & ]( int64_t tp, double* into )
+    {
+        const double* const g = a.jac + ( tp < 0 ? 0 : tp ) * 36 * N + tid;
+#pragma unroll
+        for( int k = 0; k < 36; ++k ) into[ k ] = g[ k * N ];
+    };
+    auto step = [ & ]( int64_t tp, const double* M )
+    {
+        if( tp % a.pieces == a.pieces - 1 ) add_loss_terms( a, a.t0 + tp / a.pieces, i, c );
+        double* const ce = a.cend + tp * 6 * N + tid;
+        ce[ 0 ] = c.x; ce[ N ] = c.px; ce[ 2 * N ] = c.y;
+        ce[ 3 * N ] = c.py; ce[ 4 * N ] = c.zeta; ce[ 5 * N ] = c.delta;
+        double r[ 6 ];
+#pragma unroll
+        for( int p = 0; p < 6; ++p )
+            r[ p ] = fma( M[ p ], c.x, fma( M[ 6 + p ], c.px, fma( M[ 12 + p ], c.y,
+                     fma( M[ 18 + p ], c.py, fma( M[ 24 + p ], c.zeta, M[ 30 + p ] * c.delta ) ) ) ) );
+        c = Cot{ r[ 0 ], r[ 1 ], r[ 2 ], r[ 3 ], r[ 4 ], r[ 5 ] };
+    };
+    load( last, J[ 0 ] );
+    for( int64_t tp = last; tp >= 0; tp -= 2 )
+    {
+        load( tp - 1, J[ 1 ] );
+        step( tp, J[ 0 ] );
+        if( tp == 0 ) break;
+        load( tp - 2, J[ 0 ] );
+        step( tp - 1, J[ 1 ] );
+    }
+    if( in_range ) store_cot( a.grad_coords, i, c );
+}
+
+// CHAIN: one wave goes through all pieces of all turns, last first, with its
+// cotangent; its partial sums gather over the turns.  Otherwise block
+// (turn, piece, tile) from the piece's end cotangent.
+template< bool CHAIN >
+ST_DEV void adj_reverse( const PlanArgs& a, double* lds )
+{
+    int64_t const tile = blockIdx.x % a.tiles, tp = blockIdx.x / a.tiles;
+    int64_t const tid = tile * 64 + threadIdx.x;
+    bool const in_range = tid < a.n;
+    int64_t const i = in_range ? tid : a.n - 1;
+    int64_t const row = a.n_mp * 2 * a.no;
+    Cot c{ 0.0, 0.0, 0.0, 0.0, 0.0, 0.0 };
+    if( !CHAIN )
+    {
+        int64_t const j = tp % a.pieces, k = tp / a.pieces, N = 64 * ( int64_t )a.tiles;
+        int64_t const b = j * ST_ADJ_PIECE, e = b + ST_ADJ_PIECE < a.n_elem ? b + ST_ADJ_PIECE : a.n_elem;
+        const double* const ce = a.cend + tp * 6 * N + tid;
+        if( in_range ) c = Cot{ ce[ 0 ], ce[ N ], ce[ 2 * N ], ce[ 3 * N ], ce[ 4 * N ], ce[ 5 * N ] };
+        reverse_piece< 1, true >( a, a.t0 + k, b, e, i, lds, &c,
+                                  a.partial + ( k * a.tiles + tile ) * row, a.add != 0 );
+        return;
+    }
+    for( int64_t t = a.n_turns - 1; t >= 0; --t )
+    {
+        if( in_range ) add_loss_terms( a, t, i, c );
+        for( int64_t j = a.pieces - 1; j >= 0; --j )
+        {
+            int64_t const b = j * ST_ADJ_PIECE, e = b + ST_ADJ_PIECE < a.n_elem ? b + ST_ADJ_PIECE : a.n_elem;
+            reverse_piece< 1, true >( a, t, b, e, i, lds, &c, a.partial + tile * row, t < a.n_turns - 1 );
+        }
+    }
+    if( in_range ) store_cot( a.grad_coords, i, c );
+}
+
+__global__ void __launch_bounds__( 64, 2 ) KN( st_k_adj_reverse )( PlanArgs a )
+{
+    __shared__ double lds[ ST_ADJ_SUB * 128 ];
+    adj_reverse< false >( a, lds + threadIdx.x );
+}
+
+__global__ void __launch_bounds__( 64, 2 ) KN( st_k_adj_reverse_chain )( PlanArgs a )
+{
+    __shared__ double lds[ ST_ADJ_SUB * 128 ];
+    adj_reverse< true >( a, lds + threadIdx.x );
+}
+
+// one block per multipole: the partial sums added up, times 1 / n!
+__global__ void __launch_bounds__( 256 ) KN( st_k_adj_sum )( const double* partial, int64_t partials,
+    int64_t n_mp, int no, const int32_t* mp_order, double* grad_knl, double* grad_ksl )
+{
+    __shared__ double red[ 4 ];
+    int64_t const m = blockIdx.x;
+    int const order = mp_order[ m ];
+    double f = 1.0;
+    for( int k = 0; k < no; ++k )
+    {
+        if( k > 1 ) f *= k;
+        for( int c = 0; c < 2; ++c )
+        {
+            double v = 0.0;
+            if( k <= order )
+                for( int64_t p = threadIdx.x; p < partials; p += 256 )
+                    v += partial[ ( p * n_mp + m ) * ( 2 * no ) + 2 * k + c ];
+            v = wave_sum( v );
+            if( __lane_id() == 63 ) red[ threadIdx.x >> 6 ] = v;
+            __syncthreads();
+            if( threadIdx.x == 0 )
+                ( c == 0 ? grad_knl : grad_ksl )[ m * no + k ] =
+                    ( ( red[ 0 ] + red[ 1 ] ) + ( red[ 2 ] + red[ 3 ] ) ) * ( 1.0 / f );
+            __syncthreads();
+        }
+    }
+}
+
 // ------------------------------------------------------------ launchers
 
 namespace
@@ -278,5 +805,86 @@ extern "C" hipError_t KN( st_launch_adj_reduce )( const st_adj_problem_t* p, con
     if( n_mp <= 0 || p->n <= 0 ) return hipSuccess;
     hipLaunchKernelGGL( KN( st_k_adj_reduce ), dim3( ( unsigned )n_mp ), dim3( 256 ), 0, stream,
                         p->n, mp_order, coef, grad_bal, stride );
+    return hipGetLastError();
+}
+
+namespace
+{
+PlanArgs plan_args( const st_adj_plan_t* p )
+{
+    PlanArgs a{};
+    a.lat = ( cptr_t )p->base.lat; a.hot = ( cptr_t )p->hot;
+    a.rec_off = ( cu32_t* )p->base.rec_off; a.mp_index = ( ci32_t* )p->base.mp_index;
+    a.segments = ( cptr_t )p->segments;
+    a.n_elem = p->base.n_elem; a.K = p->base.K;
+    a.n_seg = ( p->base.n_elem + p->base.K - 1 ) / p->base.K;
+    a.n_turns = p->base.n_turns; a.n = p->base.n; a.n_mp = p->n_mp;
+    a.no = ( int32_t )p->max_order + 1;
+    a.tiles = ( int32_t )st_adj_tiles( p ); a.pieces = ( int32_t )st_adj_pieces( p );
+    a.C.q0 = p->base.q0; a.C.mass0 = p->base.mass0; a.C.beta0 = p->base.beta0; a.C.p0c = p->base.p0c;
+    a.C.chi = p->base.chi; a.C.charge_ratio = p->base.charge_ratio;
+    for( int c = 0; c < 6; ++c ) a.w[ c ] = p->base.weights[ c ];
+    a.target = p->base.target;
+    a.ckpt = p->base.ckpt;
+    return a;
+}
+}  // namespace
+
+extern "C" hipError_t KN( st_launch_adj_coefficients )( const st_adj_plan_t* p, const double* knl,
+    const double* ksl, int scaled, hipStream_t stream )
+{
+    int64_t const n = p->n_mp * ( p->max_order + 1 );
+    if( n <= 0 ) return hipSuccess;
+    hipLaunchKernelGGL( KN( st_k_adj_coefficients ), dim3( ( unsigned )( ( n + 255 ) / 256 ) ), dim3( 256 ),
+                        0, stream, *p, knl, ksl, scaled );
+    return hipGetLastError();
+}
+
+extern "C" hipError_t KN( st_launch_adj_loss )( const st_adj_plan_t* p, const double* coords,
+    double* loss, int32_t* status, hipStream_t stream )
+{
+    if( p->base.n <= 0 ) return hipSuccess;
+    hipLaunchKernelGGL( KN( st_k_adj_loss ), dim3( ( unsigned )st_adj_tiles( p ) ), dim3( 64 ), 0, stream,
+                        plan_args( p ), coords, loss, status );
+    return hipGetLastError();
+}
+
+extern "C" hipError_t KN( st_launch_adj_gradients )( const st_adj_plan_t* p, const double* grad_out,
+    double* work, double* grad_coords, double* grad_knl, double* grad_ksl, hipStream_t stream )
+{
+    PlanArgs a = plan_args( p );
+    a.grad_out = grad_out;
+    a.grad_coords = grad_coords;
+    int64_t const group = st_adj_group( p ), tiles = st_adj_tiles( p ), pieces = st_adj_pieces( p );
+    a.jac = work;
+    a.cend = work + group * pieces * 36 * 64 * tiles;
+    a.partial = work + st_adj_piece_doubles( p );
+    if( p->base.n > 0 && group > 0 )
+    {
+        for( int64_t end = p->base.n_turns; end > 0; end -= group )
+        {
+            // the last turns first, groups of the same size (a turn's rows of
+            // the partial sums are added to by the groups after the first)
+            a.t0 = ( int32_t )( end > group ? end - group : 0 );
+            a.turns = ( int32_t )( end - a.t0 );
+            a.add = end < p->base.n_turns ? 1 : 0;
+            unsigned const grid = ( unsigned )( a.turns * pieces * tiles );
+            hipLaunchKernelGGL( KN( st_k_adj_jacobian ), dim3( grid ), dim3( 64 ), 0, stream, a );
+            hipLaunchKernelGGL( KN( st_k_adj_chain ), dim3( ( unsigned )tiles ), dim3( 64 ), 0, stream, a );
+            hipLaunchKernelGGL( KN( st_k_adj_reverse ), dim3( grid ), dim3( 64 ), 0, stream, a );
+            hipError_t const e = hipGetLastError();
+            if( e != hipSuccess ) return e;
+        }
+    }
+    else if( p->base.n > 0 )
+    {
+        hipLaunchKernelGGL( KN( st_k_adj_reverse_chain ), dim3( ( unsigned )tiles ), dim3( 64 ), 0, stream, a );
+        hipError_t const e = hipGetLastError();
+        if( e != hipSuccess ) return e;
+    }
+    if( p->n_mp > 0 )
+        hipLaunchKernelGGL( KN( st_k_adj_sum ), dim3( ( unsigned )p->n_mp ), dim3( 256 ), 0, stream,
+                            a.partial, p->base.n > 0 ? st_adj_partials( p ) : 0, p->n_mp, ( int )a.no,
+                            p->mp_order, grad_knl, grad_ksl );
     return hipGetLastError();
 }

@@ -18,7 +18,43 @@
         hipStream_t stream );                                                             \
     extern "C" hipError_t st_launch_adj_reduce##SUF( const st_adj_problem_t* p,          \
         const int32_t* mp_order, int64_t n_mp, const double* coef, double* grad_bal,      \
-        int64_t stride, hipStream_t stream );
+        int64_t stride, hipStream_t stream );                                             \
+    extern "C" hipError_t st_launch_adj_coefficients##SUF( const st_adj_plan_t* p,       \
+        const double* knl, const double* ksl, int scaled, hipStream_t stream );           \
+    extern "C" hipError_t st_launch_adj_loss##SUF( const st_adj_plan_t* p,               \
+        const double* coords, double* loss, int32_t* status, hipStream_t stream );        \
+    extern "C" hipError_t st_launch_adj_gradients##SUF( const st_adj_plan_t* p,          \
+        const double* grad_out, double* work, double* grad_coords, double* grad_knl,      \
+        double* grad_ksl, hipStream_t stream );
+
+// Reverse pass (adjoint_kernels.hip): elements of a piece and of the part of
+// it whose states are in LDS at a time; the particle count up to which the
+// pieces of a group of turns run side by side, and the bytes their
+// Jacobians may take.
+#define ST_ADJ_PIECE 64
+#define ST_ADJ_SUB 16
+#define ST_ADJ_PARALLEL_MAX 65536
+#define ST_ADJ_PARALLEL_BYTES ( int64_t( 1 ) << 32 )
+
+static inline int64_t st_adj_pieces( const st_adj_plan_t* p )
+{ return ( p->base.n_elem + ST_ADJ_PIECE - 1 ) / ST_ADJ_PIECE; }
+static inline int64_t st_adj_tiles( const st_adj_plan_t* p ) { return ( p->base.n + 63 ) / 64; }
+// turns whose pieces run side by side; 0: one wave goes through all pieces
+static inline int64_t st_adj_group( const st_adj_plan_t* p )
+{
+    if( p->base.n > ST_ADJ_PARALLEL_MAX || p->base.n <= 0 ) return 0;
+    int64_t const turn = st_adj_pieces( p ) * st_adj_tiles( p ) * ( 36 + 6 ) * 64 * 8;
+    int64_t const g = ST_ADJ_PARALLEL_BYTES / turn;
+    return g < p->base.n_turns ? g : p->base.n_turns;
+}
+// work: Jacobians [group][piece][36][64 tiles], end cotangents
+// [group][piece][6][64 tiles], partial sums [partials][n_mp][2 (max_order + 1)]
+static inline int64_t st_adj_partials( const st_adj_plan_t* p )
+{ return ( st_adj_group( p ) > 0 ? st_adj_group( p ) : 1 ) * st_adj_tiles( p ); }
+static inline int64_t st_adj_piece_doubles( const st_adj_plan_t* p )
+{ return st_adj_group( p ) * st_adj_pieces( p ) * ( 36 + 6 ) * 64 * st_adj_tiles( p ); }
+static inline int64_t st_adj_partial_doubles( const st_adj_plan_t* p )
+{ return st_adj_partials( p ) * p->n_mp * 2 * ( p->max_order + 1 ); }
 
 ST_DECLARE_ADJ_LAUNCHERS( _exact )
 ST_DECLARE_ADJ_LAUNCHERS( _fma )
