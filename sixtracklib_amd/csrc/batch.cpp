@@ -2,8 +2,8 @@
 //
 // Host side of the batched form (include/sixtracklib_amd/track_batch.h).
 // Device layout:
-//   * every particle buffer is uploaded as one byte image relocated to its
-//     device address (as the plain job does), all images in one
+//   * every particle buffer is uploaded as one byte image, as it is (as the
+//     plain job does), all images in one
 //     allocation; the kernels see one st_dev_particles_t view per seed;
 //   * every lattice is packed (lattice.h) into one shared allocation;
 //   * lists, counts and queues belong to the BatchRunner (batch_runner.h).
@@ -161,22 +161,26 @@ struct NS(TrackBatch)
         for( int64_t s = 0; s < n_seeds(); ++s )
         {
             NS(Buffer)* b = part_bufs[ s ];
-            if( NS(Buffer_get_size)( b ) != img_bytes[ s ] ) return fail( "particle buffer changed size" );
-            std::vector< uint64_t > staging( ( img_bytes[ s ] + 7 ) / 8 );
-            std::memcpy( staging.data(), NS(Buffer_get_const_data_begin)( b ), img_bytes[ s ] );
-            unsigned char* d = d_img + img_off[ s ];
-            if( NS(ManagedBuffer_remap_to)( reinterpret_cast< unsigned char* >( staging.data() ),
-                                            ( NS(buffer_addr_t) )( uintptr_t )d ) != 0 )
-                return fail( "relocation of particle image failed" );
-            if( !hip_ok( hipMemcpyAsync( d, staging.data(), img_bytes[ s ], hipMemcpyHostToDevice,
-                                         stream ), "upload particles" ) ||
-                !hip_ok( hipStreamSynchronize( stream ), "hipStreamSynchronize" ) ) return false;
+            if( NS(Buffer_get_size)( b ) != img_bytes[ s ] )
+            {
+                ( void )hipStreamSynchronize( stream );
+                return fail( "particle buffer changed size" );
+            }
+            // as it is: the views hold the arrays' device addresses, and
+            // collect relocates the image whatever base it holds
+            if( !hip_ok( hipMemcpyAsync( d_img + img_off[ s ], NS(Buffer_get_const_data_begin)( b ),
+                                         img_bytes[ s ], hipMemcpyHostToDevice, stream ),
+                         "upload particles" ) )
+            {
+                ( void )hipStreamSynchronize( stream );
+                return false;
+            }
             NS(Particles)* p = NS(Particles_buffer_get_particles)( b, 0 );
             for( int64_t i = 0; i < p->num_particles; ++i )
                 if( p->state[ i ] == 1 ) mt = std::min( mt, ( int64_t )p->at_turn[ i ] );
         }
         min_turn = ( mt == INT64_MAX ) ? 0 : mt;
-        return true;
+        return hip_ok( hipStreamSynchronize( stream ), "hipStreamSynchronize" );
     }
 
     bool collect()
