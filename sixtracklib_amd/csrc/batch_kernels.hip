@@ -23,6 +23,7 @@
 #include "track_lean.h"
 #include "track_lean_lds.h"
 #include "track_hot.h"
+#include "track_hot2.h"
 #include "batch.h"
 
 #ifndef ST_KSUFFIX
@@ -232,8 +233,8 @@ ST_DEV bool find_tile( const st_batch_sched_t& s, int qb, int qe, int t, int& se
 // Tile loop of the persistent track kernels (HEAVY: lattices that also
 // hold the maps outside the lean set; HOT: the scheduled record walk).
 // Without counts (HOT only): one launch of one wave per 64 particles of
-// seed 0, no list.
-template< bool HEAVY, bool HOT = false >
+// seed 0, no list.  ONE_SET: the walk of track_hot2.h.
+template< bool HEAVY, bool HOT = false, bool ONE_SET = false >
 ST_DEV void batch_track_tiles( const st_batch_sched_t& s, int64_t until_turn, int64_t max_turns,
                                int32_t* status )
 {
@@ -269,9 +270,9 @@ ST_DEV void batch_track_tiles( const st_batch_sched_t& s, int64_t until_turn, in
             if constexpr( HOT )
             {
                 cptr_t const w = ( cptr_t )s.seeds + 26 * seed;
-                track_hot_lane< HEAVY >( PDesc{ w }, list, count, ( int64_t )tile * 64 + __lane_id(),
-                                         ( cptr_t )w[ 22 ], ( cptr_t )w[ 25 ], ( int64_t )w[ 23 ],
-                                         until_turn, max_turns, status, wp );
+                track_hot_lane< HEAVY, ONE_SET >( PDesc{ w }, list, count, ( int64_t )tile * 64 + __lane_id(),
+                                                  ( cptr_t )w[ 22 ], ( cptr_t )w[ 25 ],
+                                                  ( int64_t )w[ 23 ], until_turn, max_turns, status, wp );
             }
             else if constexpr( HEAVY )
             {
@@ -307,6 +308,16 @@ KN( st_k_batch_track_hot )( st_batch_sched_t s, int64_t until_turn, int64_t max_
                             int32_t* status )
 {
     batch_track_tiles< false, true >( s, until_turn, max_turns, status );
+}
+
+// The same with one register set (track_hot2.h), eight waves per SIMD: for
+// the FMA build with more than four waves on a SIMD (524,288 particles on
+// the 20,000-element ring: 261 ns per element, with two sets 301).
+__global__ void __launch_bounds__( 64, ST_LEAN_WAVES_PER_EU )
+KN( st_k_batch_track_hot1 )( st_batch_sched_t s, int64_t until_turn, int64_t max_turns,
+                             int32_t* status )
+{
+    batch_track_tiles< false, true, true >( s, until_turn, max_turns, status );
 }
 
 // The same for lattices with monitors, beam-beam, space charge or RF
@@ -397,7 +408,7 @@ KN( st_k_batch_track2 )( st_batch_sched_t s, int64_t until_turn, int64_t max_tur
             if( !find_tile< 128 >( s, qb, qe, t, seed, list, count, tile ) ) break;  // queue drained
             cptr_t const w = ( cptr_t )s.seeds + 26 * seed;
             track_lean_lane2( PDesc{ w }, list, count, ( int64_t )tile * 128, ( cptr_t )w[ 22 ],
-                              ( int64_t )w[ 23 ], until_turn, max_turns, status, wp );
+                              ( cptr_t )w[ 25 ], ( int64_t )w[ 23 ], until_turn, max_turns, status, wp );
             if( one_tile ) return;
         }
     }
@@ -406,7 +417,10 @@ KN( st_k_batch_track2 )( st_batch_sched_t s, int64_t until_turn, int64_t max_tur
 // Mixed launch of one seed whose active particles all sit at one turn (the
 // front part of its list, split[0] of them): waves 0 .. pair_waves - 1 take
 // 128 particles each, two per lane (track_lean_lane2), the others share the
-// rest evenly, one per lane (track_lean_lane).  With a grid of 8 workgroups
+// rest evenly, one per lane (track_hot_lane); both run the walk of
+// track_hot2.h (1,048,576 particles on the 20,000-element ring, every wave
+// a pair wave: 480 ns per element FMA and 777 exact, with the compiled loop
+// 506 to 515 and 790; 640,000: 310 and 493, with it 343 and 527).  With a grid of 8 workgroups
 // of 256 per CU the dispatcher gives every SIMD one wave of each run of
 // n_cu consecutive workgroups, so pair_waves = m * 4 * n_cu puts m pair
 // waves and 8 - m single waves on every SIMD: all resident waves busy, the
@@ -424,7 +438,7 @@ KN( st_k_batch_track_mix )( st_batch_sched_t s, int64_t until_turn, int64_t max_
     int64_t const w = ( int64_t )blockIdx.x * ( blockDim.x >> 6 ) + ( threadIdx.x >> 6 );
     cptr_t const sd = ( cptr_t )s.seeds;                      // seed 0
     const int32_t* const list = ( const int32_t* )sd[ 24 ];
-    cptr_t const lat = ( cptr_t )sd[ 22 ];
+    cptr_t const lat = ( cptr_t )sd[ 22 ], hot = ( cptr_t )sd[ 25 ];
     int64_t const n_elem = ( int64_t )sd[ 23 ];
     WavePrio wp;
     if( s.wave_prio && max_turns > 0 && s.progress != nullptr )
@@ -445,7 +459,7 @@ KN( st_k_batch_track_mix )( st_batch_sched_t s, int64_t until_turn, int64_t max_
             begin = w * q + ( w < r ? w : r );
             end = begin + q + ( w < r ? 1 : 0 );
         }
-        track_lean_lane2( PDesc{ sd }, list, end, begin, lat, n_elem, until_turn, max_turns, status, wp );
+        track_lean_lane2( PDesc{ sd }, list, end, begin, lat, hot, n_elem, until_turn, max_turns, status, wp );
         return;
     }
     int64_t const U = W - pairs;                               // single waves
@@ -454,8 +468,8 @@ KN( st_k_batch_track_mix )( st_batch_sched_t s, int64_t until_turn, int64_t max_
     int64_t const q = rest / U, r = rest % U;
     int64_t const begin = 128 * pairs + u * q + ( u < r ? u : r );
     int64_t const end = begin + q + ( u < r ? 1 : 0 );
-    track_lean_lane< false >( PDesc{ sd }, list, end, begin + __lane_id(), lat, n_elem, until_turn,
-                              max_turns, status, wp );
+    track_hot_lane< false, true >( PDesc{ sd }, list, end, begin + __lane_id(), lat, hot, n_elem,
+                                   until_turn, max_turns, status, wp );
 }
 
 // ------------------------------------------------------------ launchers
@@ -513,6 +527,9 @@ extern "C" hipError_t KN( st_launch_batch_track )( const st_batch_sched_t* s,
     if( staging && !heavy )
         hipLaunchKernelGGL( KN( st_k_batch_track_lds ), dim3( ( unsigned )grid ), dim3( 256 ), 0,
                             stream, *s, until_turn, max_turns, status );
+    else if( hot == 2 && !heavy && particles_per_lane == 1 )
+        hipLaunchKernelGGL( KN( st_k_batch_track_hot1 ), dim3( ( unsigned )grid ), dim3( 64 ), 0, stream,
+                            *s, until_turn, max_turns, status );
     else if( hot && !heavy && particles_per_lane == 1 )
         hipLaunchKernelGGL( KN( st_k_batch_track_hot ), dim3( ( unsigned )grid ), dim3( 64 ), 0, stream,
                             *s, until_turn, max_turns, status );

@@ -134,15 +134,14 @@ struct Config
     // workgroups (16 waves then run on 16 CUs, each with a scalar cache of
     // its own: 54.6 against 59.2 ns per element with workgroups of four,
     // FMA build, 1,000 particles on the 20,000-element ring).  It is faster
-    // than the compiled loop from 64 particles to 8 waves per SIMD, though
-    // its SGPRs allow 7 (ns per element and wave set on that ring, exact
-    // build and FMA build, loop / walk): 65,536 particles 198 / 88 and
-    // 169 / 63; 131,072: 212 / 125 and 178 / 91; 262,144: 284 / 229 and
-    // 242 / 156; 400,000: 411 / 372 and 307 / 255; 524,288: 478 / 424 and
-    // 344 / 328.  Lattices with the out-of-line maps run its heavy variant:
-    // 1,048,576 particles on the 20,019-element ring with beam-beam and
-    // space charge 1108 / 1026 and 905 / 750, 100,000 308 / 141 and
-    // 290 / 105.
+    // than the compiled loop at every size (ns per element and launch on
+    // that ring, exact and FMA build, loop / walk): 65,536 particles
+    // 198 / 88 and 169 / 63; 131,072: 212 / 111 and 178 / 78; 262,144:
+    // 284 / 209 and 242 / 139; 393,216: 333 / 303 and 239 / 208; 524,288:
+    // 439 / 390 and 298 / 261.  Which of its two forms: walk_form.  Lattices
+    // with the out-of-line maps run its heavy variant: 1,048,576 particles
+    // on the 20,019-element ring with beam-beam and space charge
+    // 1108 / 1026 and 905 / 750, 100,000 308 / 141 and 290 / 105.
     bool walk() const { return hot != 0 && ppl == 1 && !lds(); }
 
     // the LDS-staged kernel runs lean lattices with one particle per lane
@@ -437,6 +436,31 @@ struct BatchRunner
     // workgroup when the lattice is staged through LDS)
     int64_t waves() const { return ( int64_t )grid() * cfg.tiles_per_block(); }
 
+    // Which form of the walk a launch of ``n_waves`` waves runs: 0 none, 1
+    // two register sets (track_hot.h), 2 one (track_hot2.h).  Two sets hide
+    // a record's reads within the wave, and ask the scalar cache for 32
+    // words a record; with more than four waves per SIMD the other waves
+    // hide them, and in the FMA build the scalar cache is then what the
+    // waves wait for.  ns per element, 20,000-element ring, two sets / one,
+    // FMA: 131,072 particles 78 / 108; 262,144 (four waves) 139 / 145;
+    // 320,000 172 / 169; 393,216 211 / 208; 430,000 278 / 240; 524,288
+    // 301 / 261; 16 lattices of 28,000 296 / 234.  Exact (half as many
+    // again FP64 instructions a record): 262,144 209 / 213; 393,216
+    // 303 / 307; 524,288 393 / 413, two sets throughout.
+    int walk_form( int64_t n_waves ) const
+    {
+        if( !cfg.walk() ) return 0;
+        return cfg.fma && !cfg.heavy && n_waves > 16 * ( int64_t )( n_cu > 0 ? n_cu : 256 ) ? 2 : 1;
+    }
+
+    // 64-particle tiles that hold every seed's particles
+    int64_t total_tiles() const
+    {
+        int64_t t = 0;
+        for( int64_t n : n_part ) t += ( n + 63 ) / 64;
+        return t;
+    }
+
     int grid() const
     {
         int const waves_per_block = cfg.walk() ? 1 : ( cfg.lds() ? 256 : cfg.block ) / 64;
@@ -467,14 +491,15 @@ struct BatchRunner
                          hipStream_t stream ) const
     {
         st_batch_sched_t const s = sched();
+        int const form = walk_form( std::min( waves(), total_tiles() ) );
         for( int64_t c = 0; c < chunks; ++c )
         {
             if( !enqueue_reset_select( until_turn, stream ) ) return false;
             hipError_t const e = cfg.fma
                 ? st_launch_batch_track_fma( &s, until_turn, k, d_status, cfg.block, grid(), cfg.ppl,
-                                             cfg.heavy ? 1 : 0, cfg.lds() ? 1 : 0, cfg.walk() ? 1 : 0, stream )
+                                             cfg.heavy ? 1 : 0, cfg.lds() ? 1 : 0, form, stream )
                 : st_launch_batch_track_exact( &s, until_turn, k, d_status, cfg.block, grid(), cfg.ppl,
-                                               cfg.heavy ? 1 : 0, cfg.lds() ? 1 : 0, cfg.walk() ? 1 : 0, stream );
+                                               cfg.heavy ? 1 : 0, cfg.lds() ? 1 : 0, form, stream );
             if( !hip_ok( e, "launch batch track" ) ) return false;
         }
         return true;
@@ -574,9 +599,9 @@ struct BatchRunner
         if( cfg.walk() && g <= 4 * n_cu ) s.wave_prio = 0;
         hipError_t const e = cfg.fma
             ? st_launch_batch_track_fma( &s, until_turn, k, d_status, cfg.block, g, cfg.ppl,
-                                         cfg.heavy ? 1 : 0, cfg.lds() ? 1 : 0, cfg.walk() ? 1 : 0, stream )
+                                         cfg.heavy ? 1 : 0, cfg.lds() ? 1 : 0, walk_form( g ), stream )
             : st_launch_batch_track_exact( &s, until_turn, k, d_status, cfg.block, g, cfg.ppl,
-                                           cfg.heavy ? 1 : 0, cfg.lds() ? 1 : 0, cfg.walk() ? 1 : 0, stream );
+                                           cfg.heavy ? 1 : 0, cfg.lds() ? 1 : 0, walk_form( g ), stream );
         return hip_ok( e, "launch batch track" );
     }
 
@@ -600,11 +625,13 @@ struct BatchRunner
     //     (a pair wave counts two), and of the shapes with w + m = j the one
     //     with the most pairs and at least one single wave, w = ceil((j +
     //     1) / 2), is the fastest (1-2 % above 8 waves with the fewest
-    //     pairs); used when n fills at least 90 % of the lanes (part-filled
-    //     single waves cost as much as full ones).  For j = 16 every wave
-    //     is a pair wave and n is spread evenly over them.
-    //   * At most one per resident lane: no mixed launch, the scheduled record
-    //     walk with one particle per lane is faster (Config::walk).
+    //     pairs).  It is ahead also where the last lanes are part-filled:
+    //     525,000 particles (j = 9), FMA, 285 ns per element on the
+    //     20,000-element ring, 294 with pair waves alone, 345 one per lane.
+    //     For j = 16 every wave is a pair wave and n is spread evenly over
+    //     them.
+    //   * At most one per resident lane: no mixed launch, one particle per
+    //     lane is as fast or faster (Config::walk, walk_form).
     // false when the launch does not apply (several seeds, particles at
     // several turns, a grid other than 8 workgroups of 256 per CU).
     bool mix_shape( int64_t n, int64_t& pairs, int& grid_wgs ) const
@@ -629,7 +656,7 @@ struct BatchRunner
         }
         if( n <= 64 * W ) return false;
         int64_t const w = ( j + 2 ) / 2, m = j - w;
-        if( w > 8 || 100 * n < 90 * j * per ) return false;
+        if( w > 8 ) return false;
         pairs = m * 4 * ( int64_t )n_cu;
         grid_wgs = ( int )( w * n_cu );
         return true;
@@ -694,11 +721,11 @@ struct BatchRunner
             if( decide )
             {
                 // ppl=auto: two particles per lane run the record walk once for
-                // both (8 % more particle-turns per second on the 20,000-element
-                // ring with 75 % or more of the resident waves busy), but hold
-                // half the waves of one per lane (at 65 % they are 4 % slower);
-                // they are chosen when the particles fill at least 70 % of the
-                // resident waves with 128-particle tiles.  A mixed launch
+                // both (1,048,576 particles on the 20,000-element ring, FMA
+                // build: 485 ns per element, one per lane 515), but hold half
+                // the waves of one per lane (640,000: 320 and 349; 430,000: 250
+                // and 240); they are chosen when the particles fill at least
+                // 70 % of the resident waves with 128-particle tiles.  A mixed launch
                 // (mix_shape) spreads the particles evenly over the waves of
                 // every SIMD instead where it applies; it is decided afresh
                 // before each mixed launch, as particles are lost.

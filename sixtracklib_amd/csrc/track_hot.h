@@ -50,7 +50,7 @@ namespace st
 // 4 GiB boundary.
 //
 // SGPRs: first words of a record s[36:51] and s[52:67], further words
-// s[68:99], jump target s[34:35], code base s100.
+// s[68:99], jump target s[34:35].
 
 #define ST_HOT_SGPRS \
     "s34", "s35", "s36", "s37", "s38", "s39", "s40", "s41", "s42", "s43", "s44", "s45", \
@@ -58,7 +58,7 @@ namespace st
     "s58", "s59", "s60", "s61", "s62", "s63", "s64", "s65", "s66", "s67", "s68", "s69", \
     "s70", "s71", "s72", "s73", "s74", "s75", "s76", "s77", "s78", "s79", "s80", "s81", \
     "s82", "s83", "s84", "s85", "s86", "s87", "s88", "s89", "s90", "s91", "s92", "s93", \
-    "s94", "s95", "s96", "s97", "s98", "s99", "s100", "s101"
+    "s94", "s95", "s96", "s97", "s98", "s99"
 
 #if defined( ST_FMA_BUILD )
 #define ST_HOT_ARITH R"(
@@ -202,7 +202,7 @@ namespace st
 .endif
   s_add_u32 %[off], %[off], \size
   s_load_dwordx16 s[\Y:\Y+15], %[hot], %[off] offset:0
-  s_add_u32 s34, s100, s[\X]
+  s_add_u32 s34, %[base], s[\X]
 .endm
 .macro ST_MP X, N, c0
 .if \N == 0
@@ -314,12 +314,12 @@ namespace st
   s_load_dwordx16 s[52:67], %[hot], %[off] offset:0
   s_getpc_b64 s[34:35]
 .Lpc%=:
-  s_add_u32 s100, s34, .Latable%=-.Lpc%=
+  s_add_u32 %[base], s34, .Latable%=-.Lpc%=
   s_addc_u32 s35, s35, 0
-  s_add_u32 s34, s100, 0xffff
+  s_add_u32 s34, %[base], 0xffff
   s_cselect_b32 %[info], -1, 0
   s_cbranch_scc1 .Lnone%=
-  s_add_u32 s34, s100, %[next]
+  s_add_u32 s34, %[base], %[next]
   s_setpc_b64 s[34:35]
   ST_HANDLERS 36, 52, a
 .org .Latable%=+%c[setb]
@@ -357,10 +357,11 @@ ST_DEV void hot_run( cptr_t hot, uint32_t& off, uint32_t& next, uint32_t const s
 #if defined( __HIP_DEVICE_COMPILE__ )
     double t0, t1, t2, t3;
     uint64_t m, exec;
+    uint32_t base;
     asm volatile( ST_HOT_ARITH ST_HOT_HANDLERS ST_HOT_PURGE
         : [ x ] "+v"( L.x ), [ y ] "+v"( L.y ), [ px ] "+v"( L.px ), [ py ] "+v"( L.py ),
           [ z ] "+v"( L.zeta ), [ off ] "+s"( off ), [ next ] "+s"( next ), [ lost ] "=&s"( lost ),
-          [ info ] "=&s"( info ), [ m ] "=&s"( m ), [ exec ] "=&s"( exec ), [ t0 ] "=&v"( t0 ),
+          [ info ] "=&s"( info ), [ m ] "=&s"( m ), [ exec ] "=&s"( exec ), [ base ] "=&s"( base ), [ t0 ] "=&v"( t0 ),
           [ t1 ] "=&v"( t1 ), [ t2 ] "=&v"( t2 ), [ t3 ] "=&v"( t3 )
         : [ rpp ] "v"( L.rpp ), [ rvv ] "v"( L.rvv ), [ chi ] "v"( chi ), [ hot ] "s"( hot ),
           [ act ] "s"( act ), [ stop ] "s"( stop ), [ stops ] "n"( STOP ? 1 : 0 ),
@@ -369,6 +370,10 @@ ST_DEV void hot_run( cptr_t hot, uint32_t& off, uint32_t& next, uint32_t const s
         : "vcc", "scc", ST_HOT_SGPRS );
 #endif
 }
+
+// The one-set walk of track_hot2.h (eight waves per SIMD).
+ST_DEV void hot_run_one( cptr_t hot, uint32_t& off, uint32_t& next, Lane& L, double const chi,
+                         uint64_t const act, uint64_t& lost, uint32_t& info );
 
 // The lanes ``lost`` leave at the element of the packed record r: their
 // state is stored, with path length s (bits).
@@ -389,7 +394,7 @@ ST_DEV void hot_lose( const PA& pa, int64_t i, Lane& L, uint64_t lost, uint64_t&
 // came to off with the path length the stream holds for it: the element loop
 // of track_lean.h's lean_turn<HEAVY, false> with the records of the hot
 // kinds run by hot_run.  False when nothing was run (hot_run, info = ~0).
-template< bool HEAVY, bool STOP, class PA >
+template< bool HEAVY, bool STOP, bool ONE_SET = false, class PA >
 ST_DEV bool hot_walk( const PA& pa, int64_t i, int64_t li, cptr_t lat, cptr_t hot, uint32_t off,
                       uint32_t next, uint32_t stop, Lane& L, double chi, uint64_t& act,
                       int32_t& status, int64_t start, int64_t at_turn )
@@ -399,7 +404,8 @@ ST_DEV bool hot_walk( const PA& pa, int64_t i, int64_t li, cptr_t lat, cptr_t ho
         if( STOP && off == stop ) break;
         uint64_t lost;
         uint32_t info;
-        hot_run< STOP >( hot, off, next, stop, L, chi, act, lost, info );
+        if constexpr( ONE_SET ) hot_run_one( hot, off, next, L, chi, act, lost, info );
+        else hot_run< STOP >( hot, off, next, stop, L, chi, act, lost, info );
         if( info == ~0u ) return false;
         if( lost != 0u )                              // at a Drift or an aperture
         {
@@ -444,7 +450,7 @@ ST_DEV bool hot_walk( const PA& pa, int64_t i, int64_t li, cptr_t lat, cptr_t ho
 // As track_lean_lane, the turns through the hot stream.  A turn on which
 // some lane starts at s != 0 (the first of a call that starts mid-lattice)
 // runs the loop with a per-lane s.
-template< bool HEAVY, class PA >
+template< bool HEAVY, bool ONE_SET = false, class PA >
 ST_DEV void track_hot_lane( const PA& pa, const int32_t* list, int64_t n_lanes, int64_t tid, cptr_t lat,
                             cptr_t hot, int64_t n_elem, int64_t until_turn, int64_t max_turns,
                             int32_t* status_out, const WavePrio& wp )
@@ -454,7 +460,7 @@ ST_DEV void track_hot_lane( const PA& pa, const int32_t* list, int64_t n_lanes, 
                int64_t at_turn )
         {
             // a stream starts with a TOUCH record
-            if( !hot_walk< HEAVY, false >( pa, i, li, lat, hot, 0u, ST_HOT_TOUCH * ST_HOT_SPACING, 0u, L,
+            if( !hot_walk< HEAVY, false, ONE_SET >( pa, i, li, lat, hot, 0u, ST_HOT_TOUCH * ST_HOT_SPACING, 0u, L,
                                            chi, act, status, start, at_turn ) )
                 lean_turn< HEAVY, true >( pa, i, li, lat, L, chi, act, status, start, at_turn );
         } );

@@ -171,3 +171,29 @@ def test_requests_end_with_every_particle_at_its_turn(at_turn):
     for cfg in ("fma=0", "fma=0 waves_per_cu=1", "fma=0 waves_per_cu=2 turns_per_launch=2",
                 "fma=0 hot=0", "fma=0 ppl=2", "fma=0 staging=lds"):
         assert_particles_equal(_run(eb, pb, cfg, (3, 5)), want, what=cfg)
+
+
+@pytest.mark.parametrize("n", [1, 64, 65, 127, 129, 1000])
+def test_two_particles_per_lane_are_the_loop(n):
+    """The walk with one register set, two particles per lane: every record
+    kind, pairs of which one or both lanes are empty or lost."""
+    eb = _lattice(40 + n, 3)
+    pb = _beam(n, 90 + n, n > 1)
+    for fma in (0, 1):
+        want = _run(eb, pb, "fma=%d ppl=1 hot=0" % fma, (1, 3))
+        for cfg in ("fma=%d ppl=2", "fma=%d ppl=2 balance=0", "fma=%d ppl=2 waves_per_cu=1 turns_per_launch=1"):
+            assert_particles_equal(_run(eb, pb, cfg % fma, (1, 3)), want, what=cfg % fma)
+
+
+@pytest.mark.parametrize("n,fma", [(64 * 4096 + 1, 1), (64 * 8192, 1), (64 * 8192 + 1, 1), (64 * 8192 + 1, 0),
+                                   (700001, 1), (128 * 8192 - 64, 0)])
+def test_launches_that_fill_the_chip_are_the_loop(n, fma):
+    """The walk with one register set as the sizes select it: one particle
+    per lane from more than four waves per SIMD (FMA build), and mixed
+    launches of one and two per lane above eight."""
+    eb = _lattice(60, 1)
+    pb = _beam(n, 7, True)
+    want = _run(eb, pb, "fma=%d ppl=1 hot=0" % fma, (1, 2))
+    assert 0 < np.count_nonzero(want["state"]) < n
+    for cfg in ("fma=%d", "fma=%d ppl=1"):
+        assert_particles_equal(_run(eb, pb, cfg % fma, (1, 2)), want, what=cfg % fma)
