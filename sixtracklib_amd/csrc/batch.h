@@ -37,7 +37,8 @@ typedef struct st_batch_sched_s
     unsigned long long* progress;   // [1] turns done by the waves of a balanced launch
     int32_t n_seeds;
     int32_t n_queues;
-    int32_t wave_prio;              // waves prioritised by turns left (track_lean.h)
+    int32_t wave_prio;              // waves prioritised (WavePrio, track_lean.h): 0 no, else
+                                    // turns between two looks at *progress, a power of two
 }
 st_batch_sched_t;
 

@@ -182,6 +182,7 @@ ST_DEV WavePrio launch_priority( const st_batch_sched_t& s, int64_t max_turns )
     int64_t const waves = ( int64_t )gridDim.x * ( blockDim.x >> 6 );
     wp.progress = s.progress;
     wp.n_waves = tiles < waves ? tiles : waves;
+    wp.every = s.wave_prio;
     return wp;
 }
 
@@ -446,6 +447,7 @@ KN( st_k_batch_track_mix )( st_batch_sched_t s, int64_t until_turn, int64_t max_
         wp.k = max_turns;
         wp.progress = s.progress;
         wp.n_waves = W;
+        wp.every = s.wave_prio;
     }
     int64_t const pairs = pair_waves < W ? pair_waves : W;
     if( w < pairs )

@@ -405,7 +405,7 @@ struct BatchRunner
         s.queue_begin = d_qbegin; s.queue_next = d_qnext;
         s.split = nullptr; s.gmin = nullptr; s.progress = nullptr;
         s.n_seeds = ( int32_t )n_seeds(); s.n_queues = cfg.queues;
-        s.wave_prio = cfg.wave_prio ? 1 : 0;
+        s.wave_prio = cfg.wave_prio ? prio_turns() : 0;
         return s;
     }
 
@@ -416,6 +416,24 @@ struct BatchRunner
         s.gmin = d_split + 2 * n_seeds();
         s.progress = d_progress;
         return s;
+    }
+
+    // Turns between two looks of a wave at the progress of its launch: up to
+    // 8,192 elements, a power of two.  Every look is an atomic on one
+    // address, some 8 ns after the other waves': with 8,192 waves 65 us a
+    // turn, more than a turn of a small ring takes.  402-element ring, 100
+    // turns, FMA build, ns per element, a look every turn / every 16th /
+    // every 64th: 70,000 particles 53 / 48 / 51, 200,000 117 / 100 / 96,
+    // 524,288 279 / 204 / 196; exact 100,000 74 / 74 / 77, 400,000
+    // 255 / 235 / 239.  On a 20,000-element ring every second turn is no
+    // faster than every one.
+    int32_t prio_turns() const
+    {
+        int64_t ne = 1;
+        for( int64_t e : n_elem ) ne = std::max( ne, e );
+        int32_t t = 1;
+        while( t < 1024 && 2 * t * ne <= 8192 ) t *= 2;
+        return t;
     }
 
     // turns per chunk: about 5e11 particle-element passes per launch (25

@@ -121,15 +121,17 @@ ST_DEV cptr_t rec_at( cptr_t lat, uint32_t off )
 //   progress == nullptr: by the turns the wave has left of the k the launch
 //     gives a tile, in four bands, more left = higher (the waves that will
 //     finish last, a tile started late or a slow one, go first);
-//   progress != nullptr: every wave adds its turns to *progress, and a wave
-//     behind the mean of the n_waves waves of the launch goes before one
-//     ahead of it (the waves stay within about a turn of each other).
+//   progress != nullptr: every wave adds its turns to *progress, once in
+//     ``every`` turns, and a wave behind the mean of the n_waves waves of the
+//     launch goes before one ahead of it (the waves stay within about
+//     ``every`` turns of each other).
 // k <= 0 leaves the priority alone.
 struct WavePrio
 {
     unsigned long long* progress = nullptr;
     int64_t n_waves = 0;
     int64_t k = 0;
+    int64_t every = 1;          // turns between two looks at *progress, a power of two
 };
 
 ST_DEV void set_wave_priority( int p )
@@ -150,13 +152,16 @@ ST_DEV void wave_priority( const WavePrio& wp, int64_t done )
         return;
     }
     if( done == 0 ) { set_wave_priority( 2 ); return; }
+    if( ( done & ( wp.every - 1 ) ) != 0 ) return;
+    unsigned long long const turns = ( unsigned long long )wp.every;
     unsigned long long v = 0;
-    if( __lane_id() == 0 ) v = atomicAdd( wp.progress, 1ull ) + 1ull;
+    if( __lane_id() == 0 ) v = atomicAdd( wp.progress, turns ) + turns;
     v = __shfl( v, 0 );
     int64_t const g = ( int64_t )( ( uint64_t )( uint32_t )__builtin_amdgcn_readfirstlane( ( int )( uint32_t )v ) |
                                    ( ( uint64_t )( uint32_t )__builtin_amdgcn_readfirstlane( ( int )( v >> 32 ) ) << 32 ) );
     int64_t const d = g - wp.n_waves * done;                 // > 0: behind the mean
-    set_wave_priority( d > wp.n_waves ? 3 : ( d > 0 ? 2 : ( d > -wp.n_waves ? 1 : 0 ) ) );
+    int64_t const band = wp.n_waves * wp.every;
+    set_wave_priority( d > band ? 3 : ( d > 0 ? 2 : ( d > -band ? 1 : 0 ) ) );
 }
 
 // a wave leaving its tile after done of k turns (its particles lost or at
@@ -165,7 +170,8 @@ ST_DEV void wave_priority( const WavePrio& wp, int64_t done )
 ST_DEV void wave_priority_leave( const WavePrio& wp, int64_t done )
 {
     if( wp.k <= 0 || wp.progress == nullptr || done >= wp.k ) return;
-    if( __lane_id() == 0 ) atomicAdd( wp.progress, ( unsigned long long )( wp.k - done ) );
+    int64_t const counted = done & -wp.every;
+    if( __lane_id() == 0 ) atomicAdd( wp.progress, ( unsigned long long )( wp.k - counted ) );
 }
 
 // One turn of a lean until-turn lane through the record stream: the
