@@ -3,8 +3,8 @@
 // Host side of the batched form (include/sixtracklib_amd/track_batch.h).
 // Device layout:
 //   * every particle buffer is uploaded as one byte image, as it is (as the
-//     plain job does), all images in one
-//     allocation; the kernels see one st_dev_particles_t view per seed;
+//     plain job does), all images in one allocation; the kernels see one
+//     st_dev_particles_t view per seed;
 //   * every lattice is packed (lattice.h) into one shared allocation;
 //   * lists, counts and queues belong to the BatchRunner (batch_runner.h).
 // A track_until(U) call runs C = ceil((U - t0) / K) chunks, t0 the smallest
@@ -249,7 +249,7 @@ struct NS(TrackBatch)
     // every trial), so the batch state is unchanged.  Candidates:
     //   one particle per lane, scalar-load lattice: block 64/128/256, 4 or 8
     //     resident waves per SIMD, one queue or one per XCD;
-    //   two particles per lane (128-particle tiles, 5 waves per SIMD): block
+    //   two particles per lane (128-particle tiles): block
     //     256, both queue layouts;
     //   lattice staged through LDS (256-lane workgroups): 4 or 8 waves per
     //     SIMD, both queue layouts.

@@ -303,7 +303,7 @@ KN( st_k_batch_track )( st_batch_sched_t s, int64_t until_turn, int64_t max_turn
 }
 
 // The same with the scheduled record walk (track_hot.h), in one-wave
-// workgroups.  Its 108 SGPRs allow seven waves per SIMD.
+// workgroups.  Its 106 SGPRs allow seven waves per SIMD.
 __global__ void __launch_bounds__( 64, 4 )
 KN( st_k_batch_track_hot )( st_batch_sched_t s, int64_t until_turn, int64_t max_turns,
                             int32_t* status )
