@@ -26,11 +26,23 @@ bool valid( const st_adj_problem_t* p )
     return true;
 }
 
+// the part of a plan that NS(Adjoint_coefficients) uses
+bool valid_multipoles( const st_adj_plan_t* p )
+{
+    if( p == nullptr || p->lat == nullptr || p->hot == nullptr ||
+        p->n_mp < 0 || p->max_order < 0 || p->max_order > ST_ADJ_MAX_ORDER ||
+        ( p->n_mp > 0 && ( p->mp_order == nullptr || p->mp_lat == nullptr || p->mp_hot == nullptr ) ) )
+    {
+        st_internal_set_error( "adjoint: invalid plan" );
+        return false;
+    }
+    return true;
+}
+
 bool valid_plan( const st_adj_plan_t* p )
 {
-    if( p == nullptr || !valid( &p->base ) || p->lat == nullptr || p->hot == nullptr ||
-        p->segments == nullptr || p->n_mp < 0 || p->max_order < 0 || p->max_order > ST_ADJ_MAX_ORDER ||
-        ( p->n_mp > 0 && ( p->mp_order == nullptr || p->mp_lat == nullptr || p->mp_hot == nullptr ) ) )
+    if( !valid_multipoles( p ) || !valid( &p->base ) ) return false;
+    if( p->segments == nullptr )
     {
         st_internal_set_error( "adjoint: invalid plan" );
         return false;
@@ -149,7 +161,7 @@ int NS(Adjoint_hot_build)( const uint64_t* lat, int64_t K, uint64_t* hot, int64_
 int NS(Adjoint_coefficients)( const st_adj_plan_t* p, int fma, const double* knl, const double* ksl,
     int scaled, void* stream )
 {
-    if( !valid_plan( p ) || ( p->n_mp > 0 && ( knl == nullptr || ksl == nullptr ) ) ) return -1;
+    if( !valid_multipoles( p ) || ( p->n_mp > 0 && ( knl == nullptr || ksl == nullptr ) ) ) return -1;
     hipStream_t const s = static_cast< hipStream_t >( stream );
     return done( fma ? st_launch_adj_coefficients_fma( p, knl, ksl, scaled, s )
                      : st_launch_adj_coefficients_exact( p, knl, ksl, scaled, s ), "adjoint coefficients" );
