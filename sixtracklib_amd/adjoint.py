@@ -200,12 +200,16 @@ class AdjointTracker:
             knl, ksl = self._bal0_re, self._bal0_im
         shape = (self.n_mp, self.max_order + 1)
         for t in (knl, ksl):
-            if t.dim() and t.device != self.lat.device:
+            if t.dim() != 2 or t.shape[0] != shape[0] or t.shape[1] not in (1, shape[1]):
+                raise ValueError("knl and ksl must have shape (n_multipoles, max_order + 1) = %s"
+                                 % (shape,))
+            if t.is_complex():
+                raise ValueError("knl and ksl must be real")
+            if t.device != self.lat.device:
                 raise RuntimeError("knl and ksl must be on %s" % self.lat.device)
-        # rows of max_order + 1 doubles; also from other shapes, types and
-        # strides that broadcast to them
-        knl, ksl = (t.to(self.lat.device, torch.float64).expand(shape).contiguous()
-                    for t in (knl, ksl))
+        # rows of max_order + 1 doubles; also from other types and strides,
+        # and from one column for all orders
+        knl, ksl = (t.to(torch.float64).expand(shape).contiguous() for t in (knl, ksl))
         _check(_lib.st_Adjoint_coefficients(ct.byref(plan), self.fma, knl.data_ptr(), ksl.data_ptr(),
                                             1 if own else 0, _stream()), "adjoint coefficients")
 

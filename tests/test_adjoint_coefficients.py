@@ -27,3 +27,18 @@ def test_a_lattice_without_multipoles_has_nothing_to_write():
     assert adjoint._lib.st_Adjoint_coefficients(ct.byref(plan), 0, none, none, 0, None) == 0
     plan.n_mp = 1                              # a multipole without its coefficients
     assert adjoint._lib.st_Adjoint_coefficients(ct.byref(plan), 0, none, none, 0, None) == -1
+
+
+@pytest.mark.parametrize("shape", [(), (1,), (3,), (1, 3), (2, 2), (3, 3), (2, 3, 1), (1, 2, 3)])
+def test_other_shapes_are_refused(shape):
+    tr = _tracker([2, 1])                      # coefficients: (2, 3)
+    for knl, ksl in ((torch.ones(shape, dtype=torch.float64), tr.ksl0),
+                     (tr.knl0, torch.ones(shape, dtype=torch.float64))):
+        with pytest.raises(ValueError, match="shape"):
+            tr.write_coefficients(knl, ksl)
+
+
+def test_complex_coefficients_are_refused():
+    tr = _tracker([2, 1])
+    with pytest.raises(ValueError, match="real"):
+        tr.write_coefficients(tr.knl0.to(torch.complex128), tr.ksl0)
