@@ -209,7 +209,18 @@ class AdjointTracker:
                 raise RuntimeError("knl and ksl must be on %s" % self.lat.device)
         # rows of max_order + 1 doubles; also from other types and strides,
         # and from one column for all orders
-        knl, ksl = (t.to(torch.float64).expand(shape).contiguous() for t in (knl, ksl))
+        knl, ksl = (t.detach().to(torch.float64).expand(shape).contiguous() for t in (knl, ksl))
+        if self.lat.device.type == "cpu":              # a tracker without a GPU: no kernel
+            inv = 1.0 if own else torch.tensor([1.0 / math.factorial(k) for k in range(shape[1])],
+                                                dtype=torch.float64)
+            k2 = 2 * torch.arange(shape[1])
+            for at, words in ((self._mp_lat[:, None] + k2, self.lat),
+                              (self._mp_hot[:self.n_mp, None] - k2, self.hot)):
+                at = at[self.mask].long()
+                words = words.view(torch.float64)
+                words[at] = (knl * inv)[self.mask]
+                words[at + 1] = (ksl * inv)[self.mask]
+            return
         _check(_lib.st_Adjoint_coefficients(ct.byref(plan), self.fma, knl.data_ptr(), ksl.data_ptr(),
                                             1 if own else 0, _stream()), "adjoint coefficients")
 

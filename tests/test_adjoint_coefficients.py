@@ -1,5 +1,5 @@
 """AdjointTracker.write_coefficients and NS(Adjoint_coefficients): what they
-take and what they refuse (CPU, no kernel runs)."""
+take, what they refuse, and the words they write (CPU, no kernel runs)."""
 import ctypes as ct
 
 import pytest
@@ -42,3 +42,29 @@ def test_complex_coefficients_are_refused():
     tr = _tracker([2, 1])
     with pytest.raises(ValueError, match="real"):
         tr.write_coefficients(tr.knl0.to(torch.complex128), tr.ksl0)
+
+
+def test_a_tracker_on_the_cpu_writes_both_streams():
+    """The packed lattice and the hot stream that a new lattice with these
+    strengths packs to, and the lattice's own again with the defaults."""
+    def tracker(a, b):
+        eb = CBuffer()
+        be.Drift(cbuffer=eb, length=1.5)
+        be.Multipole(cbuffer=eb, knl=a[0], ksl=b[0])
+        be.Multipole(cbuffer=eb, knl=a[1][:2], ksl=b[1][:2])
+        be.Drift(cbuffer=eb, length=0.5)
+        _, species = lattices.make_particles(1)
+        return adjoint.AdjointTracker(eb, 2, species=species, device="cpu")
+
+    knl = [[0.1, 0.2, 0.7, 0.9], [0.3, 0.4, 9.0, 9.0]]
+    ksl = [[1.1, 1.2, 1.3, 1.7], [1.3, 1.4, 9.0, 9.0]]
+    tr = tracker([[1.0, 2.0, 4.0, 6.0]] * 2, [[3.0, 5.0, 8.0, 3.0]] * 2)
+    want = tracker(knl, ksl)
+    lat, hot = tr.lat.clone(), tr.hot.clone()
+    tr.write_coefficients(torch.tensor(knl, dtype=torch.float64), torch.tensor(ksl, dtype=torch.float64))
+    assert torch.equal(tr.lat, want.lat) and torch.equal(tr.hot, want.hot)
+    assert not torch.equal(tr.lat, lat) and not torch.equal(tr.hot, hot)
+    tr.write_coefficients(tr.knl0, tr.ksl0)
+    assert torch.equal(tr.lat, lat) and torch.equal(tr.hot, hot)
+    tr = _tracker([])
+    tr.write_coefficients(tr.knl0, tr.ksl0)
