@@ -75,14 +75,16 @@ struct Config
                                  // through LDS by 256-lane workgroups (1; lean
                                  // lattices, one particle per lane)
 
+    // every token that selects a kernel or shapes a launch (a captured graph
+    // is kept under this string), in an order that parse() takes
     std::string str() const
     {
         char b[ 224 ];
         std::snprintf( b, sizeof( b ), "fma=%d block=%d waves_per_cu=%d queues=%d "
-                       "turns_per_launch=%lld graph=%d ppl=%s wave_prio=%d staging=%s%s%s",
+                       "turns_per_launch=%lld graph=%d ppl=%s mix=%d hot=%s wave_prio=%d staging=%s%s%s",
                        fma ? 1 : 0, block, waves_per_cu, queues, ( long long )turns_per_launch,
                        graph ? 1 : 0, ppl_auto ? "auto" : ( ppl == 2 ? "2" : "1" ),
-                       wave_prio ? 1 : 0, staging ? "lds" : "scalar",
+                       mix ? 1 : 0, hot < 0 ? "auto" : ( hot ? "1" : "0" ), wave_prio ? 1 : 0, staging ? "lds" : "scalar",
                        heavy ? " heavy" : "", balance ? " balance" : "" );
         return b;
     }
