@@ -40,9 +40,10 @@
  * lane it runs mixed launches, some waves of every SIMD with two particles
  * per lane and the others with one (the most pair waves that leave one
  * single wave per SIMD), in both builds; results identical), "mix=0|1"
- * (default 1: the mixed launches of ppl=auto), "hot=auto|0|1" (default
- * auto: launches of one particle per lane run the scheduled record walk
- * where it is faster; 0 never, 1 wherever it can run; results identical),
+ * (default 1: the mixed launches of ppl=auto), "hot=0|1" (default 1, also
+ * as "auto": track_until and track_line run the scheduled record walk; 0:
+ * the compiled loops, which hold one particle per lane whatever ppl and mix
+ * say, and are slower at every size; results identical),
  * "balance=0|1" (default 1: with compact=1
  * every launch gives each resident wave one 64-particle tile, the
  * particles furthest behind first, and the host reads the counts back

@@ -69,8 +69,8 @@ struct Config
                                  // (set by the owner, one particle per lane)
     bool balance = false;        // run_balanced() available (split lists)
     bool wave_prio = true;       // waves with more turns left issue first
-    int hot = -1;                // scheduled record walk (track_hot.h) where it applies: -1
-                                 // by rule, 0 never, 1 wherever it can run
+    bool hot = true;             // scheduled record walk (track_hot.h, track_hot2.h); without
+                                 // it one particle per lane through the compiled loops
     int staging = 0;             // lattice read through scalar loads (0) or staged
                                  // through LDS by 256-lane workgroups (1; lean
                                  // lattices, one particle per lane)
@@ -81,10 +81,10 @@ struct Config
     {
         char b[ 224 ];
         std::snprintf( b, sizeof( b ), "fma=%d block=%d waves_per_cu=%d queues=%d "
-                       "turns_per_launch=%lld graph=%d ppl=%s mix=%d hot=%s wave_prio=%d staging=%s%s%s",
+                       "turns_per_launch=%lld graph=%d ppl=%s mix=%d hot=%d wave_prio=%d staging=%s%s%s",
                        fma ? 1 : 0, block, waves_per_cu, queues, ( long long )turns_per_launch,
                        graph ? 1 : 0, ppl_auto ? "auto" : ( ppl == 2 ? "2" : "1" ),
-                       mix ? 1 : 0, hot < 0 ? "auto" : ( hot ? "1" : "0" ), wave_prio ? 1 : 0, staging ? "lds" : "scalar",
+                       mix ? 1 : 0, hot ? 1 : 0, wave_prio ? 1 : 0, staging ? "lds" : "scalar",
                        heavy ? " heavy" : "", balance ? " balance" : "" );
         return b;
     }
@@ -122,7 +122,7 @@ struct Config
             mix = false;
         }
         else if( k == "mix" ) mix = iv != 0;
-        else if( k == "hot" ) hot = v == "auto" ? -1 : ( iv != 0 ? 1 : 0 );
+        else if( k == "hot" ) hot = v == "auto" || iv != 0;
         else if( k == "staging" )
         {
             if( v == "scalar" || v == "0" ) staging = 0;
@@ -144,12 +144,15 @@ struct Config
     // with the out-of-line maps run its heavy variant: 1,048,576 particles
     // on the 20,019-element ring with beam-beam and space charge
     // 1108 / 1026 and 905 / 750, 100,000 308 / 141 and 290 / 105.
-    bool walk() const { return hot != 0 && ppl == 1 && !lds(); }
+    bool walk() const { return hot && ppl == 1 && !lds(); }
+
+    // particles per lane of a launch: two run in the walk only
+    int lane_particles() const { return hot ? ppl : 1; }
 
     // the LDS-staged kernel runs lean lattices with one particle per lane
     bool lds() const { return staging != 0 && !heavy; }
     // particles per tile and tiles a workgroup tracks at once
-    int64_t tile_particles() const { return lds() ? 256 : 64 * ppl; }
+    int64_t tile_particles() const { return lds() ? 256 : 64 * lane_particles(); }
     int tiles_per_block() const { return lds() || walk() ? 1 : block / 64; }
 
     bool parse( const char* cfg )
@@ -516,9 +519,9 @@ struct BatchRunner
         {
             if( !enqueue_reset_select( until_turn, stream ) ) return false;
             hipError_t const e = cfg.fma
-                ? st_launch_batch_track_fma( &s, until_turn, k, d_status, cfg.block, grid(), cfg.ppl,
+                ? st_launch_batch_track_fma( &s, until_turn, k, d_status, cfg.block, grid(), cfg.lane_particles(),
                                              cfg.heavy ? 1 : 0, cfg.lds() ? 1 : 0, form, stream )
-                : st_launch_batch_track_exact( &s, until_turn, k, d_status, cfg.block, grid(), cfg.ppl,
+                : st_launch_batch_track_exact( &s, until_turn, k, d_status, cfg.block, grid(), cfg.lane_particles(),
                                                cfg.heavy ? 1 : 0, cfg.lds() ? 1 : 0, form, stream );
             if( !hip_ok( e, "launch batch track" ) ) return false;
         }
@@ -618,9 +621,9 @@ struct BatchRunner
         // a cost: 12 us per turn with 1,024 waves
         if( cfg.walk() && g <= 4 * n_cu ) s.wave_prio = 0;
         hipError_t const e = cfg.fma
-            ? st_launch_batch_track_fma( &s, until_turn, k, d_status, cfg.block, g, cfg.ppl,
+            ? st_launch_batch_track_fma( &s, until_turn, k, d_status, cfg.block, g, cfg.lane_particles(),
                                          cfg.heavy ? 1 : 0, cfg.lds() ? 1 : 0, walk_form( g ), stream )
-            : st_launch_batch_track_exact( &s, until_turn, k, d_status, cfg.block, g, cfg.ppl,
+            : st_launch_batch_track_exact( &s, until_turn, k, d_status, cfg.block, g, cfg.lane_particles(),
                                            cfg.heavy ? 1 : 0, cfg.lds() ? 1 : 0, walk_form( g ), stream );
         return hip_ok( e, "launch batch track" );
     }
@@ -658,7 +661,7 @@ struct BatchRunner
     {
         pairs = 0;
         grid_wgs = 0;
-        if( !cfg.mix || cfg.heavy || cfg.lds() || n_seeds() != 1 ||
+        if( !cfg.mix || !cfg.hot || cfg.heavy || cfg.lds() || n_seeds() != 1 ||
             h_split == nullptr || h_split[ 1 ] != 0 || cfg.block != 256 || cfg.waves_per_cu != 32 ||
             n_cu <= 0 || n <= 0 ) return false;
         int64_t const W = waves();

@@ -233,7 +233,7 @@ struct NS(TrackJobBase)
     int queues = 1;
     int ppl = 0;                         // particles per lane of the lean until path (0: auto)
     bool mix = true;                     // with ppl auto: mixed one/two-particle launches
-    int hot = -1;                        // scheduled record walk (track_hot.h): auto, never, always
+    bool hot = true;                     // scheduled record walk (track_hot.h)
     bool balance = true;                 // one tile per wave and launch, furthest behind first
     bool wave_prio = true;               // waves with more turns left issue first
     int staging = 0;                     // lean until path: lattice via scalar loads or LDS
@@ -711,7 +711,7 @@ struct NS(TrackJobBase)
     // launches and waits less per call.
     bool direct( int64_t until_turn ) const
     {
-        return hot != 0 && ppl != 2 && staging == 0 && turns_per_launch == 0 && waves_per_cu == 0 &&
+        return hot && ppl != 2 && staging == 0 && turns_per_launch == 0 && waves_per_cu == 0 &&
                views.size() == 1u && views[ 0 ].n <= 64 * 4 * ( int64_t )n_cu &&
                until_turn <= ( int64_t( 1 ) << 24 ) / n_elem;
     }
@@ -903,7 +903,7 @@ struct NS(TrackJobBase)
         if( !begin_status() ) return end_status( false );
         bool ok = true;
         const uint64_t* lat = d_lat + rec_offsets[ b ];
-        if( hot != 0 && e > b && !lat_fails )
+        if( hot && e > b && !lat_fails )
         {
             st_hot_segment_t seg = hot_segment( b, e );
             for( size_t k = 0; k < views.size(); ++k )
@@ -952,7 +952,7 @@ struct NS(TrackJobBase)
             else if( k == "queues" ) queues = ( iv == 8 ) ? 8 : 1;
             else if( k == "ppl" ) ppl = ( v == "auto" ) ? 0 : ( iv == 2 ) ? 2 : 1;
             else if( k == "mix" ) mix = iv != 0;
-            else if( k == "hot" ) hot = ( v == "auto" ) ? -1 : ( iv != 0 ? 1 : 0 );
+            else if( k == "hot" ) hot = v == "auto" || iv != 0;
             else if( k == "balance" ) balance = iv != 0;
             else if( k == "wave_prio" ) wave_prio = iv != 0;
             else if( k == "staging" ) staging = ( v == "lds" || v == "1" ) ? 1 : 0;

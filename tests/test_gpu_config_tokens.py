@@ -1,11 +1,14 @@
 """Configuration tokens of the schedulers: what the configuration string
 tells and restores, and that a change of it reaches the next launch."""
+import numpy as np
 import pytest
 
-from helpers import assert_particles_equal, particles_dict
-from sixtracklib_amd import lattices
-from sixtracklib_amd.cobjects import CBuffer
-from sixtracklib_amd.particles import particles_in
+torch = pytest.importorskip("torch")
+
+from helpers import assert_particles_equal, particles_dict  # noqa: E402
+from sixtracklib_amd import lattices  # noqa: E402
+from sixtracklib_amd.cobjects import CBuffer  # noqa: E402
+from sixtracklib_amd.particles import particles_in  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
@@ -40,3 +43,34 @@ def test_batch_config_tells_and_restores_the_walk():
     batch.set_config("fma=1 hot=0 ppl=2 mix=1")
     batch.set_config(seen[1])                      # the string restores what it tells
     assert batch.config == seen[1]
+
+
+def _kernels(call):
+    """names of the tracking kernels that ``call`` launches"""
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        call()
+        torch.cuda.synchronize()
+    return {e.name.split("(")[0] for e in prof.events() if "_track" in e.name and "st_k_" in e.name}
+
+
+@pytest.mark.parametrize("n, cfg, walk", [
+    (1000, "ppl=auto", {"hot"}),
+    (530000, "ppl=auto", {"mix"}),             # more than one particle per resident lane
+    (1000, "ppl=2", {"track2"}),
+    (1000, "ppl=2 balance=0", {"track2"}),
+])
+def test_hot_0_runs_the_compiled_loop(n, cfg, walk):
+    """At every number of particles per lane that the walk has a kernel for."""
+    from sixtracklib_amd.trackjob import TrackJob
+    eb = lattices.fodo_ring(n_cells=4)
+    end = {}
+    for hot in ("1", "0", "auto"):
+        pb, p = lattices.gaussian_beam(n, seed=2, sigma_x=1e-4, sigma_y=1e-4)
+        job = TrackJob(eb, pb, config_str="fma=1 hot=%s %s" % (hot, cfg))
+        names = _kernels(lambda: job.track_until(2))
+        assert names, "no tracking kernel seen"
+        special = {k for k in ("hot", "mix", "track2") if any(k in name for name in names)}
+        assert special == (set() if hot == "0" else walk), (hot, names)
+        job.collect()
+        end[hot] = np.stack([np.array(p.x), np.array(p.px), np.array(p.zeta), np.array(p.delta)])
+    assert np.array_equal(end["0"], end["1"]) and np.array_equal(end["0"], end["auto"])
