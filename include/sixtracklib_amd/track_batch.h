@@ -18,7 +18,8 @@
  *
  * config_str tokens (space or comma separated):
  *   fma=0|1               arithmetic build (default 0, bit-exact)
- *   block=64|128|256      threads per block of the persistent launch
+ *   block=64|128|256      threads per block of the persistent launch (64 in
+ *                         launches of one particle per lane with hot=1)
  *   waves_per_cu=N        resident waves per CU the grid is sized for (1-32)
  *   queues=1|8            8: seeds grouped per XCD (one work queue each,
  *                         lattice shared in that XCD's L2), 1: one queue
@@ -27,6 +28,9 @@
  *   ppl=1|2               particles per lane (1): with 2 every lane tracks
  *                         two particles through the shared record walk
  *                         (128-particle tiles; results identical)
+ *   hot=0|1               1 (default): the scheduled record walk; 0: the
+ *                         compiled loop, one particle per lane whatever ppl
+ *                         says (results identical)
  *   wave_prio=0|1         waves with more turns left in their tile get
  *                         issue priority (1; results identical)
  *   staging=scalar|lds    lattice read through scalar loads by every wave
@@ -39,8 +43,8 @@
  *                         groups (no graph); 0: chunks of turns, every wave
  *                         taking tiles until none are left (graph-captured);
  *                         results identical
- * NS(TrackBatch_autotune) picks block, waves_per_cu, queues, particles per
- * lane and lattice staging by timing short trials on the batch itself, the
+ * NS(TrackBatch_autotune) picks waves_per_cu, queues, particles per lane and
+ * lattice staging (with hot=0 also block, and one particle per lane) by timing short trials on the batch itself, the
  * three fastest twice (state restored afterwards).
  */
 #ifndef SIXTRACKLIB_AMD_TRACK_BATCH_H__

@@ -247,10 +247,11 @@ struct NS(TrackBatch)
     // not the first turns with every particle alive.  The particle images
     // are saved first and restored at the end (and the advanced state before
     // every trial), so the batch state is unchanged.  Candidates:
-    //   one particle per lane, scalar-load lattice: block 64/128/256, 4 or 8
-    //     resident waves per SIMD, one queue or one per XCD;
-    //   two particles per lane (128-particle tiles): block
-    //     256, both queue layouts;
+    //   one particle per lane, scalar-load lattice: 4 or 8 waves per SIMD, one
+    //     queue or one per XCD; with hot=0 also block 64/128/256 (the walk's
+    //     workgroups are one wave whatever block says);
+    //   two particles per lane (128-particle tiles; not with hot=0): block
+    //     256, 4 or 8 waves per SIMD, both queue layouts;
     //   lattice staged through LDS (256-lane workgroups): 4 or 8 waves per
     //     SIMD, both queue layouts.
     int autotune( int64_t trial_turns, int64_t skip_turns )
@@ -293,6 +294,7 @@ struct NS(TrackBatch)
             for( int w : { 16, 32 } )
                 for( int q : { 1, 8 } )
                 {
+                    if( base.hot && b != 256 ) continue;
                     Config c = base;
                     c.ppl = 1; c.ppl_auto = false; c.staging = 0; c.block = b; c.waves_per_cu = w;
                     c.queues = q;
@@ -301,6 +303,7 @@ struct NS(TrackBatch)
         for( int w : { 16, 32 } )
             for( int q : { 1, 8 } )
             {
+                if( !base.hot ) continue;
                 Config c = base;
                 c.ppl = 2; c.ppl_auto = false; c.staging = 0; c.block = 256; c.waves_per_cu = w;
                 c.queues = q;

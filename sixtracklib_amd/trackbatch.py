@@ -84,7 +84,7 @@ class TrackBatch:
         return buf.value.decode()
 
     def autotune(self, trial_turns=2, skip_turns=None):
-        """Time every candidate (block, waves_per_cu, queues, particles per
+        """Time every candidate (waves_per_cu, queues, particles per
         lane, lattice staging) for ``trial_turns`` turns on this batch,
         starting after ``skip_turns`` turns (default 10 x trial_turns, past
         the early losses), keep the fastest and restore the batch state;

@@ -46,11 +46,11 @@ def test_batch_config_tells_and_restores_the_walk():
 
 
 def _kernels(call):
-    """names of the tracking kernels that ``call`` launches"""
+    """names of the tracking kernels that ``call`` launches, one per launch"""
     with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
         call()
         torch.cuda.synchronize()
-    return {e.name.split("(")[0] for e in prof.events() if "_track" in e.name and "st_k_" in e.name}
+    return [e.name.split("(")[0] for e in prof.events() if "_track" in e.name and "st_k_" in e.name]
 
 
 @pytest.mark.parametrize("n, cfg, walk", [
@@ -74,3 +74,19 @@ def test_hot_0_runs_the_compiled_loop(n, cfg, walk):
         job.collect()
         end[hot] = np.stack([np.array(p.x), np.array(p.px), np.array(p.zeta), np.array(p.delta)])
     assert np.array_equal(end["0"], end["1"]) and np.array_equal(end["0"], end["auto"])
+
+
+@pytest.mark.parametrize("hot, one, two", [(1, 4, 4), (0, 12, 0)])
+def test_autotune_times_every_launch_form_once(hot, one, two):
+    """Candidates of one and of two particles per lane that run other launches
+    (a workgroup of the walk is one wave whatever block says), each timed with
+    one launch of one turn, and the three fastest a second time."""
+    from sixtracklib_amd.trackbatch import TrackBatch
+    rings = lattices.lhc_like_ring_family(2, seed=0, n_cells=8, n_cavities=1)
+    parts = [lattices.matched_gaussian_beam(n, seed=1)[0] for n in (100, 700)]
+    batch = TrackBatch(rings, parts, config_str="fma=1 hot=%d" % hot)
+    names = _kernels(lambda: batch.autotune(trial_turns=1, skip_turns=0))
+    names = [k for k in names if "_lds" not in k]
+    pairs = sum("track2" in k for k in names)
+    assert one <= len(names) - pairs <= one + 3 and two <= pairs <= two + 3
+    assert _tokens(batch)["block"] in (("256",) if hot else ("64", "128", "256"))
