@@ -222,6 +222,8 @@ struct NS(TrackJobBase)
     size_t hot_words_at = 0, desc_words_at = 0;
     st::HotMap hot_map;
     bool lat_fails = false;              // holds a disabled map (ST_OP_FAIL)
+    int64_t lat_passes = 0;              // time of a turn, in element passes of the walk (direct)
+    int64_t turn_floor = INT64_MIN;      // no particle still tracked is at an earlier turn
     std::vector< uint32_t > rec_offsets, monitor_fields;
     std::vector< uint64_t > lat_host;
     bool lat_full = false;
@@ -418,10 +420,29 @@ struct NS(TrackJobBase)
     // of a 50 MB buffer took 15 ms beside 1.3 ms of transfer.
     bool upload_particles()
     {
+        find_turn_floor();
         return hip_ok( hipMemcpyAsync( d_pbuf, NS(Buffer_get_const_data_begin)( pbuf ), pbuf_bytes,
                                        hipMemcpyHostToDevice, stream ), "hipMemcpyAsync H2D" ) &&
                hip_ok( hipStreamSynchronize( stream ), "hipStreamSynchronize" );
     }
+
+    // turn_floor of the host's particles, for a set that direct() may take
+    // (the arrays' places in the image are those of the view, whatever
+    // address the image holds for itself)
+    void find_turn_floor()
+    {
+        turn_floor = INT64_MIN;
+        if( !small_set() ) return;
+        const unsigned char* const h = NS(Buffer_get_const_data_begin)( pbuf );
+        auto host = [ & ]( const int64_t* d )
+        { return reinterpret_cast< const int64_t* >( h + ( reinterpret_cast< const unsigned char* >( d ) - d_pbuf ) ); };
+        const int64_t *const state = host( views[ 0 ].state ), *const at_turn = host( views[ 0 ].at_turn );
+        int64_t least = INT64_MAX;
+        for( int64_t i = 0; i < views[ 0 ].n; ++i )
+            if( state[ i ] == 1 ) least = std::min( least, at_turn[ i ] );
+        turn_floor = least == INT64_MAX ? 0 : least;
+    }
+    bool small_set() const { return views.size() == 1u && views[ 0 ].n <= 64 * 4 * ( int64_t )n_cu; }
 
     bool download_image( NS(Buffer)* b, const unsigned char* d, size_t bytes )
     {
@@ -470,13 +491,18 @@ struct NS(TrackJobBase)
         lat_host.resize( lat_host.size() + ST_LAT_PAD_WORDS, 0u );
         lat_full = false;
         lat_fails = false;
+        lat_passes = 0;
         max_rec_words = 0;
         for( int64_t i = 0; i < n_elem; ++i )
         {
             unsigned const op = ST_REC_OP( lat_host[ rec_offsets[ i ] ] );
+            int64_t const rec_words = rec_offsets[ i + 1 ] - rec_offsets[ i ];
             if( !ST_OP_IS_LEAN( op ) ) lat_full = true;
             if( op == ST_OP_FAIL ) lat_fails = true;
-            max_rec_words = std::max< int64_t >( max_rec_words, rec_offsets[ i + 1 ] - rec_offsets[ i ] );
+            // the maps out of line take up to 20 us and more with their
+            // length (a BeamBeam6D's slices); 64 passes a word are more
+            lat_passes += ST_OP_IS_LEAN( op ) ? 1 : 64 * rec_words;
+            max_rec_words = std::max( max_rec_words, rec_words );
         }
         // point the monitors that have an output set at its device header
         if( plan.monitor_elems.size() > 0 && d_obuf != nullptr )
@@ -609,6 +635,7 @@ struct NS(TrackJobBase)
             if( scratch_address( device, true ) == nullptr ) return false;
         }
         pbuf_bytes = NS(Buffer_get_size)( pbuf );
+        views.clear();
         if( !hip_ok( hipMalloc( &d_pbuf, pbuf_bytes ), "hipMalloc particles" ) ) return false;
         if( !upload_particles() ) return false;
         if( obuf != nullptr )
@@ -617,8 +644,8 @@ struct NS(TrackJobBase)
             if( !hip_ok( hipMalloc( &d_obuf, obuf_bytes ), "hipMalloc output" ) ) return false;
             if( !upload_image( obuf, d_obuf, obuf_bytes ) ) return false;
         }
-        views.clear();
         for( uint64_t k : sets ) views.push_back( device_view( pbuf, d_pbuf, k ) );
+        find_turn_floor();
         if( !pack_lattice() ) return false;
         if( plan.has_ebe ) ebe_view = device_view( obuf, d_obuf, ebe_offset );
         set_sizes_u64.assign( set_sizes.begin(), set_sizes.end() );
@@ -706,14 +733,14 @@ struct NS(TrackJobBase)
     // track_until of one particle set of at most one wave per SIMD: one
     // launch of one wave per 64 particles, no select passes and no counts
     // read back (a lost particle's lane costs such a launch nothing).  The
-    // launch is not split, so the request is bounded: 2^24 element passes,
-    // about 1.5 s.  402-element ring, 1,000 particles, one turn: 85 us of
-    // launches and waits less per call.
+    // launch is not split, so the turns to go are bounded: 2^24 element
+    // passes, about 1.5 s.  402-element ring, 1,000 particles, one turn: 85 us
+    // of launches and waits less per call, at any turn.
     bool direct( int64_t until_turn ) const
     {
-        return hot && ppl != 2 && staging == 0 && turns_per_launch == 0 && waves_per_cu == 0 &&
-               views.size() == 1u && views[ 0 ].n <= 64 * 4 * ( int64_t )n_cu &&
-               until_turn <= ( int64_t( 1 ) << 24 ) / n_elem;
+        return hot && ppl != 2 && staging == 0 && turns_per_launch == 0 && waves_per_cu == 0 && small_set() &&
+               ( until_turn <= turn_floor ||
+                 ( uint64_t )until_turn - ( uint64_t )turn_floor <= ( uint64_t( 1 ) << 24 ) / ( uint64_t )lat_passes );
     }
 
     bool launch_direct( int64_t until_turn, int32_t* status )
@@ -741,6 +768,14 @@ struct NS(TrackJobBase)
         return runner_ready;
     }
 
+    // the status of a call after which every particle still tracked is at
+    // until_turn or later
+    int32_t reached( int64_t until_turn, int32_t status )
+    {
+        if( status == 0 && n_elem > 0 ) turn_floor = std::max( turn_floor, until_turn );
+        return status;
+    }
+
     int32_t track_until( int64_t until_turn )
     {
         if( !begin_status() ) return end_status( false );
@@ -748,9 +783,11 @@ struct NS(TrackJobBase)
         if( compact && n_elem > 0 )
         {
             int64_t n_active = 0, min_turn = 0;
-            if( balance && direct( until_turn ) ) return end_status( launch_direct( until_turn, h_status ) );
-            if( balance ) return end_status( ensure_runner() &&
-                                             runner.run_balanced( until_turn, h_status, stream ) );
+            if( balance && direct( until_turn ) )
+                return reached( until_turn, end_status( launch_direct( until_turn, h_status ) ) );
+            if( balance )
+                return reached( until_turn, end_status( ensure_runner() &&
+                                                        runner.run_balanced( until_turn, h_status, stream ) ) );
             ok = ensure_runner() && runner.select_sync( until_turn, stream, n_active, min_turn );
             if( ok && n_active > 0 )
             {
@@ -758,7 +795,7 @@ struct NS(TrackJobBase)
                 int64_t const chunks = ( until_turn - min_turn + k - 1 ) / k;
                 ok = runner.run( until_turn, chunks, k, h_status, stream );
             }
-            return end_status( ok );
+            return reached( until_turn, end_status( ok ) );
         }
         for( const st_dev_particles_t& v : views )
         {
@@ -767,7 +804,7 @@ struct NS(TrackJobBase)
                 : st_launch_track_until_exact( &v, d_lat, n_elem, until_turn, lat_full, h_status, block, stream );
             ok = ok && hip_ok( err, "launch track_until" );
         }
-        return end_status( ok );
+        return reached( until_turn, end_status( ok ) );
     }
 
     // track_until with every scratch array of the call in the device's
@@ -839,7 +876,7 @@ struct NS(TrackJobBase)
         float ms = 0.0f;
         last_kernel_ms = ( hipEventElapsedTime( &ms, ev_start, ev_stop ) == hipSuccess ) ? ms : -1.0f;
         last_status = *h_status;
-        return last_status;
+        return reached( until_turn, last_status );
     }
 
     int32_t track_ebe( int64_t until_turn )
@@ -864,7 +901,7 @@ struct NS(TrackJobBase)
                 : st_launch_track_ebe_exact( &v, d_lat, n_elem, until_turn, &ebe_device_cfg(), plan.ebe_cap, &ebe_view, h_status, from_turn, block, stream );
             ok = ok && hip_ok( err, "launch track_elem_by_elem" );
         }
-        return end_status( ok );
+        return reached( until_turn, end_status( ok ) );
     }
 
     st_ebe_config_t dev_cfg{};
@@ -914,7 +951,7 @@ struct NS(TrackJobBase)
                     : st_launch_track_line_hot_exact( views[ k ].n, &seg, lat, ( int64_t )( e - b ), finish, lat_full, h_status, stream );
                 ok = ok && hip_ok( err, "launch track_line" );
             }
-            return end_status( ok );
+            return line_tracked( finish, end_status( ok ) );
         }
         for( const st_dev_particles_t& v : views )
         {
@@ -923,7 +960,14 @@ struct NS(TrackJobBase)
                 : st_launch_track_line_exact( &v, lat, ( int64_t )( e - b ), finish, h_status, block, stream );
             ok = ok && hip_ok( err, "launch track_line" );
         }
-        return end_status( ok );
+        return line_tracked( finish, end_status( ok ) );
+    }
+
+    // finish: every particle still tracked is one turn further
+    int32_t line_tracked( bool finish, int32_t status )
+    {
+        if( finish && status == 0 && turn_floor < INT64_MAX ) ++turn_floor;
+        return status;
     }
 
     void parse_config( const char* cfg )

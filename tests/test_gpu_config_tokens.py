@@ -6,7 +6,7 @@ import pytest
 torch = pytest.importorskip("torch")
 
 from helpers import assert_particles_equal, particles_dict  # noqa: E402
-from sixtracklib_amd import lattices  # noqa: E402
+from sixtracklib_amd import beam_elements as be, lattices  # noqa: E402
 from sixtracklib_amd.cobjects import CBuffer  # noqa: E402
 from sixtracklib_amd.particles import particles_in  # noqa: E402
 
@@ -45,12 +45,14 @@ def test_batch_config_tells_and_restores_the_walk():
     assert batch.config == seen[1]
 
 
-def _kernels(call):
-    """names of the tracking kernels that ``call`` launches, one per launch"""
+def _kernels(call, every=False):
+    """names of the tracking kernels that ``call`` launches, one per launch;
+    with ``every`` of all of the library's"""
     with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
         call()
         torch.cuda.synchronize()
-    return [e.name.split("(")[0] for e in prof.events() if "_track" in e.name and "st_k_" in e.name]
+    return [e.name.split("(")[0] for e in prof.events()
+            if "st_k_" in e.name and (every or "_track" in e.name)]
 
 
 @pytest.mark.parametrize("n, cfg, walk", [
@@ -90,3 +92,54 @@ def test_autotune_times_every_launch_form_once(hot, one, two):
     pairs = sum("track2" in k for k in names)
     assert one <= len(names) - pairs <= one + 3 and two <= pairs <= two + 3
     assert _tokens(batch)["block"] in (("256",) if hot else ("64", "128", "256"))
+
+
+def _all_lost_at_once(heavy=False):
+    """402 elements, or 3 with a space-charge map; no particle passes the first."""
+    eb = CBuffer(max_slots=65536, max_objects=512, max_pointers=512)
+    be.LimitRect(cbuffer=eb, min_x=-1e-12, max_x=1e-12, min_y=-1e-12, max_y=1e-12)
+    if heavy:
+        be.SCCoasting(cbuffer=eb, number_of_particles=1e10, circumference=1e3, sigma_x=1e-3,
+                               sigma_y=1e-3, length=1.0, x_co=0.0, y_co=0.0, min_sigma_diff=1e-10,
+                               enabled=1)
+    for _ in range(1 if heavy else 401):
+        be.Drift(cbuffer=eb, length=0.1)
+    return eb
+
+
+# one launch holds 2^24 element passes: 41,734 turns of 402 elements; a map out
+# of line counts as many passes as it may take longer than one
+@pytest.mark.parametrize("heavy, at_turn, until, one_launch", [
+    (False, 0, 41734, True), (False, 0, 41735, False),
+    (False, 10**6, 10**6 + 1, True), (False, 2**40, 2**40 + 41734, True),
+    (False, -41000, 734, True), (False, -41000, 735, False),
+    (True, 0, 1000, True), (True, 0, 2**24 // 3, False),
+])
+def test_one_launch_for_as_many_turns_as_are_to_go(heavy, at_turn, until, one_launch):
+    from sixtracklib_amd.trackjob import TrackJob
+    pb, p = lattices.gaussian_beam(100, seed=2, sigma_x=1e-4, sigma_y=1e-4)
+    p.at_turn[:] = at_turn
+    p.at_turn[7], p.state[7] = at_turn - 10**9, 0       # lost: not to be tracked
+    job = TrackJob(_all_lost_at_once(heavy), pb)
+    for _ in range(2):                                  # made with the job, and pushed
+        names = _kernels(lambda: job.track_until(until), every=True)
+        assert (len(names) == 1) == one_launch, names
+        job.push_particles()
+
+
+def test_one_launch_a_turn_far_from_turn_0():
+    """The turns a job has tracked count as done: track_until, track_line."""
+    from sixtracklib_amd.trackjob import TrackJob
+    eb = lattices.fodo_ring(n_cells=100)
+    pb, p = lattices.gaussian_beam(64, seed=2, sigma_x=1e-6, sigma_y=1e-6, sigma_px=1e-8, sigma_py=1e-8)
+    p.at_turn[:] = 41730
+    job = TrackJob(eb, pb)
+    for turn in range(41731, 41740):
+        names = _kernels(lambda: job.track_until(turn), every=True)
+        assert len(names) == 1, (turn, names)
+    for _ in range(3):
+        job.track_line(0, eb.n_objects, finish_turn=True)
+    names = _kernels(lambda: job.track_until(41743), every=True)
+    assert len(names) == 1
+    job.collect()
+    assert np.all(np.array(p.state) == 1) and np.all(np.array(p.at_turn) == 41743)
