@@ -179,7 +179,7 @@ int NS(Adjoint_loss)( const st_adj_plan_t* p, int fma, const double* coords, dou
 int64_t NS(Adjoint_gradient_doubles)( const st_adj_plan_t* p )
 {
     if( p == nullptr || p->base.n < 0 || p->base.n_elem <= 0 || p->n_mp < 0 ) return -1;
-    return st_adj_piece_doubles( p ) + st_adj_partial_doubles( p );
+    return st_adj_piece_doubles( p ) + st_adj_partial_doubles( p ) + st_adj_state_doubles( p );
 }
 
 int NS(Adjoint_gradients)( const st_adj_plan_t* p, int fma, const double* grad_out, double* work,

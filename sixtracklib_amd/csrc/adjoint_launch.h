@@ -39,22 +39,35 @@
 static inline int64_t st_adj_pieces( const st_adj_plan_t* p )
 { return ( p->base.n_elem + ST_ADJ_PIECE - 1 ) / ST_ADJ_PIECE; }
 static inline int64_t st_adj_tiles( const st_adj_plan_t* p ) { return ( p->base.n + 63 ) / 64; }
+// states at piece starts are kept (adjoint_kernels.hip, state_slot)
+static inline bool st_adj_keeps_states( const st_adj_plan_t* p ) { return p->base.K > ST_ADJ_PIECE; }
 // turns whose pieces run side by side; 0: one wave goes through all pieces
 static inline int64_t st_adj_group( const st_adj_plan_t* p )
 {
     if( p->base.n > ST_ADJ_PARALLEL_MAX || p->base.n <= 0 ) return 0;
-    int64_t const turn = st_adj_pieces( p ) * st_adj_tiles( p ) * ( 36 + 6 ) * 64 * 8;
+    int64_t const turn = st_adj_pieces( p ) * st_adj_tiles( p ) *
+                         ( 36 + 6 + ( st_adj_keeps_states( p ) ? 9 : 0 ) ) * 64 * 8;
     int64_t const g = ST_ADJ_PARALLEL_BYTES / turn;
     return g < p->base.n_turns ? g : p->base.n_turns;
 }
 // work: Jacobians [group][piece][36][64 tiles], end cotangents
-// [group][piece][6][64 tiles], partial sums [partials][n_mp][2 (max_order + 1)]
+// [group][piece][6][64 tiles], partial sums [partials][n_mp][2 (max_order + 1)],
+// kept states [group][piece][9][64 tiles], or of the pieces of one
+// checkpoint's range where one wave goes through all pieces
 static inline int64_t st_adj_partials( const st_adj_plan_t* p )
 { return ( st_adj_group( p ) > 0 ? st_adj_group( p ) : 1 ) * st_adj_tiles( p ); }
 static inline int64_t st_adj_piece_doubles( const st_adj_plan_t* p )
 { return st_adj_group( p ) * st_adj_pieces( p ) * ( 36 + 6 ) * 64 * st_adj_tiles( p ); }
 static inline int64_t st_adj_partial_doubles( const st_adj_plan_t* p )
 { return st_adj_partials( p ) * p->n_mp * 2 * ( p->max_order + 1 ); }
+static inline int64_t st_adj_state_doubles( const st_adj_plan_t* p )
+{
+    if( !st_adj_keeps_states( p ) ) return 0;
+    int64_t const range = p->base.K < p->base.n_elem ? p->base.K : p->base.n_elem;
+    int64_t const slots = st_adj_group( p ) > 0 ? st_adj_group( p ) * st_adj_pieces( p )
+                                                : ( range + ST_ADJ_PIECE - 1 ) / ST_ADJ_PIECE;
+    return slots * 9 * 64 * st_adj_tiles( p );
+}
 
 ST_DECLARE_ADJ_LAUNCHERS( _exact )
 ST_DECLARE_ADJ_LAUNCHERS( _fma )
