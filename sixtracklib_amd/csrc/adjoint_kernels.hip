@@ -243,23 +243,29 @@ __global__ void __launch_bounds__( 256 ) KN( st_k_adj_reduce )( int64_t n,
 //     the transposed Jacobian of every piece of 64 elements of every turn,
 //     all pieces side by side (six cotangents through the piece at once,
 //     sharing its states and coefficients); st_k_adj_chain carries the
-//     cotangent from piece to piece, 36 multiply-adds each; st_k_adj_reverse
-//     then goes through every piece once more, again side by side, from its
-//     now known end cotangent, for the coefficient gradients.  Above
+//     cotangent from piece to piece, 36 multiply-adds each.  Terms of those
+//     products cancel, which leaves twice the rounding error of going element
+//     by element; so st_k_adj_through goes through every piece so, side by
+//     side, from the end cotangent found, and st_k_adj_chain_refine carries
+//     on what each piece got wrong (error of the coordinates' gradients
+//     against 80-bit arithmetic on the same states, 16 lattices: 4.2e-15
+//     without, 1.78e-15 with this, turn by turn 1.83e-15).  st_k_adj_reverse
+//     goes through every piece once more for the coefficient gradients.  Above
 //     ST_ADJ_PARALLEL_MAX particles the waves fill the chip without that,
 //     and st_k_adj_reverse alone goes through the pieces one after another;
-//   * a piece's states are recomputed from the nearest checkpoint in parts
-//     of 16 elements, the two coordinates each map's Jacobian needs kept in
-//     LDS (16 KB a wave) instead of nine in memory;
+//   * a piece's states are made from the checkpoints in parts of 8 elements,
+//     the two coordinates each map's Jacobian needs kept in LDS (8 KB a wave;
+//     with parts of 16 half as many waves fit a CU: 293 against 237 us for
+//     st_k_adj_reverse, 168 and 127 for st_k_adj_through);
 //   * the sums over particles are formed in the wave (DPP adds, a fixed
 //     order) instead of through four values per particle and multipole.
 // 4,096 particles, 1,000 elements, 10 turns, exact build: forward 3.9 -> 0.78
-// ms, reverse 9.6 -> 0.70 ms (Jacobians 0.25, chain 0.08, pieces 0.34, sums
-// 0.03).  Reverse and forward, before / now: 64 particles 10.8 / 1.2 ms,
-// 16,384 17.7 / 3.4, 262,144 particles and 2 turns 21.3 / 6.0.  Side by side
-// costs two and a half sweeps instead of one: at 65,536 particles and 2
-// turns 2.4 ms against 2.9 from one wave through all pieces, which wins
-// above.
+// ms, reverse 9.6 -> 0.79 ms (Jacobians 0.25, chain 0.07, through 0.13, its
+// refinement 0.07, coefficients 0.23, sums 0.03).  Backward pass as called,
+// before / now: 64 particles, 10 turns 7.2 / 0.36 ms, 16,384 and 10 turns
+// 13.7 / 2.7.  Side by side costs three and a half sweeps instead of one and
+// wins as long as the particles leave SIMDs idle: 2 turns, 65,536 particles
+// side by side 2.3 ms, 70,000 with one wave through all pieces 2.7.
 namespace
 {
 struct PlanArgs
@@ -278,8 +284,9 @@ struct PlanArgs
     const double* target;
     double* ckpt;
     const double* grad_out;
-    double *jac, *cend, *partial, *grad_coords;
-    double* states;              // K > ST_ADJ_PIECE: states at piece starts, else nullptr
+    double *jac, *cend, *cstart, *partial, *grad_coords;
+    double* states;              // first states of parts (state_slot)
+    int64_t parts, units;
 };
 
 // sum over the 64 lanes, in lane 63, in a fixed order (rows of 16 by shifts,
@@ -342,54 +349,54 @@ ST_DEV void run_elements( const PlanArgs& a, int64_t b, int64_t e, Lane& L, doub
     }
 }
 
-// Checkpoint c of turn t.
-ST_DEV Lane checkpoint( const PlanArgs& a, int64_t t, int64_t c, int64_t i )
+// The kernels of the reverse pass go through pieces of 64 elements in parts of
+// 16, the last first, and each part starts from its first state.  Those are
+// made once from the checkpoints and kept (8 doubles a particle, N particles
+// apart, part by part): a wave goes through a unit of parts, the range of a
+// checkpoint, or a piece where K is smaller, so every element is passed once
+// whatever K is.
+ST_DEV double* state_slot( const PlanArgs& a, int64_t slot )
+{ return a.states + slot * ST_ADJ_STATE * 64 * ( int64_t )a.tiles; }
+
+// first part of unit u
+ST_DEV int64_t unit_begin( const PlanArgs& a, int64_t u )
 {
-    Lane L;
-    get_lane( a.ckpt + ( ( t * a.n_seg + c ) * 9 ) * a.n, a.n, i, L );
-    return L;
+    return a.K > ST_ADJ_PIECE ? ( u * a.K + ST_ADJ_SUB - 1 ) / ST_ADJ_SUB
+                              : u * ( ST_ADJ_PIECE / ST_ADJ_SUB );
 }
 
-// A piece's first state is recomputed from the checkpoint before it.  Up to
-// K = ST_ADJ_PIECE that is less than a piece.  Above, every piece would go
-// through the range again that the pieces before it went through, K / 2
-// elements each; the range is gone through once instead and the states at
-// its pieces' starts are kept, ``slot`` piece by piece (9 doubles a particle,
-// N particles apart).  4,000 elements, K = 4,000, backward pass: 70,000 particles
-// 28.8 -> 5.6 ms (K = 64: 4.4), 4,096 and 4 turns 7.0 -> 2.1 ms (K = 64: 1.2).
-ST_DEV double* state_slot( const PlanArgs& a, int64_t slot )
-{ return a.states + slot * 9 * 64 * ( int64_t )a.tiles; }
-
-// first piece that starts in the range of checkpoint c
-ST_DEV int64_t first_piece( const PlanArgs& a, int64_t c ) { return ( c * a.K + ST_ADJ_PIECE - 1 ) / ST_ADJ_PIECE; }
-
-// the states at the starts of pieces first_piece( c ) .. last of turn t, from
-// slot on
-ST_DEV void keep_states( const PlanArgs& a, int64_t t, int64_t c, int64_t last, int64_t i, int64_t tid,
+// the first states of parts p .. end - 1 of turn t, from slot on
+ST_DEV void keep_states( const PlanArgs& a, int64_t t, int64_t p, int64_t end, int64_t i, int64_t tid,
                          int64_t slot )
 {
-    Lane L = checkpoint( a, t, c, i );
-    int64_t e = c * a.K;
-    for( int64_t j = first_piece( a, c ); j <= last; ++j, ++slot )
+    int64_t const N = 64 * ( int64_t )a.tiles;
+    Lane L;
+    for( int64_t e = 0, c = -1; p < end; ++p, ++slot )
     {
-        run_elements< false >( a, e, j * ST_ADJ_PIECE, L, nullptr );
-        e = j * ST_ADJ_PIECE;
-        put_lane( state_slot( a, slot ), 64 * ( int64_t )a.tiles, tid, L );
+        int64_t const b = p * ST_ADJ_SUB;
+        if( b / a.K != c )
+        {
+            c = b / a.K;
+            e = c * a.K;
+            get_lane( a.ckpt + ( ( t * a.n_seg + c ) * 9 ) * a.n, a.n, i, L );
+        }
+        run_elements< false >( a, e, b, L, nullptr );
+        e = b;
+        double* const s = state_slot( a, slot ) + tid;
+        s[ 0 ] = L.x;        s[ N ] = L.px;         s[ 2 * N ] = L.y;   s[ 3 * N ] = L.py;
+        s[ 4 * N ] = L.zeta; s[ 5 * N ] = L.delta;  s[ 6 * N ] = L.rpp; s[ 7 * N ] = L.rvv;
     }
 }
 
-// state at the start of piece j of turn t, from its slot or recomputed
-ST_DEV Lane piece_state( const PlanArgs& a, int64_t t, int64_t j, int64_t i, int64_t tid, int64_t slot )
+ST_DEV Lane kept_state( const PlanArgs& a, int64_t tid, int64_t slot )
 {
+    int64_t const N = 64 * ( int64_t )a.tiles;
+    const double* const s = state_slot( a, slot ) + tid;
     Lane L;
-    if( a.states != nullptr )
-    {
-        get_lane( state_slot( a, slot ), 64 * ( int64_t )a.tiles, tid, L );
-        return L;
-    }
-    int64_t const e = j * ST_ADJ_PIECE, c = e / a.K;
-    L = checkpoint( a, t, c, i );
-    run_elements< false >( a, c * a.K, e, L, nullptr );
+    L.x = s[ 0 ];        L.px = s[ N ];        L.y = s[ 2 * N ];   L.py = s[ 3 * N ];
+    L.zeta = s[ 4 * N ]; L.delta = s[ 5 * N ]; L.rpp = s[ 6 * N ]; L.rvv = s[ 7 * N ];
+    L.psigma = L.s = 0.0;                           // no map below reads them
+    L.state = 1;
     return L;
 }
 
@@ -464,8 +471,8 @@ ST_DEV void reverse_elements( const PlanArgs& a, int64_t b, int64_t e, const Lan
 #pragma unroll
             for( int q = 0; q < COLS; ++q )
             {
-                c[ q ].x = fma( -c[ q ].px, dre, fma( c[ q ].py, dim, c[ q ].x ) );
-                c[ q ].y = fma( c[ q ].px, dim, fma( c[ q ].py, dre, c[ q ].y ) );
+                c[ q ].x += fma( -c[ q ].px, dre, c[ q ].py * dim );   // one rounding at the
+                c[ q ].y += fma( c[ q ].px, dim, c[ q ].py * dre );    // size of x, of y
             }
             break;
         }
@@ -499,50 +506,53 @@ ST_DEV void reverse_elements( const PlanArgs& a, int64_t b, int64_t e, const Lan
     }
 }
 
-// Piece j of turn t from its first state: the states at the starts of its
-// parts, then part by part, the last first.
+// Parts begin .. end - 1, the last first; slot holds the first state of part
+// begin, those after it the others'.  A part's state is loaded while the part
+// behind it is gone through.
 template< int COLS, bool COEF >
-ST_DEV void reverse_piece( const PlanArgs& a, int64_t j, const Lane& first, double* lds, Cot* c,
+ST_DEV void reverse_parts( const PlanArgs& a, int64_t begin, int64_t end, int64_t tid, int64_t slot,
+                           double* lds, Cot* c, double* part, bool add )
+{
+    if( begin >= end ) return;
+    Lane first = kept_state( a, tid, slot + ( end - 1 - begin ) );
+    for( int64_t p = end - 1; p >= begin; --p )
+    {
+        int64_t const b = p * ST_ADJ_SUB, e = b + ST_ADJ_SUB < a.n_elem ? b + ST_ADJ_SUB : a.n_elem;
+        Lane L = first;
+        first = kept_state( a, tid, slot + ( p > begin ? p - 1 - begin : 0 ) );
+        run_elements< true >( a, b, e, L, lds );
+        reverse_elements< COLS, COEF >( a, b, e, L, lds, c, part, add );
+    }
+}
+
+// Piece j of a turn whose parts' states are from slot on.
+template< int COLS, bool COEF >
+ST_DEV void reverse_piece( const PlanArgs& a, int64_t j, int64_t tid, int64_t slot, double* lds, Cot* c,
                            double* part, bool add )
 {
     constexpr int PARTS = ST_ADJ_PIECE / ST_ADJ_SUB;
-    int64_t const b = j * ST_ADJ_PIECE, e = b + ST_ADJ_PIECE < a.n_elem ? b + ST_ADJ_PIECE : a.n_elem;
-    Lane at[ PARTS ];
-    at[ 0 ] = first;
-#pragma unroll
-    for( int k = 1; k < PARTS; ++k )
-    {
-        int64_t const pb = b + ( k - 1 ) * ST_ADJ_SUB, pe = pb + ST_ADJ_SUB;
-        at[ k ] = at[ k - 1 ];
-        if( pe < e ) run_elements< false >( a, pb, pe, at[ k ], nullptr );
-    }
-#pragma unroll
-    for( int k = PARTS - 1; k >= 0; --k )
-    {
-        int64_t const pb = b + k * ST_ADJ_SUB, pe = pb + ST_ADJ_SUB < e ? pb + ST_ADJ_SUB : e;
-        if( pb >= e ) continue;
-        Lane L = at[ k ];
-        run_elements< true >( a, pb, pe, L, lds );
-        reverse_elements< COLS, COEF >( a, pb, pe, L, lds, c, part, add );
-    }
+    int64_t const first = j * PARTS;
+    reverse_parts< COLS, COEF >( a, first, first + PARTS < a.parts ? first + PARTS : a.parts, tid, slot + first,
+                                 lds, c, part, add );
 }
 
-// loss terms of turn t added to the cotangent at its end
-ST_DEV void add_loss_terms( const PlanArgs& a, int64_t t, int64_t i, Cot& c )
+// component p of the loss terms of turn t, weight w, g = 2 x the loss's cotangent
+ST_DEV double loss_term( const PlanArgs& a, double w, int64_t t, int p, int64_t i, double g )
 {
     const double* const b = a.ckpt + ( ( t + 1 ) * a.n_seg * 9 ) * a.n;   // the next turn's first
-    const double* const tg = a.target + t * 6;
-    double const g = 2.0 * *a.grad_out;
-    c.x += g * a.w[ 0 ] * ( b[ 0 * a.n + i ] - tg[ 0 ] );
-    c.px += g * a.w[ 1 ] * ( b[ 1 * a.n + i ] - tg[ 1 ] );
-    c.y += g * a.w[ 2 ] * ( b[ 2 * a.n + i ] - tg[ 2 ] );
-    c.py += g * a.w[ 3 ] * ( b[ 3 * a.n + i ] - tg[ 3 ] );
-    c.zeta += g * a.w[ 4 ] * ( b[ 4 * a.n + i ] - tg[ 4 ] );
-    c.delta += g * a.w[ 5 ] * ( b[ 5 * a.n + i ] - tg[ 5 ] );
+    return g * w * ( b[ p * a.n + i ] - a.target[ t * 6 + p ] );
 }
 
-ST_DEV Cot load_cot( const double* g, int64_t i )
-{ return Cot{ g[ 6 * i ], g[ 6 * i + 1 ], g[ 6 * i + 2 ], g[ 6 * i + 3 ], g[ 6 * i + 4 ], g[ 6 * i + 5 ] }; }
+ST_DEV void add_loss_terms( const PlanArgs& a, int64_t t, int64_t i, Cot& c )
+{
+    double const g = 2.0 * *a.grad_out;
+    c.x += loss_term( a, a.w[ 0 ], t, 0, i, g );
+    c.px += loss_term( a, a.w[ 1 ], t, 1, i, g );
+    c.y += loss_term( a, a.w[ 2 ], t, 2, i, g );
+    c.py += loss_term( a, a.w[ 3 ], t, 3, i, g );
+    c.zeta += loss_term( a, a.w[ 4 ], t, 4, i, g );
+    c.delta += loss_term( a, a.w[ 5 ], t, 5, i, g );
+}
 
 ST_DEV void store_cot( double* g, int64_t i, const Cot& c )
 {
@@ -651,15 +661,16 @@ __global__ void __launch_bounds__( 64, 4 ) KN( st_k_adj_loss )( PlanArgs a, cons
     if( !ok ) report_failure( status );
 }
 
-// block (turn, checkpoint, tile), tile fastest: the states at the starts of
-// the pieces in the checkpoint's range, slot (turn, piece)
+// block (turn, unit, tile), tile fastest: the first states of the unit's
+// parts, slot (turn, part)
 __global__ void __launch_bounds__( 64, 4 ) KN( st_k_adj_states )( PlanArgs a )
 {
-    int64_t const tile = blockIdx.x % a.tiles, tc = blockIdx.x / a.tiles;
-    int64_t const c = tc % a.n_seg, k = tc / a.n_seg;
+    int64_t const tile = blockIdx.x % a.tiles, tu = blockIdx.x / a.tiles;
+    int64_t const u = tu % a.units, k = tu / a.units;
     int64_t const tid = tile * 64 + threadIdx.x;
-    int64_t const end = first_piece( a, c + 1 ) < a.pieces ? first_piece( a, c + 1 ) : a.pieces;
-    keep_states( a, a.t0 + k, c, end - 1, tid < a.n ? tid : a.n - 1, tid, k * a.pieces + first_piece( a, c ) );
+    int64_t const begin = unit_begin( a, u ), next = unit_begin( a, u + 1 );
+    keep_states( a, a.t0 + k, begin, next < a.parts ? next : a.parts, tid < a.n ? tid : a.n - 1, tid,
+                 k * a.parts + begin );
 }
 
 // block (turn, piece, tile), tile fastest: d (cotangent at the piece's
@@ -668,15 +679,20 @@ __global__ void __launch_bounds__( 64, 2 ) KN( st_k_adj_jacobian )( PlanArgs a )
 {
     __shared__ double lds[ ST_ADJ_SUB * 128 ];
     int64_t const tile = blockIdx.x % a.tiles, tp = blockIdx.x / a.tiles;
-    int64_t const j = tp % a.pieces, t = a.t0 + tp / a.pieces;
+    int64_t const j = tp % a.pieces, k = tp / a.pieces;
     int64_t const tid = tile * 64 + threadIdx.x;
-    int64_t const i = tid < a.n ? tid : a.n - 1;
     Cot c[ 6 ];
 #pragma unroll
     for( int q = 0; q < 6; ++q )
         c[ q ] = Cot{ q == 0 ? 1.0 : 0.0, q == 1 ? 1.0 : 0.0, q == 2 ? 1.0 : 0.0,
                       q == 3 ? 1.0 : 0.0, q == 4 ? 1.0 : 0.0, q == 5 ? 1.0 : 0.0 };
-    reverse_piece< 6, false >( a, j, piece_state( a, t, j, i, tid, tp ), lds + threadIdx.x, c, nullptr, false );
+    if( a.K <= ST_ADJ_PIECE )                          // its unit is this piece
+    {
+        int64_t const begin = unit_begin( a, j ), next = unit_begin( a, j + 1 );
+        keep_states( a, a.t0 + k, begin, next < a.parts ? next : a.parts, tid < a.n ? tid : a.n - 1, tid,
+                     k * a.parts + begin );
+    }
+    reverse_piece< 6, false >( a, j, tid, k * a.parts, lds + threadIdx.x, c, nullptr, false );
     int64_t const N = 64 * ( int64_t )a.tiles;
     double* const J = a.jac + tp * 36 * N + tid;
 #pragma unroll
@@ -689,47 +705,99 @@ __global__ void __launch_bounds__( 64, 2 ) KN( st_k_adj_jacobian )( PlanArgs a )
 }
 
 // The cotangent through the pieces of the group's turns, last first; every
-// piece's end cotangent is kept.  The next piece's Jacobian is loaded while
-// one is applied.
-__global__ void __launch_bounds__( 64, 1 ) KN( st_k_adj_chain )( PlanArgs a )
+// piece's end cotangent is kept.  REFINE: once more, each piece's start
+// cotangent from the one that st_k_adj_through found for the kept end
+// cotangent, and the Jacobian applied to the little by which the end
+// cotangent has changed.
+//
+// The pieces are a chain, so what bounds it is how fast the CUs that hold it
+// take in the Jacobians, and one CU takes in some 35 GB/s, whatever its waves
+// have in flight (64 particles a block: 0.5 us a piece, with one wave or with
+// six).  So a block has 16 particles, whose rows are a cache line each, and
+// two waves of 48 lanes, three components each.
+template< bool REFINE >
+ST_DEV void adj_chain( const PlanArgs& a )
 {
-    int64_t const tid = ( int64_t )blockIdx.x * 64 + threadIdx.x;
-    bool const in_range = tid < a.n;
-    int64_t const i = in_range ? tid : a.n - 1;
+    __shared__ double v[ 2 ][ 6 ][ 16 ];               // by turns: what the Jacobian is applied to
+    __shared__ double weight[ 6 ];
+    if( threadIdx.x < 6 ) weight[ threadIdx.x ] = a.w[ threadIdx.x ];
+    __syncthreads();
+    int const l = ( int )threadIdx.x & 63, k = l & 15;
+    bool const idle = l >= 48;                         // kept for the barriers
+    int const p = 3 * ( int )( threadIdx.x >> 6 ) + ( idle ? 0 : l >> 4 );
+    int64_t const tid = ( int64_t )blockIdx.x * 16 + k;
+    int64_t const i = tid < a.n ? tid : a.n - 1;
     int64_t const N = 64 * ( int64_t )a.tiles;
-    Cot c{ 0.0, 0.0, 0.0, 0.0, 0.0, 0.0 };
-    if( a.add ) c = load_cot( a.grad_coords, i );
-    double J[ 2 ][ 36 ];
+    double const g = 2.0 * *a.grad_out;
     int64_t const last = ( int64_t )a.turns * a.pieces - 1;
     auto load = [ & ]( int64_t tp, double* into )
     {
-        const double* const g = a.jac + ( tp < 0 ? 0 : tp ) * 36 * N + tid;
+        if( tp < 0 || idle ) return;
+        const double* const J = a.jac + ( tp * 36 + p ) * N + tid;
 #pragma unroll
-        for( int k = 0; k < 36; ++k ) into[ k ] = g[ k * N ];
+        for( int q = 0; q < 6; ++q ) into[ q ] = J[ 6 * q * N ];
+        if( REFINE )
+        {
+            into[ 6 ] = a.cend[ ( tp * 6 + p ) * N + tid ];
+            into[ 7 ] = a.cstart[ ( tp * 6 + p ) * N + tid ];
+        }
     };
+    double c = a.add ? a.grad_coords[ 6 * i + p ] : 0.0;
     auto step = [ & ]( int64_t tp, const double* M )
     {
-        if( tp % a.pieces == a.pieces - 1 ) add_loss_terms( a, a.t0 + tp / a.pieces, i, c );
-        double* const ce = a.cend + tp * 6 * N + tid;
-        ce[ 0 ] = c.x; ce[ N ] = c.px; ce[ 2 * N ] = c.y;
-        ce[ 3 * N ] = c.py; ce[ 4 * N ] = c.zeta; ce[ 5 * N ] = c.delta;
-        double r[ 6 ];
-#pragma unroll
-        for( int p = 0; p < 6; ++p )
-            r[ p ] = fma( M[ p ], c.x, fma( M[ 6 + p ], c.px, fma( M[ 12 + p ], c.y,
-                     fma( M[ 18 + p ], c.py, fma( M[ 24 + p ], c.zeta, M[ 30 + p ] * c.delta ) ) ) ) );
-        c = Cot{ r[ 0 ], r[ 1 ], r[ 2 ], r[ 3 ], r[ 4 ], r[ 5 ] };
+        double( *const w )[ 16 ] = v[ tp & 1 ];
+        if( !idle )
+        {
+            if( tp % a.pieces == a.pieces - 1 ) c += loss_term( a, weight[ p ], a.t0 + tp / a.pieces, p, i, g );
+            a.cend[ ( tp * 6 + p ) * N + tid ] = c;
+            w[ p ][ k ] = REFINE ? c - M[ 6 ] : c;
+        }
+        __syncthreads();
+        double const r = fma( M[ 0 ], w[ 0 ][ k ], fma( M[ 1 ], w[ 1 ][ k ], fma( M[ 2 ], w[ 2 ][ k ],
+                         fma( M[ 3 ], w[ 3 ][ k ], fma( M[ 4 ], w[ 4 ][ k ], M[ 5 ] * w[ 5 ][ k ] ) ) ) ) );
+        c = REFINE ? M[ 7 ] + r : r;
     };
-    load( last, J[ 0 ] );
-    for( int64_t tp = last; tp >= 0; tp -= 2 )
+    constexpr int AHEAD = 4;
+    double M[ AHEAD ][ 8 ] = {};
+#pragma unroll
+    for( int j = 0; j < AHEAD - 1; ++j ) load( last - j, M[ j ] );
+    for( int64_t tp = last; tp >= 0; tp -= AHEAD )
     {
-        load( tp - 1, J[ 1 ] );
-        step( tp, J[ 0 ] );
-        if( tp == 0 ) break;
-        load( tp - 2, J[ 0 ] );
-        step( tp - 1, J[ 1 ] );
+#pragma unroll
+        for( int j = 0; j < AHEAD; ++j )
+        {
+            if( tp - j < 0 ) break;
+            load( tp - j - ( AHEAD - 1 ), M[ ( j + AHEAD - 1 ) % AHEAD ] );
+            step( tp - j, M[ j ] );
+        }
     }
-    if( in_range ) store_cot( a.grad_coords, i, c );
+    if( REFINE && !idle && tid < a.n ) a.grad_coords[ 6 * i + p ] = c;
+}
+
+__global__ void __launch_bounds__( 128 ) KN( st_k_adj_chain )( PlanArgs a )
+{
+    adj_chain< false >( a );
+}
+
+__global__ void __launch_bounds__( 128 ) KN( st_k_adj_chain_refine )( PlanArgs a )
+{
+    adj_chain< true >( a );
+}
+
+// block (turn, piece, tile): a piece's start cotangent, element by element
+// from its end cotangent
+__global__ void __launch_bounds__( 64, 2 ) KN( st_k_adj_through )( PlanArgs a )
+{
+    __shared__ double lds[ ST_ADJ_SUB * 128 ];
+    int64_t const tile = blockIdx.x % a.tiles, tp = blockIdx.x / a.tiles;
+    int64_t const j = tp % a.pieces, k = tp / a.pieces, N = 64 * ( int64_t )a.tiles;
+    int64_t const tid = tile * 64 + threadIdx.x;
+    const double* const ce = a.cend + tp * 6 * N + tid;
+    Cot c{ ce[ 0 ], ce[ N ], ce[ 2 * N ], ce[ 3 * N ], ce[ 4 * N ], ce[ 5 * N ] };
+    reverse_piece< 1, false >( a, j, tid, k * a.parts, lds + threadIdx.x, &c, nullptr, false );
+    double* const cs = a.cstart + tp * 6 * N + tid;
+    cs[ 0 ] = c.x; cs[ N ] = c.px; cs[ 2 * N ] = c.y;
+    cs[ 3 * N ] = c.py; cs[ 4 * N ] = c.zeta; cs[ 5 * N ] = c.delta;
 }
 
 // CHAIN: one wave goes through all pieces of all turns, last first, with its
@@ -749,25 +817,21 @@ ST_DEV void adj_reverse( const PlanArgs& a, double* lds )
         int64_t const j = tp % a.pieces, k = tp / a.pieces, N = 64 * ( int64_t )a.tiles;
         const double* const ce = a.cend + tp * 6 * N + tid;
         if( in_range ) c = Cot{ ce[ 0 ], ce[ N ], ce[ 2 * N ], ce[ 3 * N ], ce[ 4 * N ], ce[ 5 * N ] };
-        reverse_piece< 1, true >( a, j, piece_state( a, a.t0 + k, j, i, tid, tp ), lds, &c,
+        reverse_piece< 1, true >( a, j, tid, k * a.parts, lds, &c,
                                   a.partial + ( k * a.tiles + tile ) * row, a.add != 0 );
         return;
     }
     for( int64_t t = a.n_turns - 1; t >= 0; --t )
     {
         if( in_range ) add_loss_terms( a, t, i, c );
-        int64_t kept = a.n_seg, first = 0;         // checkpoint whose pieces' states are kept, from slot 0
-        for( int64_t j = a.pieces - 1; j >= 0; --j )
+        // unit by unit, the last first; its states from slot 0 on
+        int64_t end = a.parts;
+        for( int64_t u = a.units - 1; u >= 0; --u )
         {
-            int64_t const r = j * ST_ADJ_PIECE / a.K;
-            if( a.states != nullptr && r != kept )
-            {
-                keep_states( a, t, r, j, i, tid, 0 );
-                kept = r;
-                first = first_piece( a, r );
-            }
-            reverse_piece< 1, true >( a, j, piece_state( a, t, j, i, tid, j - first ), lds, &c,
-                                      a.partial + tile * row, t < a.n_turns - 1 );
+            int64_t const begin = unit_begin( a, u );
+            keep_states( a, t, begin, end, i, tid, 0 );
+            reverse_parts< 1, true >( a, begin, end, tid, 0, lds, &c, a.partial + tile * row, t < a.n_turns - 1 );
+            end = begin < end ? begin : end;
         }
     }
     if( in_range ) store_cot( a.grad_coords, i, c );
@@ -878,6 +942,7 @@ PlanArgs plan_args( const st_adj_plan_t* p )
     a.n_turns = p->base.n_turns; a.n = p->base.n; a.n_mp = p->n_mp;
     a.no = ( int32_t )p->max_order + 1;
     a.tiles = ( int32_t )st_adj_tiles( p ); a.pieces = ( int32_t )st_adj_pieces( p );
+    a.parts = st_adj_parts( p ); a.units = st_adj_units( p );
     a.C.q0 = p->base.q0; a.C.mass0 = p->base.mass0; a.C.beta0 = p->base.beta0; a.C.p0c = p->base.p0c;
     a.C.chi = p->base.chi; a.C.charge_ratio = p->base.charge_ratio;
     for( int c = 0; c < 6; ++c ) a.w[ c ] = p->base.weights[ c ];
@@ -915,8 +980,9 @@ extern "C" hipError_t KN( st_launch_adj_gradients )( const st_adj_plan_t* p, con
     int64_t const group = st_adj_group( p ), tiles = st_adj_tiles( p ), pieces = st_adj_pieces( p );
     a.jac = work;
     a.cend = work + group * pieces * 36 * 64 * tiles;
+    a.cstart = a.cend + group * pieces * 6 * 64 * tiles;
     a.partial = work + st_adj_piece_doubles( p );
-    a.states = st_adj_keeps_states( p ) ? a.partial + st_adj_partial_doubles( p ) : nullptr;
+    a.states = a.partial + st_adj_partial_doubles( p );
     if( p->base.n > 0 && group > 0 )
     {
         for( int64_t end = p->base.n_turns; end > 0; end -= group )
@@ -927,11 +993,13 @@ extern "C" hipError_t KN( st_launch_adj_gradients )( const st_adj_plan_t* p, con
             a.turns = ( int32_t )( end - a.t0 );
             a.add = end < p->base.n_turns ? 1 : 0;
             unsigned const grid = ( unsigned )( a.turns * pieces * tiles );
-            if( a.states != nullptr )
-                hipLaunchKernelGGL( KN( st_k_adj_states ), dim3( ( unsigned )( a.turns * a.n_seg * tiles ) ),
+            if( a.K > ST_ADJ_PIECE )
+                hipLaunchKernelGGL( KN( st_k_adj_states ), dim3( ( unsigned )( a.turns * a.units * tiles ) ),
                                     dim3( 64 ), 0, stream, a );
             hipLaunchKernelGGL( KN( st_k_adj_jacobian ), dim3( grid ), dim3( 64 ), 0, stream, a );
-            hipLaunchKernelGGL( KN( st_k_adj_chain ), dim3( ( unsigned )tiles ), dim3( 64 ), 0, stream, a );
+            hipLaunchKernelGGL( KN( st_k_adj_chain ), dim3( ( unsigned )( 4 * tiles ) ), dim3( 128 ), 0, stream, a );
+            hipLaunchKernelGGL( KN( st_k_adj_through ), dim3( grid ), dim3( 64 ), 0, stream, a );
+            hipLaunchKernelGGL( KN( st_k_adj_chain_refine ), dim3( ( unsigned )( 4 * tiles ) ), dim3( 128 ), 0, stream, a );
             hipLaunchKernelGGL( KN( st_k_adj_reverse ), dim3( grid ), dim3( 64 ), 0, stream, a );
             hipError_t const e = hipGetLastError();
             if( e != hipSuccess ) return e;

@@ -28,45 +28,50 @@
         double* grad_ksl, hipStream_t stream );
 
 // Reverse pass (adjoint_kernels.hip): elements of a piece and of the part of
-// it whose states are in LDS at a time; the particle count up to which the
-// pieces of a group of turns run side by side, and the bytes their
-// Jacobians may take.
+// it whose states are in LDS at a time, doubles of a kept state; the particle
+// count up to which the pieces of a group of turns run side by side, and the
+// bytes that may take.
 #define ST_ADJ_PIECE 64
-#define ST_ADJ_SUB 16
+#define ST_ADJ_SUB 8
+#define ST_ADJ_STATE 8
 #define ST_ADJ_PARALLEL_MAX 65536
 #define ST_ADJ_PARALLEL_BYTES ( int64_t( 1 ) << 32 )
 
 static inline int64_t st_adj_pieces( const st_adj_plan_t* p )
 { return ( p->base.n_elem + ST_ADJ_PIECE - 1 ) / ST_ADJ_PIECE; }
 static inline int64_t st_adj_tiles( const st_adj_plan_t* p ) { return ( p->base.n + 63 ) / 64; }
-// states at piece starts are kept (adjoint_kernels.hip, state_slot)
-static inline bool st_adj_keeps_states( const st_adj_plan_t* p ) { return p->base.K > ST_ADJ_PIECE; }
+static inline int64_t st_adj_parts( const st_adj_plan_t* p )
+{ return ( p->base.n_elem + ST_ADJ_SUB - 1 ) / ST_ADJ_SUB; }
+// units whose parts' first states a wave makes: the ranges of the checkpoints,
+// or the pieces where K is smaller
+static inline int64_t st_adj_units( const st_adj_plan_t* p )
+{ return p->base.K > ST_ADJ_PIECE ? ( p->base.n_elem + p->base.K - 1 ) / p->base.K : st_adj_pieces( p ); }
 // turns whose pieces run side by side; 0: one wave goes through all pieces
 static inline int64_t st_adj_group( const st_adj_plan_t* p )
 {
     if( p->base.n > ST_ADJ_PARALLEL_MAX || p->base.n <= 0 ) return 0;
-    int64_t const turn = st_adj_pieces( p ) * st_adj_tiles( p ) *
-                         ( 36 + 6 + ( st_adj_keeps_states( p ) ? 9 : 0 ) ) * 64 * 8;
+    int64_t const turn = ( st_adj_pieces( p ) * ( 36 + 6 + 6 ) + st_adj_parts( p ) * ST_ADJ_STATE ) *
+                         64 * st_adj_tiles( p ) * 8;
     int64_t const g = ST_ADJ_PARALLEL_BYTES / turn;
     return g < p->base.n_turns ? g : p->base.n_turns;
 }
-// work: Jacobians [group][piece][36][64 tiles], end cotangents
-// [group][piece][6][64 tiles], partial sums [partials][n_mp][2 (max_order + 1)],
-// kept states [group][piece][9][64 tiles], or of the pieces of one
-// checkpoint's range where one wave goes through all pieces
+// work: Jacobians [group][piece][36][64 tiles], end and start cotangents
+// [group][piece][6][64 tiles] each, partial sums [partials][n_mp][2 (max_order + 1)],
+// first states of parts [group][part][8][64 tiles], or of the parts of one
+// unit where one wave goes through all pieces
 static inline int64_t st_adj_partials( const st_adj_plan_t* p )
 { return ( st_adj_group( p ) > 0 ? st_adj_group( p ) : 1 ) * st_adj_tiles( p ); }
 static inline int64_t st_adj_piece_doubles( const st_adj_plan_t* p )
-{ return st_adj_group( p ) * st_adj_pieces( p ) * ( 36 + 6 ) * 64 * st_adj_tiles( p ); }
+{ return st_adj_group( p ) * st_adj_pieces( p ) * ( 36 + 6 + 6 ) * 64 * st_adj_tiles( p ); }
 static inline int64_t st_adj_partial_doubles( const st_adj_plan_t* p )
 { return st_adj_partials( p ) * p->n_mp * 2 * ( p->max_order + 1 ); }
 static inline int64_t st_adj_state_doubles( const st_adj_plan_t* p )
 {
-    if( !st_adj_keeps_states( p ) ) return 0;
-    int64_t const range = p->base.K < p->base.n_elem ? p->base.K : p->base.n_elem;
-    int64_t const slots = st_adj_group( p ) > 0 ? st_adj_group( p ) * st_adj_pieces( p )
-                                                : ( range + ST_ADJ_PIECE - 1 ) / ST_ADJ_PIECE;
-    return slots * 9 * 64 * st_adj_tiles( p );
+    int64_t const unit = p->base.K > ST_ADJ_PIECE ? p->base.K : ST_ADJ_PIECE;
+    int64_t const range = unit < p->base.n_elem ? unit : p->base.n_elem;
+    int64_t const slots = st_adj_group( p ) > 0 ? st_adj_group( p ) * st_adj_parts( p )
+                                                : ( range + ST_ADJ_SUB - 1 ) / ST_ADJ_SUB;
+    return slots * ST_ADJ_STATE * 64 * st_adj_tiles( p );
 }
 
 ST_DECLARE_ADJ_LAUNCHERS( _exact )

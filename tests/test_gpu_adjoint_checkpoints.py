@@ -27,6 +27,11 @@ def test_gradients_over_K_one_wave_through_all_pieces(K):
     _compare(_lattice(200, 5), 65601, 2, K, False, default=False)
 
 
+def test_gradients_in_groups_that_do_not_divide_the_turns():
+    """2,000 elements, 65,536 particles: a group of turns is two."""
+    _compare(lattices.adjoint_sublattice(n_cells=40, tune=8.62), 65536, 3, 64, False, default=False)
+
+
 def _backward_seconds(eb, n, turns, K):
     from sixtracklib_amd.adjoint import AdjointTracker
     rng = np.random.default_rng(1)
@@ -48,7 +53,7 @@ def _backward_seconds(eb, n, turns, K):
 @pytest.mark.parametrize("n, turns", [(4096, 4), (70000, 1)])
 def test_the_backward_pass_is_linear_in_K(n, turns):
     """4,000 elements and one checkpoint a turn: the range is gone through once
-    more than with K = 64 (measured 1.8 and 1.3 times the time; 5.9 and 6.6
+    more than with K = 64 (measured 1.6 and 1.2 times the time; 5.9 and 6.6
     when each of the 63 pieces went through what lies before it)."""
     eb = lattices.adjoint_sublattice(n_cells=80, tune=17.24)
     assert _backward_seconds(eb, n, turns, 4000) < 3.0 * _backward_seconds(eb, n, turns, 64)

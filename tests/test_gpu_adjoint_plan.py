@@ -127,7 +127,7 @@ def test_gradients_of_more_particles_than_run_side_by_side():
 
 
 def test_gradients_in_groups_of_turns():
-    """4,000 elements, 65,536 particles: a group of turns is three."""
+    """4,000 elements, 65,536 particles: a group of turns is one."""
     _compare(lattices.adjoint_sublattice(n_cells=80, tune=17.24), 65536, 4, 64, False, default=False)
 
 
