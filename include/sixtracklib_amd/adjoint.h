@@ -124,14 +124,23 @@ ST_API int NS(Adjoint_coefficients)( const st_adj_plan_t* p, int fma, const doub
 ST_API int NS(Adjoint_loss)( const st_adj_plan_t* p, int fma, const double* coords, double* loss,
     int32_t* status, void* stream );
 
-/* doubles of work NS(Adjoint_gradients) needs */
+/* doubles of work NS(Adjoint_gradients) needs, at most 4 GiB of them or what
+ * one wave through all elements needs */
 ST_API int64_t NS(Adjoint_gradient_doubles)( const st_adj_plan_t* p );
+/* The same for callers short of memory: the most that is at most max_doubles
+ * (fewer turns at a time, slower), or, where that is less than one turn takes,
+ * what one wave through all elements needs, which may be more. */
+ST_API int64_t NS(Adjoint_gradient_doubles_within)( const st_adj_plan_t* p, int64_t max_doubles );
 
 /* gradients of grad_out (device scalar) x the sum of the losses after
  * NS(Adjoint_loss): grad_coords [n][6]; grad_knl, grad_ksl
  * [n_mp][max_order + 1], zero above a multipole's order */
 ST_API int NS(Adjoint_gradients)( const st_adj_plan_t* p, int fma, const double* grad_out,
     double* work, double* grad_coords, double* grad_knl, double* grad_ksl, void* stream );
+/* with work_doubles of work, as NS(Adjoint_gradient_doubles_within) gives them */
+ST_API int NS(Adjoint_gradients_within)( const st_adj_plan_t* p, int fma, const double* grad_out,
+    double* work, int64_t work_doubles, double* grad_coords, double* grad_knl, double* grad_ksl,
+    void* stream );
 
 #if defined( __cplusplus )
 }

@@ -85,10 +85,11 @@ _lib.st_Adjoint_coefficients.argtypes = [ct.POINTER(AdjPlan), ct.c_int, ct.c_voi
 _lib.st_Adjoint_loss.restype = ct.c_int
 _lib.st_Adjoint_loss.argtypes = [ct.POINTER(AdjPlan), ct.c_int, ct.c_void_p, ct.c_void_p,
                                  ct.c_void_p, ct.c_void_p]
-_lib.st_Adjoint_gradient_doubles.restype = ct.c_int64
-_lib.st_Adjoint_gradient_doubles.argtypes = [ct.POINTER(AdjPlan)]
-_lib.st_Adjoint_gradients.restype = ct.c_int
-_lib.st_Adjoint_gradients.argtypes = [ct.POINTER(AdjPlan), ct.c_int] + [ct.c_void_p] * 6
+_lib.st_Adjoint_gradient_doubles_within.restype = ct.c_int64
+_lib.st_Adjoint_gradient_doubles_within.argtypes = [ct.POINTER(AdjPlan), ct.c_int64]
+_lib.st_Adjoint_gradients_within.restype = ct.c_int
+_lib.st_Adjoint_gradients_within.argtypes = ([ct.POINTER(AdjPlan), ct.c_int] + [ct.c_void_p] * 2 +
+                                             [ct.c_int64] + [ct.c_void_p] * 4)
 
 
 def _check(rc, what):
@@ -302,6 +303,20 @@ def _forward(tr, coords, knl, ksl, tgt):
     return loss, (X, ckpt)
 
 
+def _work(plan, device):
+    """Work memory of the gradients: as much as they can use, less where the
+    device has no room for it."""
+    limit = 2**62
+    while True:
+        doubles = int(_lib.st_Adjoint_gradient_doubles_within(ct.byref(plan), limit))
+        try:
+            return torch.empty(max(doubles, 1), dtype=torch.float64, device=device)
+        except torch.OutOfMemoryError:
+            if doubles > limit or limit == 0:          # nothing smaller is left
+                raise
+            limit = doubles // 2 if doubles > 1 else 0
+
+
 class _TrackLoss(torch.autograd.Function):
     @staticmethod
     def forward(ctx, coords, knl, ksl, tgt, tr):
@@ -323,13 +338,12 @@ class _TrackLoss(torch.autograd.Function):
         plan = tr.plan(n, tgt, ckpt)
         # the lattice may have been rewritten since the forward pass
         tr.write_coefficients(*((tr.knl0, tr.ksl0) if ctx.default else (knl, ksl)), plan)
-        work = torch.empty(int(_lib.st_Adjoint_gradient_doubles(ct.byref(plan))) + 1,
-                           dtype=torch.float64, device=dev)
         grad_coords = torch.empty(n, 6, dtype=torch.float64, device=dev)
         grad_knl = torch.empty(tr.n_mp, tr.max_order + 1, dtype=torch.float64, device=dev)
         grad_ksl = torch.empty_like(grad_knl)
         g = grad_out.to(torch.float64).reshape(1).contiguous()
-        _check(_lib.st_Adjoint_gradients(ct.byref(plan), tr.fma, g.data_ptr(), work.data_ptr(),
-                                         grad_coords.data_ptr(), grad_knl.data_ptr(),
-                                         grad_ksl.data_ptr(), _stream()), "adjoint gradients")
+        work = _work(plan, dev)
+        _check(_lib.st_Adjoint_gradients_within(ct.byref(plan), tr.fma, g.data_ptr(), work.data_ptr(),
+                                                work.numel(), grad_coords.data_ptr(), grad_knl.data_ptr(),
+                                                grad_ksl.data_ptr(), _stream()), "adjoint gradients")
         return grad_coords, grad_knl, grad_ksl, None, None

@@ -176,14 +176,20 @@ int NS(Adjoint_loss)( const st_adj_plan_t* p, int fma, const double* coords, dou
                      : st_launch_adj_loss_exact( p, coords, loss, status, s ), "adjoint loss" );
 }
 
-int64_t NS(Adjoint_gradient_doubles)( const st_adj_plan_t* p )
+int64_t NS(Adjoint_gradient_doubles_within)( const st_adj_plan_t* p, int64_t max_doubles )
 {
-    if( p == nullptr || p->base.n < 0 || p->base.n_elem <= 0 || p->n_mp < 0 ) return -1;
-    return st_adj_piece_doubles( p ) + st_adj_partial_doubles( p ) + st_adj_state_doubles( p );
+    if( p == nullptr || p->base.n < 0 || p->base.n_elem <= 0 || p->base.K <= 0 || p->n_mp < 0 ||
+        p->max_order < 0 ) return -1;
+    return st_adj_work_doubles( p, st_adj_group( p, max_doubles ) );
 }
 
-int NS(Adjoint_gradients)( const st_adj_plan_t* p, int fma, const double* grad_out, double* work,
-    double* grad_coords, double* grad_knl, double* grad_ksl, void* stream )
+int64_t NS(Adjoint_gradient_doubles)( const st_adj_plan_t* p )
+{
+    return NS(Adjoint_gradient_doubles_within)( p, INT64_MAX );
+}
+
+int NS(Adjoint_gradients_within)( const st_adj_plan_t* p, int fma, const double* grad_out, double* work,
+    int64_t work_doubles, double* grad_coords, double* grad_knl, double* grad_ksl, void* stream )
 {
     if( !valid_plan( p ) || grad_out == nullptr || work == nullptr || grad_coords == nullptr ||
         ( p->n_mp > 0 && ( grad_knl == nullptr || grad_ksl == nullptr ) ) )
@@ -191,10 +197,22 @@ int NS(Adjoint_gradients)( const st_adj_plan_t* p, int fma, const double* grad_o
         st_internal_set_error( "adjoint gradients: invalid arguments" );
         return -1;
     }
+    int64_t const group = st_adj_group( p, work_doubles );
+    if( work_doubles < st_adj_work_doubles( p, group ) )
+    {
+        st_internal_set_error( "adjoint gradients: not enough work memory" );
+        return -1;
+    }
     hipStream_t const s = static_cast< hipStream_t >( stream );
-    return done( fma ? st_launch_adj_gradients_fma( p, grad_out, work, grad_coords, grad_knl, grad_ksl, s )
-                     : st_launch_adj_gradients_exact( p, grad_out, work, grad_coords, grad_knl, grad_ksl, s ),
+    return done( fma ? st_launch_adj_gradients_fma( p, grad_out, work, group, grad_coords, grad_knl, grad_ksl, s )
+                     : st_launch_adj_gradients_exact( p, grad_out, work, group, grad_coords, grad_knl, grad_ksl, s ),
                  "adjoint gradients" );
+}
+
+int NS(Adjoint_gradients)( const st_adj_plan_t* p, int fma, const double* grad_out, double* work,
+    double* grad_coords, double* grad_knl, double* grad_ksl, void* stream )
+{
+    return NS(Adjoint_gradients_within)( p, fma, grad_out, work, INT64_MAX, grad_coords, grad_knl, grad_ksl, stream );
 }
 
 }  // extern "C"

@@ -972,17 +972,18 @@ extern "C" hipError_t KN( st_launch_adj_loss )( const st_adj_plan_t* p, const do
 }
 
 extern "C" hipError_t KN( st_launch_adj_gradients )( const st_adj_plan_t* p, const double* grad_out,
-    double* work, double* grad_coords, double* grad_knl, double* grad_ksl, hipStream_t stream )
+    double* work, int64_t group, double* grad_coords, double* grad_knl, double* grad_ksl, hipStream_t stream )
 {
     PlanArgs a = plan_args( p );
     a.grad_out = grad_out;
     a.grad_coords = grad_coords;
-    int64_t const group = st_adj_group( p ), tiles = st_adj_tiles( p ), pieces = st_adj_pieces( p );
+    int64_t const tiles = st_adj_tiles( p ), pieces = st_adj_pieces( p );
+    int64_t const partials = p->base.n > 0 ? ( group > 0 ? group : 1 ) * tiles : 0;
     a.jac = work;
-    a.cend = work + group * pieces * 36 * 64 * tiles;
+    a.cend = a.jac + group * pieces * 36 * 64 * tiles;
     a.cstart = a.cend + group * pieces * 6 * 64 * tiles;
-    a.partial = work + st_adj_piece_doubles( p );
-    a.states = a.partial + st_adj_partial_doubles( p );
+    a.states = a.cstart + group * pieces * 6 * 64 * tiles;
+    a.partial = work + st_adj_work_doubles( p, group ) - partials * st_adj_row_doubles( p );
     if( p->base.n > 0 && group > 0 )
     {
         for( int64_t end = p->base.n_turns; end > 0; end -= group )
@@ -1013,7 +1014,7 @@ extern "C" hipError_t KN( st_launch_adj_gradients )( const st_adj_plan_t* p, con
     }
     if( p->n_mp > 0 )
         hipLaunchKernelGGL( KN( st_k_adj_sum ), dim3( ( unsigned )p->n_mp ), dim3( 256 ), 0, stream,
-                            a.partial, p->base.n > 0 ? st_adj_partials( p ) : 0, p->n_mp, ( int )a.no,
+                            a.partial, partials, p->n_mp, ( int )a.no,
                             p->mp_order, grad_knl, grad_ksl );
     return hipGetLastError();
 }

@@ -24,8 +24,8 @@
     extern "C" hipError_t st_launch_adj_loss##SUF( const st_adj_plan_t* p,               \
         const double* coords, double* loss, int32_t* status, hipStream_t stream );        \
     extern "C" hipError_t st_launch_adj_gradients##SUF( const st_adj_plan_t* p,          \
-        const double* grad_out, double* work, double* grad_coords, double* grad_knl,      \
-        double* grad_ksl, hipStream_t stream );
+        const double* grad_out, double* work, int64_t group, double* grad_coords,         \
+        double* grad_knl, double* grad_ksl, hipStream_t stream );
 
 // Reverse pass (adjoint_kernels.hip): elements of a piece and of the part of
 // it whose states are in LDS at a time, doubles of a kept state; the particle
@@ -46,33 +46,37 @@ static inline int64_t st_adj_parts( const st_adj_plan_t* p )
 // or the pieces where K is smaller
 static inline int64_t st_adj_units( const st_adj_plan_t* p )
 { return p->base.K > ST_ADJ_PIECE ? ( p->base.n_elem + p->base.K - 1 ) / p->base.K : st_adj_pieces( p ); }
-// turns whose pieces run side by side; 0: one wave goes through all pieces
-static inline int64_t st_adj_group( const st_adj_plan_t* p )
+static inline int64_t st_adj_row_doubles( const st_adj_plan_t* p )
+{ return p->n_mp * 2 * ( p->max_order + 1 ); }
+// work, pieces of a group of turns side by side: Jacobians
+// [group][piece][36][64 tiles], end and start cotangents
+// [group][piece][6][64 tiles] each, first states of parts
+// [group][part][8][64 tiles], partial sums [group][tiles][row];
+// one wave through all pieces: first states of the parts of one unit, partial
+// sums [tiles][row]
+static inline int64_t st_adj_turn_doubles( const st_adj_plan_t* p )
 {
-    if( p->base.n > ST_ADJ_PARALLEL_MAX || p->base.n <= 0 ) return 0;
-    int64_t const turn = ( st_adj_pieces( p ) * ( 36 + 6 + 6 ) + st_adj_parts( p ) * ST_ADJ_STATE ) *
-                         64 * st_adj_tiles( p ) * 8;
-    int64_t const g = ST_ADJ_PARALLEL_BYTES / turn;
-    return g < p->base.n_turns ? g : p->base.n_turns;
+    return st_adj_tiles( p ) * ( 64 * ( st_adj_pieces( p ) * ( 36 + 6 + 6 ) + st_adj_parts( p ) * ST_ADJ_STATE ) +
+                                 st_adj_row_doubles( p ) );
 }
-// work: Jacobians [group][piece][36][64 tiles], end and start cotangents
-// [group][piece][6][64 tiles] each, partial sums [partials][n_mp][2 (max_order + 1)],
-// first states of parts [group][part][8][64 tiles], or of the parts of one
-// unit where one wave goes through all pieces
-static inline int64_t st_adj_partials( const st_adj_plan_t* p )
-{ return ( st_adj_group( p ) > 0 ? st_adj_group( p ) : 1 ) * st_adj_tiles( p ); }
-static inline int64_t st_adj_piece_doubles( const st_adj_plan_t* p )
-{ return st_adj_group( p ) * st_adj_pieces( p ) * ( 36 + 6 + 6 ) * 64 * st_adj_tiles( p ); }
-static inline int64_t st_adj_partial_doubles( const st_adj_plan_t* p )
-{ return st_adj_partials( p ) * p->n_mp * 2 * ( p->max_order + 1 ); }
-static inline int64_t st_adj_state_doubles( const st_adj_plan_t* p )
+static inline int64_t st_adj_unit_doubles( const st_adj_plan_t* p )
 {
     int64_t const unit = p->base.K > ST_ADJ_PIECE ? p->base.K : ST_ADJ_PIECE;
     int64_t const range = unit < p->base.n_elem ? unit : p->base.n_elem;
-    int64_t const slots = st_adj_group( p ) > 0 ? st_adj_group( p ) * st_adj_parts( p )
-                                                : ( range + ST_ADJ_SUB - 1 ) / ST_ADJ_SUB;
-    return slots * ST_ADJ_STATE * 64 * st_adj_tiles( p );
+    return st_adj_tiles( p ) * ( 64 * ( ( range + ST_ADJ_SUB - 1 ) / ST_ADJ_SUB ) * ST_ADJ_STATE +
+                                 st_adj_row_doubles( p ) );
 }
+// turns whose pieces run side by side with at most ``doubles`` of work; 0: one
+// wave goes through all pieces
+static inline int64_t st_adj_group( const st_adj_plan_t* p, int64_t doubles )
+{
+    if( p->base.n > ST_ADJ_PARALLEL_MAX || p->base.n <= 0 || doubles < 0 ) return 0;
+    int64_t const most = ST_ADJ_PARALLEL_BYTES / 8;
+    int64_t const g = ( doubles < most ? doubles : most ) / st_adj_turn_doubles( p );
+    return g < p->base.n_turns ? g : p->base.n_turns;
+}
+static inline int64_t st_adj_work_doubles( const st_adj_plan_t* p, int64_t group )
+{ return group > 0 ? group * st_adj_turn_doubles( p ) : st_adj_unit_doubles( p ); }
 
 ST_DECLARE_ADJ_LAUNCHERS( _exact )
 ST_DECLARE_ADJ_LAUNCHERS( _fma )

@@ -1,5 +1,6 @@
 """AdjointTracker.write_coefficients and NS(Adjoint_coefficients): what they
-take, what they refuse, and the words they write (CPU, no kernel runs)."""
+take, what they refuse, and the words they write; the work memory of the
+gradients (CPU, no kernel runs)."""
 import ctypes as ct
 
 import pytest
@@ -68,3 +69,25 @@ def test_a_tracker_on_the_cpu_writes_both_streams():
     assert torch.equal(tr.lat, lat) and torch.equal(tr.hot, hot)
     tr = _tracker([])
     tr.write_coefficients(tr.knl0, tr.ksl0)
+
+
+@pytest.mark.parametrize("n", [1, 64, 1000, 65536, 70000])
+def test_work_memory_for_fewer_turns_at_a_time(n):
+    """As many whole turns as fit, and below one turn what a single wave
+    through all elements needs."""
+    tr = _tracker([2, 1] * 50)
+    tr.n_turns = 7
+    plan = tr.plan(n, tr.knl0, tr.lat)
+    within = adjoint._lib.st_Adjoint_gradient_doubles_within
+    most = within(ct.byref(plan), 2**62)
+    least = within(ct.byref(plan), 0)
+    assert 0 < least <= most <= 2**29
+    if n > 65536:                              # the waves fill the chip one by one
+        assert most == least
+        return
+    assert most % 7 == 0
+    turn = most // 7
+    assert least < turn
+    for limit in (0, turn - 1, turn, turn + 1, 3 * turn - 1, 3 * turn, 6 * turn + 5, 7 * turn, 8 * turn):
+        turns = min(limit // turn, 7)
+        assert within(ct.byref(plan), limit) == (turns * turn if turns else least)

@@ -57,3 +57,44 @@ def test_the_backward_pass_is_linear_in_K(n, turns):
     when each of the 63 pieces went through what lies before it)."""
     eb = lattices.adjoint_sublattice(n_cells=80, tune=17.24)
     assert _backward_seconds(eb, n, turns, 4000) < 3.0 * _backward_seconds(eb, n, turns, 64)
+
+
+@pytest.mark.parametrize("K", [64, 300])
+def test_gradients_where_the_device_is_short_of_memory(K, monkeypatch):
+    """Room for all turns at once, for a few and for none (the allocations
+    that find no room are refused here)."""
+    from sixtracklib_amd.adjoint import AdjointTracker
+    n, turns = 4096, 10
+    rng = np.random.default_rng(1)
+    _, species = lattices.make_particles(1)
+    tr = AdjointTracker(lattices.adjoint_sublattice(), turns, species=species, K=K)
+    scale = np.array([3e-4, 3e-6, 3e-4, 3e-6, 0.05, 1e-4])
+    X = torch.tensor(rng.normal(size=(n, 6)) * scale, device="cuda", requires_grad=True)
+    knl, ksl = tr.knl0.clone().requires_grad_(), tr.ksl0.clone().requires_grad_()
+    empty, made = torch.empty, []
+
+    def within(room):
+        def f(*size, **kw):
+            if len(size) == 1 and isinstance(size[0], int):
+                if 8 * size[0] > room:
+                    raise torch.OutOfMemoryError("no room for %d bytes" % (8 * size[0]))
+                made.append(8 * size[0])
+            return empty(*size, **kw)
+        return f
+
+    grads, most = [], []
+    for room in (1e12, 2.5e8, 2e7):
+        loss = tr.loss(X, knl, ksl)
+        del made[:]
+        monkeypatch.setattr(torch, "empty", within(room))
+        grads.append(torch.autograd.grad(loss, [X, knl, ksl]))
+        monkeypatch.undo()
+        most.append(max(made))
+    assert most[0] > 2.5e8 >= most[1] > 2e7 >= most[2]
+    for some in grads[1:]:
+        for a, b in zip(some, grads[0]):
+            assert float((a - b).norm()) <= 2e-12 * float(b.norm())
+    loss = tr.loss(X, knl, ksl)
+    monkeypatch.setattr(torch, "empty", within(1e5))
+    with pytest.raises(torch.OutOfMemoryError):
+        torch.autograd.grad(loss, [X, knl, ksl])
