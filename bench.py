@@ -46,10 +46,10 @@ HBM_PEAK_GBS = 8000.0
 # FETCH_SIZE and writes 1,048,576 KiB of WRITE_SIZE, hence x2048 and x1024 B):
 # a track launch of the plain 1000-turn job of the 1M-particle ring (mean of
 # its 25 launches, 21 of them mixed and 4 with one particle per lane:
-# 7,450,806 / 10,832,802 KiB) and one turn of element-by-element
+# 3,338,098 / 4,068,784 KiB) and one turn of element-by-element
 # tracking of the collective ring with 100k particles in the exact build
 # (one 10-turn call / 10: 1,473,333 / 2,052,266,253 KiB)
-TRACK_LAUNCH_HBM_BYTES = 7450806 * 2048 + 10832802 * 1024
+TRACK_LAUNCH_HBM_BYTES = 3338098 * 2048 + 4068784 * 1024
 EBE_TURN_HBM_BYTES = (1473333 * 2048 + 2052266253 * 1024) // 10
 
 
@@ -515,7 +515,7 @@ def main():
                                        "(FETCH_SIZE reads 0.5x, WRITE_SIZE 1.0x); waves with two "
                                        "particles per lane read the particle constants and delta and "
                                        "write delta and psigma at each Cavity (registers hold only the "
-                                       "Drift/Multipole state): 26.4 GB per launch at 94 GB/s",
+                                       "Drift/Multipole state): 11.0 GB per launch at 39 GB/s",
                      "algorithmic_hbm_bytes_per_launch": alg_bytes},
         "cpu_baseline": cpu,
         "batched": batched,

@@ -260,8 +260,8 @@ __global__ void __launch_bounds__( 256 ) KN( st_k_adj_reduce )( int64_t n,
 //   * the sums over particles are formed in the wave (DPP adds, a fixed
 //     order) instead of through four values per particle and multipole.
 // 4,096 particles, 1,000 elements, 10 turns, exact build: forward 3.9 -> 0.78
-// ms, reverse 9.6 -> 0.79 ms (Jacobians 0.25, chain 0.07, through 0.13, its
-// refinement 0.07, coefficients 0.23, sums 0.03).  Backward pass as called,
+// ms, reverse 9.6 -> 0.75 ms (Jacobians 0.25, chain 0.05, through 0.13, its
+// refinement 0.06, coefficients 0.23, sums 0.03).  Backward pass as called,
 // before / now: 64 particles, 10 turns 7.2 / 0.36 ms, 16,384 and 10 turns
 // 13.7 / 2.7.  Side by side costs three and a half sweeps instead of one and
 // wins as long as the particles leave SIMDs idle: 2 turns, 65,536 particles
@@ -714,7 +714,8 @@ __global__ void __launch_bounds__( 64, 2 ) KN( st_k_adj_jacobian )( PlanArgs a )
 // take in the Jacobians, and one CU takes in some 35 GB/s, whatever its waves
 // have in flight (64 particles a block: 0.5 us a piece, with one wave or with
 // six).  So a block has 16 particles, whose rows are a cache line each, and
-// two waves of 48 lanes, three components each.
+// two waves of 48 lanes, three components each: 0.34 us a piece, 0.38 with
+// REFINE.
 template< bool REFINE >
 ST_DEV void adj_chain( const PlanArgs& a )
 {
@@ -743,12 +744,16 @@ ST_DEV void adj_chain( const PlanArgs& a )
         }
     };
     double c = a.add ? a.grad_coords[ 6 * i + p ] : 0.0;
+    int t = a.t0 + a.turns, left = 0;                  // turn, pieces of it before this one
     auto step = [ & ]( int64_t tp, const double* M )
     {
         double( *const w )[ 16 ] = v[ tp & 1 ];
+        bool const turn_end = left == 0;
+        if( turn_end ) { --t; left = a.pieces; }
+        --left;
         if( !idle )
         {
-            if( tp % a.pieces == a.pieces - 1 ) c += loss_term( a, weight[ p ], a.t0 + tp / a.pieces, p, i, g );
+            if( turn_end ) c += loss_term( a, weight[ p ], t, p, i, g );
             a.cend[ ( tp * 6 + p ) * N + tid ] = c;
             w[ p ][ k ] = REFINE ? c - M[ 6 ] : c;
         }
@@ -757,7 +762,7 @@ ST_DEV void adj_chain( const PlanArgs& a )
                          fma( M[ 3 ], w[ 3 ][ k ], fma( M[ 4 ], w[ 4 ][ k ], M[ 5 ] * w[ 5 ][ k ] ) ) ) ) );
         c = REFINE ? M[ 7 ] + r : r;
     };
-    constexpr int AHEAD = 4;
+    constexpr int AHEAD = 8;
     double M[ AHEAD ][ 8 ] = {};
 #pragma unroll
     for( int j = 0; j < AHEAD - 1; ++j ) load( last - j, M[ j ] );
