@@ -167,8 +167,11 @@ __global__ void __launch_bounds__( 256 ) KN( st_k_batch_select_split )( st_batch
 
 // Issue-priority rule of a track launch (WavePrio, track_lean.h): none
 // without wave_prio; balanced launches keep their waves level with the
-// mean progress of the min(tiles, resident waves) waves that have a tile;
-// the persistent-chunk form bands by turns left.
+// mean progress of the min(tiles, waves) waves of the launch that have a
+// tile (all of them resident at eight waves per SIMD; where the kernel holds
+// fewer, st_k_batch_track_hot and st_k_batch_track_heavy_hot with more tiles
+// than that, those still to start hold the mean down and the rule does
+// little); the persistent-chunk form bands by turns left.
 template< int TILE >
 ST_DEV WavePrio launch_priority( const st_batch_sched_t& s, int64_t max_turns )
 {
@@ -333,8 +336,8 @@ KN( st_k_batch_track_heavy )( st_batch_sched_t s, int64_t until_turn, int64_t ma
 
 // The same with the scheduled record walk (track_hot.h): a lattice of
 // 20,019 elements, 19 of them beam-beam or space charge, 100,000 particles:
-// 289 ns per element with the compiled loop, 105 with this (FMA build; 308
-// and 141 exact).  109 to 113 VGPRs, four waves per SIMD; held to 72 VGPRs
+// 291 ns per element with the compiled loop, 101 with this (FMA build; 315
+// and 139 exact).  109 to 113 VGPRs, four waves per SIMD; held to 72 VGPRs
 // for seven it spills and measures the same.
 __global__ void __launch_bounds__( 64, 4 )
 KN( st_k_batch_track_heavy_hot )( st_batch_sched_t s, int64_t until_turn, int64_t max_turns,

@@ -13,11 +13,14 @@
 // the caller's stream; nothing here synchronises except select_sync().
 //
 // run_balanced(U) is the alternative for one request on a host thread that
-// may wait: every launch gives each resident wave at most one tile, taken
+// may wait: every launch gives each of W waves at most one tile, taken
 // from the particles furthest behind first, and the host reads the counts
-// back between groups of launches.  With T tiles and W resident waves, W < T < 2W,
-// the persistent form ends every chunk with T - W tiles on a nearly idle
-// chip; here every launch but the last of a request fills the W waves.
+// back between groups of launches.  With T tiles, W < T < 2W, the persistent
+// form ends every chunk with T - W tiles on a nearly idle chip; here every
+// launch but the last of a request fills the W waves.  W is eight waves per
+// SIMD, what the compiled loops and the walk with one register set hold; the
+// walk with two holds seven and its heavy variant four, and the waves past
+// that start as others end (measured with that: Config::walk).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -136,14 +139,14 @@ struct Config
     // workgroups (16 waves then run on 16 CUs, each with a scalar cache of
     // its own: 54.6 against 59.2 ns per element with workgroups of four,
     // FMA build, 1,000 particles on the 20,000-element ring).  It is faster
-    // than the compiled loop at every size (ns per element and launch on
-    // that ring, exact and FMA build, loop / walk): 65,536 particles
-    // 198 / 88 and 169 / 63; 131,072: 212 / 111 and 178 / 78; 262,144:
-    // 284 / 209 and 242 / 139; 393,216: 333 / 303 and 239 / 208; 524,288:
-    // 439 / 390 and 298 / 261.  Which of its two forms: walk_form.  Lattices
-    // with the out-of-line maps run its heavy variant: 1,048,576 particles
-    // on the 20,019-element ring with beam-beam and space charge
-    // 1108 / 1026 and 905 / 750, 100,000 308 / 141 and 290 / 105.
+    // than the compiled loop at every size (ns per element on that ring, all
+    // on one box, exact and FMA build, loop / walk): 1,000 particles 189 / 77
+    // and 166 / 54; 65,536: 193 / 86 and 169 / 62; 131,072: 213 / 121 and
+    // 178 / 87; 262,144: 260 / 220 and 242 / 151; 393,216: 350 / 318 and
+    // 280 / 221; 524,288: 447 / 410 and 330 / 276.  Which of its two forms:
+    // walk_form.  Lattices with the out-of-line maps run its heavy variant:
+    // 1,048,576 particles on the 20,019-element ring with beam-beam and space
+    // charge 1180 / 968 and 992 / 740, 100,000 315 / 139 and 291 / 101.
     bool walk() const { return hot && ppl == 1 && !lds(); }
 
     // particles per lane of a launch: two run in the walk only
@@ -464,8 +467,8 @@ struct BatchRunner
     // a record's reads within the wave, and ask the scalar cache for 32
     // words a record; with more than four waves per SIMD the other waves
     // hide them, and in the FMA build the scalar cache is then what the
-    // waves wait for.  ns per element, 20,000-element ring, two sets / one,
-    // FMA: 131,072 particles 78 / 108; 262,144 (four waves) 139 / 145;
+    // waves wait for.  ns per element, 20,000-element ring, two sets / one
+    // (on a box some 5 % faster than that of Config::walk), FMA: 131,072 particles 78 / 108; 262,144 (four waves) 139 / 145;
     // 320,000 172 / 169; 393,216 211 / 208; 430,000 278 / 240; 524,288
     // 301 / 261; 16 lattices of 28,000 296 / 234.  Exact (half as many
     // again FP64 instructions a record): 262,144 209 / 213; 393,216

@@ -6,8 +6,8 @@
 // few waves per SIMD a record costs its instructions one after the other,
 // scalar work included, plus what it waits for: 41 to 69 cycles for scalar
 // loads that hit the scalar cache, 166 for one that misses to L2, about 35
-// for a taken jump.  The compiled loop of track_lean.h spends 170 ns (FMA
-// build) to 198 ns (exact) per element of a 20,000-element ring, whether 64
+// for a taken jump.  The compiled loop of track_lean.h spends 166 ns (FMA
+// build) to 193 ns (exact) per element of a 20,000-element ring, whether 64
 // or 65,536 particles are tracked; the FP64 instructions of an average
 // element take 25 to 35 ns.  Here
 //   * every record of the hot stream (lattice_hot.h) names the handler of
@@ -27,8 +27,8 @@
 //   * the lanes lost or done are out of exec, so an aperture test needs no
 //     mask operation.
 // Measured on that ring (ns per element, compiled loop / this): exact build
-// 198 / 78 with 1,000 to 16,000 particles, 198 / 88 with 65,536; FMA build
-// 166 / 55 and 169 / 63.
+// 189 / 77 with 1,000 particles, 192 / 77 with 16,000, 193 / 86 with 65,536;
+// FMA build 166 / 54, 168 / 55 and 169 / 62.
 // Maps are those of track_device.h with the same IEEE operations (each
 // fused where that build fuses), so the results are the same bits.
 #pragma once

@@ -377,7 +377,7 @@ struct NS(TrackJobBase)
 
     // the device addresses of every Particles object of the job's device
     // copy of the particle buffer (the reference's kernel fetches them on
-    // the device; here they follow from the image's relocation)
+    // the device; here they follow from the image's address)
     bool fetch_paddr()
     {
         if( paddr_buf == nullptr || d_pbuf == nullptr ) return false;
