@@ -85,6 +85,10 @@ _lib.st_Adjoint_coefficients.argtypes = [ct.POINTER(AdjPlan), ct.c_int, ct.c_voi
 _lib.st_Adjoint_loss.restype = ct.c_int
 _lib.st_Adjoint_loss.argtypes = [ct.POINTER(AdjPlan), ct.c_int, ct.c_void_p, ct.c_void_p,
                                  ct.c_void_p, ct.c_void_p]
+_lib.st_Adjoint_gradient_doubles.restype = ct.c_int64
+_lib.st_Adjoint_gradient_doubles.argtypes = [ct.POINTER(AdjPlan)]
+_lib.st_Adjoint_gradients.restype = ct.c_int
+_lib.st_Adjoint_gradients.argtypes = [ct.POINTER(AdjPlan), ct.c_int] + [ct.c_void_p] * 6
 _lib.st_Adjoint_gradient_doubles_within.restype = ct.c_int64
 _lib.st_Adjoint_gradient_doubles_within.argtypes = [ct.POINTER(AdjPlan), ct.c_int64]
 _lib.st_Adjoint_gradients_within.restype = ct.c_int

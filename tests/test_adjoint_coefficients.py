@@ -82,6 +82,7 @@ def test_work_memory_for_fewer_turns_at_a_time(n):
     most = within(ct.byref(plan), 2**62)
     least = within(ct.byref(plan), 0)
     assert 0 < least <= most <= 2**29
+    assert most == adjoint._lib.st_Adjoint_gradient_doubles(ct.byref(plan))
     if n > 65536:                              # the waves fill the chip one by one
         assert most == least
         return
