@@ -140,7 +140,7 @@ struct Config
     // its own: 54.6 against 59.2 ns per element with workgroups of four,
     // FMA build, 1,000 particles on the 20,000-element ring).  It is faster
     // than the compiled loop at every size (ns per element on that ring, all
-    // on one box, exact and FMA build, loop / walk): 1,000 particles 189 / 77
+    // on one card, exact and FMA build, loop / walk): 1,000 particles 189 / 77
     // and 166 / 54; 65,536: 193 / 86 and 169 / 62; 131,072: 213 / 121 and
     // 178 / 87; 262,144: 260 / 220 and 242 / 151; 393,216: 350 / 318 and
     // 280 / 221; 524,288: 447 / 410 and 330 / 276.  Which of its two forms:
@@ -468,7 +468,8 @@ struct BatchRunner
     // words a record; with more than four waves per SIMD the other waves
     // hide them, and in the FMA build the scalar cache is then what the
     // waves wait for.  ns per element, 20,000-element ring, two sets / one
-    // (on a box some 5 % faster than that of Config::walk), FMA: 131,072 particles 78 / 108; 262,144 (four waves) 139 / 145;
+    // (on a card some 5 % faster than that of Config::walk), FMA: 131,072
+    // particles 78 / 108; 262,144 (four waves) 139 / 145;
     // 320,000 172 / 169; 393,216 211 / 208; 430,000 278 / 240; 524,288
     // 301 / 261; 16 lattices of 28,000 296 / 234.  Exact (half as many
     // again FP64 instructions a record): 262,144 209 / 213; 393,216
